@@ -48,11 +48,18 @@ int pmt_filter_fwd(int nelx, int nely, int nelz, int kx, int ky, int kz, const d
  * padded coordinates mapping to each element coordinate, concatenated x|y|z (inv_ptr holds
  * nelx+1, nely+1, max(nelz,1)+1 entries, absolute offsets into inv_idx).  Every element coordinate
  * farther than (k-1)/2 from both ends of its axis must map from its own padded coordinate only (true
- * for the reference's padding modes): the default kernels reduce those from LDS tiles and walk the lists
+ * for the reference's padding modes): the default kernels reduce those from LDS boxes and use the lists
  * only within that distance of a face. */
 int pmt_filter_bwd(int nelx, int nely, int nelz, int kx, int ky, int kz, const double* w,
                    const int32_t* inv_ptr, const int32_t* inv_idx, const double* dy, double* dx,
                    void* stream);
+/* The same adjoint with a workspace of pmt_filter_work_size(...) doubles (NULL: pmt_filter_bwd), which holds
+ * the correlation at each padded cell, so the elements at the faces add up their cells instead of
+ * evaluating each with all its taps.  The same bits with and without. */
+long long pmt_filter_work_size(int nelx, int nely, int nelz, int kx, int ky, int kz);
+int pmt_filter_bwd_work(int nelx, int nely, int nelz, int kx, int ky, int kz, const double* w,
+                        const int32_t* inv_ptr, const int32_t* inv_idx, const double* dy, double* dx, double* work,
+                        void* stream);
 
 /* DensityFilter (pymoto/modules/filter.py:223-378): y_i = so_i * sum_j H_ij * si_j * x_j with
  * H_ij = max(0, radius - |i - j|) over the window |j - i|_inf <= int(radius) clipped to the grid
@@ -172,9 +179,9 @@ int pmt_k0_extend(int dim, const double* K0_host, double* ext_host);
  * the reflection basis from the transformed child densities, no stencil stored (default; used when
  * k0_pattern has PMT_K0_REFLECTION and the level is not the coarsest), 0 = half stencil.  Read by
  * pmt_mg_create: it applies to hierarchies created afterwards.
- * PMT_TUNE_FILTER: FilterConv kernels for the 3^3 / 5^3 (3^2 / 5^2) extents, 1 = LDS-tiled z-streamed
- * blocks (default), 0 = one thread per element gathering through the caches; both sum the taps in the
- * same order.
+ * PMT_TUNE_FILTER: FilterConv kernels for extents k x k x kz up to 15 whose box of outputs fits LDS, 1 = boxes
+ * staged in LDS (default), 0 = one thread per element gathering through the caches; both sum the taps in
+ * the same order.
  * pmt_get_tuning returns the current value or a negative status.
  * (No reference counterpart: the launch shapes picked by the autotuner, pymoto_amd/tune.py.) */
 #define PMT_TUNE_FINE_KERNEL 1

@@ -9,6 +9,7 @@
 // padded cells that map onto it (per-axis inverse lists; interior elements have exactly one) and
 // evaluates the 'full' correlation there - a gather, so no atomics and a deterministic sum.
 #include <algorithm>
+#include <type_traits>
 
 #include "launch.h"
 
@@ -79,7 +80,7 @@ filter_bwd_kernel(int nx, int ny, int nz, int kx, int ky, int kz, const double* 
       const int b = inv_idx[ib];
       for (int ia = px[i]; ia < px[i + 1]; ++ia) {
         const int a = inv_idx[ia];
-        // correlate 'full' at padded cell (a, b, c)
+        double cell = 0.0;  // correlate 'full' at padded cell (a, b, c)
         for (int r = 0; r < kz; ++r) {
           const int cc = c - (kz - 1) + r;
           if (cc < 0 || cc >= nz) continue;
@@ -89,10 +90,11 @@ filter_bwd_kernel(int nx, int ny, int nz, int kx, int ky, int kz, const double* 
             for (int p = 0; p < kx; ++p) {
               const int aa = a - (kx - 1) + p;
               if (aa < 0 || aa >= nx) continue;
-              acc = fma(w[((long long)p * ky + q) * kz + r], dy[((long long)cc * ny + bb) * nx + aa], acc);
+              cell = fma(w[((long long)p * ky + q) * kz + r], dy[((long long)cc * ny + bb) * nx + aa], cell);
             }
           }
         }
+        acc += cell;
       }
     }
   }
@@ -145,18 +147,52 @@ filter_fwd_fixed_kernel(int nx, int ny, int nz, const double* __restrict__ w, co
 
 // The element's padded cells are exactly its own position shifted by the half widths (the element is at
 // least (K-1)/2 from every mirrored, replicated or wrapped face, or the padding is constant).
-template <int KXY, int KZ>
 __device__ inline bool filter_single_cell(const int32_t* __restrict__ inv_ptr, const int32_t* __restrict__ inv_idx,
-                                          int nx, int ny, int i, int j, int k) {
+                                          int nx, int ny, int hx, int hz, int i, int j, int k) {
   const int32_t* px = inv_ptr;
   const int32_t* py = inv_ptr + (nx + 1);
   const int32_t* pz = inv_ptr + (nx + 1) + (ny + 1);
-  return px[i + 1] - px[i] == 1 && inv_idx[px[i]] == i + (KXY - 1) / 2 && py[j + 1] - py[j] == 1 &&
-         inv_idx[py[j]] == j + (KXY - 1) / 2 && pz[k + 1] - pz[k] == 1 && inv_idx[pz[k]] == k + (KZ - 1) / 2;
+  return px[i + 1] - px[i] == 1 && inv_idx[px[i]] == i + hx && py[j + 1] - py[j] == 1 &&
+         inv_idx[py[j]] == j + hx && pz[k + 1] - pz[k] == 1 && inv_idx[pz[k]] == k + hz;
 }
 
-// dx_e of element (i, j, k) by its inverse lists: the 'full' correlation of dy at every padded cell
-// that maps onto it, in list order (the taps in the order r, q, p)
+// The 'full' correlation of dy at padded cell (a, b, c), the taps in the order r, q, p.  The loads of a
+// plane of taps are issued together, with the address of a tap outside the grid clamped to 0 (a branch
+// around each load would wait for every one of them in turn).
+template <int KXY, int KZ>
+__device__ inline double filter_bwd_cell(int nx, int ny, int nz, const double* __restrict__ w,
+                                         const double* __restrict__ dy, int a, int b, int c) {
+  double acc = 0.0;
+#pragma unroll(KXY <= 3 ? KZ : 1)
+  for (int r = 0; r < KZ; ++r) {
+    const int cc = c - (KZ - 1) + r;
+    double v[KXY][KXY];
+    bool in[KXY][KXY];
+#pragma unroll
+    for (int q = 0; q < KXY; ++q) {
+      const int bb = b - (KXY - 1) + q;
+      const bool row = cc >= 0 && cc < nz && bb >= 0 && bb < ny;
+      const long long base = row ? ((long long)cc * ny + bb) * nx : 0;
+#pragma unroll
+      for (int p = 0; p < KXY; ++p) {
+        const int aa = a - (KXY - 1) + p;
+        in[q][p] = row && aa >= 0 && aa < nx;
+        v[q][p] = dy[in[q][p] ? base + aa : 0];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < KXY; ++q)
+#pragma unroll
+      for (int p = 0; p < KXY; ++p) {
+        const double t = fma(w[(p * KXY + q) * KZ + r], v[q][p], acc);
+        acc = in[q][p] ? t : acc;
+      }
+  }
+  return acc;
+}
+
+// dx_e of element (i, j, k) by its inverse lists: the sum, in list order, of the correlation at every
+// padded cell that maps onto it
 template <int KXY, int KZ>
 __device__ inline double filter_bwd_gather(int nx, int ny, int nz, const double* __restrict__ w,
                                            const int32_t* __restrict__ inv_ptr, const int32_t* __restrict__ inv_idx,
@@ -165,30 +201,10 @@ __device__ inline double filter_bwd_gather(int nx, int ny, int nz, const double*
   const int32_t* py = inv_ptr + (nx + 1);
   const int32_t* pz = inv_ptr + (nx + 1) + (ny + 1);
   double acc = 0.0;
-  for (int ic = pz[k]; ic < pz[k + 1]; ++ic) {
-    const int c = inv_idx[ic];
-    for (int ib = py[j]; ib < py[j + 1]; ++ib) {
-      const int b = inv_idx[ib];
-      for (int ia = px[i]; ia < px[i + 1]; ++ia) {
-        const int a = inv_idx[ia];
-#pragma unroll
-        for (int r = 0; r < KZ; ++r) {
-          const int cc = c - (KZ - 1) + r;
-#pragma unroll
-          for (int q = 0; q < KXY; ++q) {
-            const int bb = b - (KXY - 1) + q;
-#pragma unroll
-            for (int p = 0; p < KXY; ++p) {
-              const int aa = a - (KXY - 1) + p;
-              const bool in = cc >= 0 && cc < nz && bb >= 0 && bb < ny && aa >= 0 && aa < nx;
-              const long long m = in ? ((long long)cc * ny + bb) * nx + aa : 0;
-              if (in) acc = fma(w[(p * KXY + q) * KZ + r], dy[m], acc);
-            }
-          }
-        }
-      }
-    }
-  }
+  for (int ic = pz[k]; ic < pz[k + 1]; ++ic)
+    for (int ib = py[j]; ib < py[j + 1]; ++ib)
+      for (int ia = px[i]; ia < px[i + 1]; ++ia)
+        acc += filter_bwd_cell<KXY, KZ>(nx, ny, nz, w, dy, inv_idx[ia], inv_idx[ib], inv_idx[ic]);
   return acc;
 }
 
@@ -206,281 +222,292 @@ filter_bwd_fixed_kernel(int nx, int ny, int nz, const double* __restrict__ w, co
   dx[e] = filter_bwd_gather<KXY, KZ>(nx, ny, nz, w, inv_ptr, inv_idx, dy, i, j, k);
 }
 
-// Shell of the tiled adjoint: the elements within the half widths of a face, where every padding mode puts
-// the elements with more than one padded cell (mirrored, replicated or wrapped cells map there), in three
-// disjoint slab sets - x slabs (all j, k), y slabs (interior i), z slabs (interior i, j).  Those with a
-// single cell are left to the tiled kernel.
-template <int KXY, int KZ>
-__global__ void __launch_bounds__(256)
-filter_bwd_shell_kernel(int nx, int ny, int nz, const double* __restrict__ w, const int32_t* __restrict__ inv_ptr,
-                        const int32_t* __restrict__ inv_idx, const double* __restrict__ dy, double* __restrict__ dx) {
-  constexpr int HX = (KXY - 1) / 2, HZ = (KZ - 1) / 2;
-  const int wx = min(nx, 2 * HX), wy = min(ny, 2 * HX), wz = min(nz, 2 * HZ);
+// Cell t of the shell of half widths hx (x and y) and hz of an nx x ny x nz box, in three disjoint slab sets
+// - x slabs (all j, k), y slabs (interior i), z slabs (interior i, j).  False past the last.
+__device__ inline bool shell_cell(long long t, int nx, int ny, int nz, int hx, int hz, int& i, int& j, int& k) {
+  const int wx = min(nx, 2 * hx), wy = min(ny, 2 * hx), wz = min(nz, 2 * hz);
   const long long cx = (long long)wx * ny * nz, cy = (long long)(nx - wx) * wy * nz;
   const long long cz = (long long)(nx - wx) * (ny - wy) * wz;
-  long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   // slab index a of width wa on an axis of extent n: the first half-width, then the last
   auto side = [](int a, int wa, int n, int h) { return (a < h || wa == n) ? a : n - wa + a; };
-  int i, j, k;
   if (t < cx) {
-    i = side((int)(t % wx), wx, nx, HX);
+    i = side((int)(t % wx), wx, nx, hx);
     t /= wx;
     j = (int)(t % ny);
     k = (int)(t / ny);
   } else if ((t -= cx) < cy) {
     i = wx / 2 + (int)(t % (nx - wx));
     t /= (nx - wx);
-    j = side((int)(t % wy), wy, ny, HX);
+    j = side((int)(t % wy), wy, ny, hx);
     k = (int)(t / wy);
   } else if ((t -= cy) < cz) {
     i = wx / 2 + (int)(t % (nx - wx));
     t /= (nx - wx);
     j = wy / 2 + (int)(t % (ny - wy));
-    k = side((int)(t / (ny - wy)), wz, nz, HZ);
+    k = side((int)(t / (ny - wy)), wz, nz, hz);
   } else {
-    return;
+    return false;
   }
-  if (filter_single_cell<KXY, KZ>(inv_ptr, inv_idx, nx, ny, i, j, k)) return;
+  return true;
+}
+
+inline long long shell_cells(long long nx, long long ny, long long nz, int hx, int hz) {
+  const long long wx = std::min(nx, 2LL * hx), wy = std::min(ny, 2LL * hx), wz = std::min(nz, 2LL * hz);
+  return wx * ny * nz + (nx - wx) * wy * nz + (nx - wx) * (ny - wy) * wz;
+}
+
+// The elements with more than one padded cell (mirrored, replicated or wrapped cells map there) lie within
+// the half widths of a face with every padding mode.  With a workspace g of the padded extents the box
+// kernel evaluates the correlation once per padded cell and filter_bwd_fold_kernel adds up each such
+// element's cells, eight loads at a time: an element in a corner has 8 (symmetric) to 64 (edge, 7^3) of
+// them, and walking those with all their taps in one thread bounded the whole adjoint (21.6 us of 49 at
+// 256x128x128 with 3^3; 461 us at 75x51x33 with 7^3).  Without a workspace the list walk stays
+// (filter_bwd_shell_kernel).
+__global__ void __launch_bounds__(256)
+filter_bwd_fold_kernel(int nx, int ny, int nz, int kxy, int kz, const int32_t* __restrict__ inv_ptr,
+                       const int32_t* __restrict__ inv_idx, const double* __restrict__ g, double* __restrict__ dx) {
+  const int hx = (kxy - 1) / 2, hz = (kz - 1) / 2;
+  int i, j, k;
+  if (!shell_cell((long long)blockIdx.x * blockDim.x + threadIdx.x, nx, ny, nz, hx, hz, i, j, k)) return;
+  if (filter_single_cell(inv_ptr, inv_idx, nx, ny, hx, hz, i, j, k)) return;
+  const int32_t* px = inv_ptr + i;
+  const int32_t* py = inv_ptr + (nx + 1) + j;
+  const int32_t* pz = inv_ptr + (nx + 1) + (ny + 1) + k;
+  const int pa = px[0], pb = py[0], pc = pz[0];
+  const int na = px[1] - pa, nb = py[1] - pb, cells = na * nb * (pz[1] - pc);
+  const long long lx = nx + kxy - 1, ly = ny + kxy - 1;
+  double acc = 0.0;
+  for (int t = 0; t < cells; t += 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int q = min(t + u, cells - 1), r = q / na, c = r / nb;
+      v[u] = g[(inv_idx[pc + c] * ly + inv_idx[pb + r - c * nb]) * lx + inv_idx[pa + q - r * na]];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = t + u < cells ? acc + v[u] : acc;
+  }
+  dx[((long long)k * ny + j) * nx + i] = acc;
+}
+
+template <int KXY, int KZ>
+__global__ void __launch_bounds__(256)
+filter_bwd_shell_kernel(int nx, int ny, int nz, const double* __restrict__ w, const int32_t* __restrict__ inv_ptr,
+                        const int32_t* __restrict__ inv_idx, const double* __restrict__ dy, double* __restrict__ dx) {
+  int i, j, k;
+  constexpr int HX = (KXY - 1) / 2, HZ = (KZ - 1) / 2;
+  if (!shell_cell((long long)blockIdx.x * blockDim.x + threadIdx.x, nx, ny, nz, HX, HZ, i, j, k)) return;
+  if (filter_single_cell(inv_ptr, inv_idx, nx, ny, HX, HZ, i, j, k)) return;
   dx[((long long)k * ny + j) * nx + i] = filter_bwd_gather<KXY, KZ>(nx, ny, nz, w, inv_ptr, inv_idx, dy, i, j, k);
 }
 
-// LDS-tiled forms of the fixed-extent kernels (default).  A block of 64 x 4 threads owns 64 x 16 output
-// columns (a thread the column of 4 outputs above its row) and walks a chunk of nzc element planes in z;
-// the input planes the tile needs pass through a ring of KZ LDS planes of (64 + KXY - 1) x (16 + KXY - 1)
-// values, each fetched once from HBM while the previous plane is reduced.  A thread reads the
-// (4 + KXY - 1) x KXY values of a plane that its 4 outputs share once and carries the 4 tap chains
-// together (a quarter of the LDS reads of one output per thread), and every chain sums its taps in the
-// order of the gather kernels above (r, then q, then p), so both forms give the same bits.
-constexpr int kFiltTX = 64, kFiltTY = 4, kFiltOY = 4;
-constexpr int kFiltRY = kFiltTY * kFiltOY;  // output rows of a tile
-int g_filter_tiled = 1;                     // PMT_TUNE_FILTER: 1 tiled (default), 0 per-element gathers
+int g_filter_tiled = 1;  // PMT_TUNE_FILTER: 1 boxes in LDS (default), 0 per-element gathers
 
-// Forward: the padded value at (a, b, c) is cz[c] if mz[c] < 0, else cy[b] if my[b] < 0, else cx[a] if
-// mx[a] < 0, else x[mz[c], my[b], mx[a]]; everything but mz[c] is the same for every plane, so each
-// thread resolves its cells' in-plane sources once and a plane costs one load per cell.
-template <int KXY, int KZ>
-__global__ void __launch_bounds__(kFiltTX * kFiltTY)
-filter_fwd_tiled_kernel(int nx, int ny, int nz, int tiles_x, int tiles_y, int nzc, int zero, const double* __restrict__ w,
-                        const int32_t* __restrict__ map, const double* __restrict__ cval, const double* __restrict__ x,
-                        double* __restrict__ y) {
-  constexpr int LX = kFiltTX + KXY - 1, LY = kFiltRY + KXY - 1, LP = LX * LY, NT = kFiltTX * kFiltTY;
-  constexpr int PER = (LP + NT - 1) / NT;  // plane values loaded per thread
-  constexpr int WY = kFiltOY + KXY - 1;    // rows of a thread's window
-  __shared__ double ring[KZ][LP];
-  const int tid = threadIdx.x, tx = tid % kFiltTX, ty = tid / kFiltTX;
-  const int tile = blockIdx.x % (tiles_x * tiles_y), chunk = blockIdx.x / (tiles_x * tiles_y);
-  const int i0 = (tile % tiles_x) * kFiltTX, j0 = (tile / tiles_x) * kFiltRY;
-  const int kbeg = chunk * nzc, kend = min(kbeg + nzc, nz);
-  const int Lx = nx + KXY - 1, Ly = ny + KXY - 1, Lz = nz + KZ - 1;
-  const int nxy = nx * ny;
-  const int32_t* mx = map;
-  const int32_t* my = map + Lx;
-  const int32_t* mz = map + Lx + Ly;
-  const double* cz = cval + Lx + Ly;
-  // in-plane source of each cell this thread loads: element offset (>= 0), or -1 with its constant in
-  // cst (constant row or column), or -2 outside the padded grid / the tile (value 0)
-  int src[PER];
-  double cst[PER];
+// Box kernels (KXY x KXY x kz): the whole window of a box of outputs in LDS at once.  256 threads as
+// 32 x nty x ntz, a thread the column of OY outputs above its row; per z tap the OY rows it needs slide by
+// one per y tap, so a value is read from LDS once per z tap for OY outputs.  The weights of a z tap lie one
+// per lane and are broadcast through scalar registers (v_readlane; as scalar loads, KXY^2 strided ones per z
+// tap, each wait also drained the LDS reads).  The taps are summed in the order of the gather kernels (r,
+// then q, then p): the same bits.  FWD: outputs are elements, the box holds their padded cells, resolved
+// through the maps.  Adjoint: outputs are the padded cells, the box holds dy (zero outside the grid); the
+// cell of an element without other cells is its result, every other one goes to the workspace g (if given)
+// for filter_bwd_fold_kernel.
+// Forward / adjoint with its fold: 21.9 / 35.2 us at 256x128x128 with 3^3, 13.1 / 21.3 us at 130x70x60 with 5^3,
+// 13.6 / 17.6 us at 75x51x33 with 7^3.  A ring of LDS planes streamed in z took 26.3 / 47.6 and 62.9 / 151 us
+// (5^3 held 450 registers, one wave per SIMD), the per-element gathers 69 / 165 us for 7^3 (which the adjoint
+// without a workspace still takes).
+template <int KXY, int OY, bool FWD>
+__global__ void __launch_bounds__(256)
+filter_box_kernel(int nx, int ny, int nz, int kz, int nty, int tiles_x, int tiles_y, unsigned m_ly,
+                   const double* __restrict__ w, const int32_t* __restrict__ m0, const int32_t* __restrict__ m1,
+                   const double* __restrict__ cval, const double* __restrict__ in, double* __restrict__ out,
+                   double* __restrict__ g) {
+  constexpr int HX = (KXY - 1) / 2, LX = 32 + KXY - 1, NW = (KXY * KXY + 63) / 64;
+  extern __shared__ double box[];
+  const int ntz = 8 / nty, hz = (kz - 1) / 2, ly = OY * nty + KXY - 1, lz = ntz + kz - 1;
+  const int tid = threadIdx.x, lane = tid & 63, tx = tid & 31, ty = (tid >> 5) % nty, tz = (tid >> 5) / nty;
+  const int tile = blockIdx.x % (tiles_x * tiles_y);
+  const int i0 = (tile % tiles_x) * 32, j0 = (tile / tiles_x) * OY * nty, k0 = (blockIdx.x / (tiles_x * tiles_y)) * ntz;
+  const int plx = nx + KXY - 1, ply = ny + KXY - 1, plz = nz + kz - 1;
+  const int nbox = LX * ly * lz;
+  // source index of the box's columns, rows and planes: >= 0 inside, -1 constant padding, -2 nothing (0)
+  int* sx = (int*)(box + nbox);
+  int* sy = sx + LX;
+  int* sz = sy + ly;
+  // adjoint: whether the element at an output column, row or plane has only its own cell on that axis
+  int* one = sz + lz;
+  if (!FWD)
+    for (int t = tid; t < 32 + OY * nty + ntz; t += 256) {
+      const int ax = t < 32 ? 0 : t < 32 + OY * nty ? 1 : 2;
+      const int e = ax == 0 ? i0 + t - HX : ax == 1 ? j0 + t - 32 - HX : k0 + t - 32 - OY * nty - hz;
+      const int n = ax == 0 ? nx : ax == 1 ? ny : nz, h = ax == 2 ? hz : HX;
+      const int32_t* ptr = m0 + (ax == 0 ? 0 : ax == 1 ? nx + 1 : nx + ny + 2);
+      one[t] = e >= 0 && e < n && ptr[e + 1] - ptr[e] == 1 && m1[ptr[e]] == e + h;
+    }
+  for (int t = tid; t < LX + ly + lz; t += 256) {
+    const int ax = t < LX ? 0 : t < LX + ly ? 1 : 2;
+    const int q = ax == 0 ? t : ax == 1 ? t - LX : t - LX - ly;
+    const int at = (ax == 0 ? i0 : ax == 1 ? j0 : k0) + q, n = ax == 0 ? nx : ax == 1 ? ny : nz;
+    const int kk = ax == 2 ? kz : KXY;
+    int v;
+    if (FWD) {
+      v = at < n + kk - 1 ? m0[(ax == 0 ? 0 : ax == 1 ? plx : plx + ply) + at] : -2;
+      if (v < -1) v = at < n + kk - 1 ? -1 : -2;
+    } else {
+      v = at - (kk - 1);
+      if (v < 0 || v >= n) v = -2;
+    }
+    sx[t] = v;
+  }
+  __syncthreads();
+  // 8 values per thread and step: their loads are in flight together
+  for (int q0 = tid; q0 < nbox; q0 += 256 * 8) {
+    double v[8];
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int q = tid + t * NT;
-    const int a = i0 + q % LX, b = j0 + q / LX;
-    src[t] = -2;
-    cst[t] = 0.0;
-    if (q < LP && a < Lx && b < Ly) {
-      const int mb = my[b];
-      if (mb < 0) {
-        src[t] = -1;
-        cst[t] = cval[Lx + b];
-      } else {
-        const int ma = mx[a];
-        if (ma < 0) {
-          src[t] = -1;
-          cst[t] = cval[a];
-        } else {
-          src[t] = mb * nx + ma;
-        }
+    for (int u = 0; u < 8; ++u) {
+      const int q = q0 + 256 * u;
+      const int a = q % LX, t = q / LX, c = (int)(((unsigned)t * m_ly) >> 20), b = t - c * ly;
+      v[u] = 0.0;
+      if (q < nbox) {
+        const int ma = sx[a], mb = sy[b], mc = sz[c];
+        if (ma >= 0 && mb >= 0 && mc >= 0)
+          v[u] = in[(mc * ny + mb) * nx + ma];
+        else if (FWD && ma != -2 && mb != -2 && mc != -2)
+          v[u] = cval[mc < 0 ? plx + ply + k0 + c : mb < 0 ? plx + j0 + b : i0 + a];
       }
     }
-  }
-  auto fetch = [&](int c, double (&v)[PER]) {
-    const int mc = c < Lz ? mz[c] : 0;
-    const double czc = (c < Lz && mc < 0) ? cz[c] : 0.0;
 #pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      double val = src[t] == -1 ? cst[t] : 0.0;
-      if (src[t] >= 0 && mc >= 0) val = x[mc * nxy + src[t]];  // a constant plane (mc < 0) reads nothing
-      v[t] = (mc < 0 && src[t] != -2) ? czc : val;
-    }
+    for (int u = 0; u < 8; ++u)
+      if (q0 + 256 * u < nbox) box[q0 + 256 * u] = v[u];
+  }
+  __syncthreads();
+  double acc[OY];
+#pragma unroll
+  for (int o = 0; o < OY; ++o) acc[o] = 0.0;
+  double wl[NW], wn[NW];  // weights of this z tap and the next: lane l holds tap (p, q) = (l / KXY, l % KXY)
+  auto weights = [&](int r, double (&d)[NW]) {
+#pragma unroll
+    for (int h = 0; h < NW; ++h) d[h] = 64 * h + lane < KXY * KXY ? w[(64 * h + lane) * kz + r] : 0.0;
   };
-  auto store = [&](int c, const double (&v)[PER]) {
+  weights(0, wl);
+  for (int r = 0; r < kz; ++r) {
+    weights(r + 1 < kz ? r + 1 : r, wn);
+    const double* pl = box + ((FWD ? tz + kz - 1 - r : tz + r) * ly + ty * OY) * LX + tx;
+    double win[OY][KXY];  // row y of the column's window in slot y % OY
+    auto load = [&](int y) {
 #pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int q = tid + t * NT;
-      if (q < LP) ring[c % KZ][q] = v[t];
-    }
-  };
-  double v[PER];
-  for (int c = kbeg; c < kbeg + KZ - 1; ++c) {
-    fetch(c, v);
-    store(c, v);
-  }
-  fetch(kbeg + KZ - 1, v);
-  const int i = i0 + tx, jb = j0 + ty * kFiltOY;
-  for (int k = kbeg; k < kend; ++k) {
-    store(k + KZ - 1, v);  // padded plane k + KZ - 1 completes the window of output plane k
-    __syncthreads();
-    if (k + 1 < kend) fetch(k + KZ, v);  // next plane's loads in flight during the reduction
-    // the weights are re-read per plane through the scalar cache (zero is 0; hoisted out of the loop they
-    // would occupy KXY^2 KZ register pairs per thread)
-    const double* wk = w + zero * k;
-    double acc[kFiltOY];
+      for (int p = 0; p < KXY; ++p) win[y % OY][p] = pl[y * LX + p];
+    };
 #pragma unroll
-    for (int o = 0; o < kFiltOY; ++o) acc[o] = 0.0;
+    for (int o = 0; o < OY; ++o) load(FWD ? KXY - 1 + o : o);
 #pragma unroll
-    for (int r = 0; r < KZ; ++r) {
-      const double* pl = ring[(k + KZ - 1 - r) % KZ] + ty * kFiltOY * LX + tx;
-      double win[WY][KXY];
+    for (int q = 0; q < KXY; ++q) {
+      if (q > 0) load(FWD ? KXY - 1 - q : q + OY - 1);
 #pragma unroll
-      for (int yy = 0; yy < WY; ++yy)
+      for (int p = 0; p < KXY; ++p) {
+        const int l = p * KXY + q;
+        const long long bits = __double_as_longlong(wl[l / 64]);
+        const unsigned lo = __builtin_amdgcn_readlane((int)bits, l % 64);
+        const unsigned hi = __builtin_amdgcn_readlane((int)(bits >> 32), l % 64);
+        const double wt = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 #pragma unroll
-        for (int p = 0; p < KXY; ++p) win[yy][p] = pl[yy * LX + p];
-#pragma unroll
-      for (int q = 0; q < KXY; ++q)
-#pragma unroll
-        for (int p = 0; p < KXY; ++p) {
-          const double wt = wk[(p * KXY + q) * KZ + r];
-#pragma unroll
-          for (int o = 0; o < kFiltOY; ++o) acc[o] = fma(wt, win[o + KXY - 1 - q][KXY - 1 - p], acc[o]);
-        }
-      if constexpr (KXY > 3) __builtin_amdgcn_sched_barrier(0);  // one plane's window live at a time
-    }
-#pragma unroll
-    for (int o = 0; o < kFiltOY; ++o)
-      if (i < nx && jb + o < ny) y[(k * ny + jb + o) * nx + i] = acc[o];
-    __syncthreads();  // the slot of plane k is overwritten next
-  }
-}
-
-// Adjoint: dx_e = sum over the padded cells mapping to e of the 'full' correlation of dy there.  The
-// tiled kernel reduces, from an LDS ring of dy planes (zero outside the grid), the elements whose only
-// padded cell is their own position (all but a shell of (K-1)/2 along mirrored, replicated or wrapped
-// faces; every element with constant padding); filter_bwd_shell_kernel then does the shell's elements
-// by their inverse lists, so no wave of the tiled kernel diverges into the list walk.
-template <int KXY, int KZ>
-__global__ void __launch_bounds__(kFiltTX * kFiltTY)
-filter_bwd_tiled_kernel(int nx, int ny, int nz, int tiles_x, int tiles_y, int nzc, int zero, const double* __restrict__ w,
-                        const int32_t* __restrict__ inv_ptr, const int32_t* __restrict__ inv_idx,
-                        const double* __restrict__ dy, double* __restrict__ dx) {
-  constexpr int HX = (KXY - 1) / 2, HZ = (KZ - 1) / 2;
-  constexpr int LX = kFiltTX + KXY - 1, LY = kFiltRY + KXY - 1, LP = LX * LY, NT = kFiltTX * kFiltTY;
-  constexpr int PER = (LP + NT - 1) / NT;
-  constexpr int WY = kFiltOY + KXY - 1;
-  __shared__ double ring[KZ][LP];
-  const int tid = threadIdx.x, tx = tid % kFiltTX, ty = tid / kFiltTX;
-  const int tile = blockIdx.x % (tiles_x * tiles_y), chunk = blockIdx.x / (tiles_x * tiles_y);
-  const int i0 = (tile % tiles_x) * kFiltTX, j0 = (tile / tiles_x) * kFiltRY;
-  const int kbeg = chunk * nzc, kend = min(kbeg + nzc, nz);
-  const int32_t* px = inv_ptr;
-  const int32_t* py = inv_ptr + (nx + 1);
-  const int32_t* pz = inv_ptr + (nx + 1) + (ny + 1);
-  // element (in-plane) offset of each cell this thread loads; -1 outside the grid (value 0)
-  int src[PER];
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int q = tid + t * NT;
-    const int ii = i0 - HX + q % LX, jj = j0 - HX + q / LX;
-    src[t] = (q < LP && ii >= 0 && ii < nx && jj >= 0 && jj < ny) ? jj * nx + ii : -1;
-  }
-  const int nxy = nx * ny;
-  auto fetch = [&](int kk, double (&v)[PER]) {
-    const bool zin = kk >= 0 && kk < nz;
-#pragma unroll
-    for (int t = 0; t < PER; ++t) v[t] = (zin && src[t] >= 0) ? dy[kk * nxy + src[t]] : 0.0;
-  };
-  auto store = [&](int kk, const double (&v)[PER]) {
-#pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int q = tid + t * NT;
-      if (q < LP) ring[(kk + KZ) % KZ][q] = v[t];
-    }
-  };
-  const int i = i0 + tx, jb = j0 + ty * kFiltOY;
-  // x and y parts of the single-cell test, once per thread
-  const bool xin = i < nx && px[i + 1] - px[i] == 1 && inv_idx[px[i]] == i + HX;
-  bool yin[kFiltOY];
-#pragma unroll
-  for (int o = 0; o < kFiltOY; ++o) {
-    const int j = jb + o;
-    yin[o] = xin && j < ny && py[j + 1] - py[j] == 1 && inv_idx[py[j]] == j + HX;
-  }
-  double v[PER];
-  for (int kk = kbeg - HZ; kk < kbeg + HZ; ++kk) {
-    fetch(kk, v);
-    store(kk, v);
-  }
-  fetch(kbeg + HZ, v);
-  for (int k = kbeg; k < kend; ++k) {
-    store(k + HZ, v);  // dy plane k + HZ completes the window of element plane k
-    __syncthreads();
-    if (k + 1 < kend) fetch(k + HZ + 1, v);
-    const bool zone = pz[k + 1] - pz[k] == 1 && inv_idx[pz[k]] == k + HZ;  // the same for the whole block
-    const double* wk = w + zero * k;  // re-read per plane (see the forward kernel)
-    if (zone) {
-      // element (i, j, k) at cell (i + HX, j + HX, k + HZ): dy at (i - HX + p, j - HX + q, k - HZ + r)
-      double acc[kFiltOY];
-#pragma unroll
-      for (int o = 0; o < kFiltOY; ++o) acc[o] = 0.0;
-#pragma unroll
-      for (int r = 0; r < KZ; ++r) {
-        const double* pl = ring[(k - HZ + r + KZ) % KZ] + ty * kFiltOY * LX + tx;
-        double win[WY][KXY];
-#pragma unroll
-        for (int yy = 0; yy < WY; ++yy)
-#pragma unroll
-          for (int p = 0; p < KXY; ++p) win[yy][p] = pl[yy * LX + p];
-#pragma unroll
-        for (int q = 0; q < KXY; ++q)
-#pragma unroll
-          for (int p = 0; p < KXY; ++p) {
-            const double wt = wk[(p * KXY + q) * KZ + r];
-#pragma unroll
-            for (int o = 0; o < kFiltOY; ++o) acc[o] = fma(wt, win[o + q][p], acc[o]);
-          }
-        if constexpr (KXY > 3) __builtin_amdgcn_sched_barrier(0);  // one plane's window live at a time
+        for (int o = 0; o < OY; ++o)
+          acc[o] = fma(wt, FWD ? win[(o + KXY - 1 - q) % OY][KXY - 1 - p] : win[(o + q) % OY][p], acc[o]);
       }
-#pragma unroll
-      for (int o = 0; o < kFiltOY; ++o)
-        if (yin[o]) dx[(k * ny + jb + o) * nx + i] = acc[o];
     }
-    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < NW; ++h) wl[h] = wn[h];
+  }
+  const int a = i0 + tx, c = k0 + tz;
+  if (a >= (FWD ? nx : plx) || c >= (FWD ? nz : plz)) return;
+#pragma unroll
+  for (int o = 0; o < OY; ++o) {
+    const int b = j0 + ty * OY + o;
+    if (b >= (FWD ? ny : ply)) break;
+    if (FWD) {
+      out[(c * ny + b) * nx + a] = acc[o];
+      continue;
+    }
+    if (one[tx] & one[32 + ty * OY + o] & one[32 + OY * nty + tz])
+      out[((c - hz) * ny + b - HX) * nx + a - HX] = acc[o];
+    else if (g)
+      g[((long long)c * ply + b) * plx + a] = acc[o];
   }
 }
 
-template <int KXY, int KZ>
-void launch_filter_tiled(bool fwd, int nx, int ny, int nz, const double* w, const int32_t* m0, const int32_t* m1,
-                         const double* cv, const double* in, double* out, hipStream_t s) {
-  const int tiles_x = (nx + kFiltTX - 1) / kFiltTX, tiles_y = (ny + kFiltRY - 1) / kFiltRY;
-  // planes per block: about three blocks per CU (a block re-reads KZ - 1 halo planes), 4 to 16 planes
-  const long long want = 3LL * device_cu_count();
-  const int nzc = (int)std::max(4LL, std::min(16LL, (long long)nz * tiles_x * tiles_y / std::max(1LL, want)));
-  const unsigned blocks = (unsigned)(tiles_x * tiles_y * ((nz + nzc - 1) / nzc));
-  if (fwd) {
-    filter_fwd_tiled_kernel<KXY, KZ><<<blocks, kFiltTX * kFiltTY, 0, s>>>(nx, ny, nz, tiles_x, tiles_y, nzc, 0, w, m0,
-                                                                        cv, in, out);
-  } else {
-    filter_bwd_tiled_kernel<KXY, KZ><<<blocks, kFiltTX * kFiltTY, 0, s>>>(nx, ny, nz, tiles_x, tiles_y, nzc, 0, w, m0,
-                                                                        m1, in, out);
-    constexpr int HX = (KXY - 1) / 2, HZ = (KZ - 1) / 2;
-    const long long wx = std::min(nx, 2 * HX), wy = std::min(ny, 2 * HX), wz = std::min(nz, 2 * HZ);
-    const long long shell = wx * ny * nz + (nx - wx) * wy * nz + (nx - wx) * (ny - wy) * wz;
-    if (shell > 0)
-      filter_bwd_shell_kernel<KXY, KZ><<<blocks_for(shell, 256), 256, 0, s>>>(nx, ny, nz, w, m0, m1, in, out);
+struct FilterBox {
+  int oy, nty, ly;
+  size_t lds;
+};
+
+// The box over an lx x ly x lz range of outputs: 32 x 8 x 4 (one plane: 32 x 32) with 4 outputs per thread;
+// half as high with 2 while those boxes are too few to give every CU two.  (Twice as high with 8, less halo
+// per output: 24.5 instead of 21.4 us for 3^3 forward at 256x128x128.)
+inline FilterBox filter_box(int kxy, int kz, long long lx, long long ly, long long lz) {
+  FilterBox b;
+  b.nty = kz == 1 ? 8 : 2;
+  const long long boxes = (lx + 31) / 32 * ((ly + 4 * b.nty - 1) / (4 * b.nty)) * ((lz + 8 / b.nty - 1) / (8 / b.nty));
+  b.oy = boxes < 2LL * device_cu_count() ? 2 : 4;
+  b.ly = b.oy * b.nty + kxy - 1;
+  const int x = 32 + kxy - 1, z = 8 / b.nty + kz - 1;
+  b.lds = sizeof(double) * x * b.ly * z + sizeof(int) * (x + b.ly + z + 32 + b.oy * b.nty + 8 / b.nty);
+  return b;
+}
+
+// whether the box kernels take these extents: boxes above 64 KB of LDS (3D from 11^3) stay with the gather
+// kernels, and so does the adjoint of the kernels above 5 without a workspace
+inline bool filter_box_ok(bool fwd, int nx, int ny, int nz, int kx, int ky, int kz, const double* work) {
+  if (kx != ky || kx < 3 || kx > 15) return false;
+  if (!fwd && !work && !(kx <= 5 && (kz == kx || kz == 1))) return false;
+  return (fwd ? filter_box(kx, kz, nx, ny, nz) : filter_box(kx, kz, nx + kx - 1, ny + kx - 1, nz + kz - 1)).lds <= 65536;
+}
+
+template <int KXY>
+void launch_filter_box_k(bool fwd, int nx, int ny, int nz, int kz, const double* w, const int32_t* m0,
+                          const int32_t* m1, const double* cv, const double* in, double* out, double* work,
+                          hipStream_t s) {
+  const int lx = fwd ? nx : nx + KXY - 1, ly = fwd ? ny : ny + KXY - 1, lz = fwd ? nz : nz + kz - 1;
+  const FilterBox b = filter_box(KXY, kz, lx, ly, lz);
+  const int ntz = 8 / b.nty, tiles_x = (lx + 31) / 32, tiles_y = (ly + b.oy * b.nty - 1) / (b.oy * b.nty);
+  const unsigned blocks = (unsigned)(tiles_x * tiles_y * ((lz + ntz - 1) / ntz));
+  const unsigned m_ly = (1u << 20) / b.ly + 1;  // t / ly for t < ly * lz, ly <= 46, lz <= 18
+  auto run = [&](auto kernel) {
+    kernel<<<blocks, 256, b.lds, s>>>(nx, ny, nz, kz, b.nty, tiles_x, tiles_y, m_ly, w, m0, m1, cv, in, out, work);
+  };
+  auto pick = [&](auto is_fwd) {
+    constexpr bool F = decltype(is_fwd)::value;
+    if (b.oy == 4) return run(filter_box_kernel<KXY, 4, F>);
+    run(filter_box_kernel<KXY, 2, F>);
+  };
+  if (fwd) return pick(std::true_type{});
+  pick(std::false_type{});
+  const unsigned shell = blocks_for(shell_cells(nx, ny, nz, (KXY - 1) / 2, (kz - 1) / 2), 256);
+  if (work) {
+    filter_bwd_fold_kernel<<<shell, 256, 0, s>>>(nx, ny, nz, KXY, kz, m0, m1, work, out);
+  } else if constexpr (KXY <= 5) {
+    if (kz == 1)
+      filter_bwd_shell_kernel<KXY, 1><<<shell, 256, 0, s>>>(nx, ny, nz, w, m0, m1, in, out);
+    else
+      filter_bwd_shell_kernel<KXY, KXY><<<shell, 256, 0, s>>>(nx, ny, nz, w, m0, m1, in, out);
   }
 }
 
-// the tiled kernels index with 32-bit element numbers
-inline bool filter_tiled_ok(long long nel) { return g_filter_tiled && nel < (1LL << 31); }
+void launch_filter_box(bool fwd, int nx, int ny, int nz, int kxy, int kz, const double* w, const int32_t* m0,
+                        const int32_t* m1, const double* cv, const double* in, double* out, double* work,
+                        hipStream_t s) {
+  switch (kxy) {
+    case 3: return launch_filter_box_k<3>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    case 5: return launch_filter_box_k<5>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    case 7: return launch_filter_box_k<7>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    case 9: return launch_filter_box_k<9>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    case 11: return launch_filter_box_k<11>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    case 13: return launch_filter_box_k<13>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+    default: return launch_filter_box_k<15>(fwd, nx, ny, nz, kz, w, m0, m1, cv, in, out, work, s);
+  }
+}
+
+// the box kernels index with 32-bit element numbers
+inline bool filter_32bit_ok(long long nel) { return g_filter_tiled && nel < (1LL << 31); }
 
 // DensityFilter (pymoto/modules/filter.py:223-378): y_i = so_i * sum_j H_ij (si_j * x_j) over the
 // clipped window |j - i|_inf <= int(radius) with H_ij = max(0, radius - |i - j|) in element units.
@@ -520,14 +547,9 @@ int pmt_filter_fwd(int nelx, int nely, int nelz, int kx, int ky, int kz, const d
   const long long nel = (long long)nelx * nely * nz;
   const unsigned nb = blocks_for(nel, 256);
   hipStream_t s = (hipStream_t)stream;
-  if (filter_tiled_ok(nel) && kx == ky && ((kx == 3 && (kz == 3 || kz == 1)) || (kx == 5 && (kz == 5 || kz == 1)))) {
-    if (kx == 3)
-      (kz == 3 ? launch_filter_tiled<3, 3> : launch_filter_tiled<3, 1>)(true, nelx, nely, nz, w, map, nullptr, cval, x,
-                                                                       y, s);
-    else
-      (kz == 5 ? launch_filter_tiled<5, 5> : launch_filter_tiled<5, 1>)(true, nelx, nely, nz, w, map, nullptr, cval, x,
-                                                                       y, s);
-    return check_launch("filter_fwd_tiled_kernel");
+  if (filter_32bit_ok(nel) && filter_box_ok(true, nelx, nely, nz, kx, ky, kz, nullptr)) {
+    launch_filter_box(true, nelx, nely, nz, kx, kz, w, map, nullptr, cval, x, y, nullptr, s);
+    return check_launch("filter_box_kernel");
   }
   if (kx == 3 && ky == 3 && kz == 3)
     filter_fwd_fixed_kernel<3, 3><<<nb, 256, 0, s>>>(nelx, nely, nz, w, map, cval, x, y);
@@ -556,6 +578,16 @@ int pmt_density_filter(int nelx, int nely, int nelz, double radius, const double
 
 int pmt_filter_bwd(int nelx, int nely, int nelz, int kx, int ky, int kz, const double* w, const int32_t* inv_ptr,
                    const int32_t* inv_idx, const double* dy, double* dx, void* stream) {
+  return pmt_filter_bwd_work(nelx, nely, nelz, kx, ky, kz, w, inv_ptr, inv_idx, dy, dx, nullptr, stream);
+}
+
+long long pmt_filter_work_size(int nelx, int nely, int nelz, int kx, int ky, int kz) {
+  if (!grid_ok(nelx, nely, nelz) || kx < 1 || ky < 1 || kz < 1) return arg_error("pmt_filter_work_size: bad argument");
+  return ((long long)nelx + kx - 1) * ((long long)nely + ky - 1) * ((long long)(nelz > 0 ? nelz : 1) + kz - 1);
+}
+
+int pmt_filter_bwd_work(int nelx, int nely, int nelz, int kx, int ky, int kz, const double* w, const int32_t* inv_ptr,
+                        const int32_t* inv_idx, const double* dy, double* dx, double* work, void* stream) {
   if (!grid_ok(nelx, nely, nelz) || kx < 1 || ky < 1 || kz < 1 || !(kx & 1) || !(ky & 1) || !(kz & 1) || !w ||
       !inv_ptr || !inv_idx || !dy || !dx)
     return arg_error("pmt_filter_bwd: bad argument");
@@ -564,14 +596,9 @@ int pmt_filter_bwd(int nelx, int nely, int nelz, int kx, int ky, int kz, const d
   const long long nel = (long long)nelx * nely * nz;
   const unsigned nb = blocks_for(nel, 256);
   hipStream_t s = (hipStream_t)stream;
-  if (filter_tiled_ok(nel) && kx == ky && ((kx == 3 && (kz == 3 || kz == 1)) || (kx == 5 && (kz == 5 || kz == 1)))) {
-    if (kx == 3)
-      (kz == 3 ? launch_filter_tiled<3, 3> : launch_filter_tiled<3, 1>)(false, nelx, nely, nz, w, inv_ptr, inv_idx,
-                                                                       nullptr, dy, dx, s);
-    else
-      (kz == 5 ? launch_filter_tiled<5, 5> : launch_filter_tiled<5, 1>)(false, nelx, nely, nz, w, inv_ptr, inv_idx,
-                                                                       nullptr, dy, dx, s);
-    return check_launch("filter_bwd_tiled_kernel");
+  if (filter_32bit_ok(nel) && filter_box_ok(false, nelx, nely, nz, kx, ky, kz, work)) {
+    launch_filter_box(false, nelx, nely, nz, kx, kz, w, inv_ptr, inv_idx, nullptr, dy, dx, work, s);
+    return check_launch("filter_box_kernel");
   }
   if (kx == 3 && ky == 3 && kz == 3)
     filter_bwd_fixed_kernel<3, 3><<<nb, 256, 0, s>>>(nelx, nely, nz, w, inv_ptr, inv_idx, dy, dx);

@@ -99,7 +99,7 @@ class FilterConv(Module):
             p = self.weights.shape[ax] // 2
             m, v = _axis_map(sizes[ax], p, *self.bcs[ax])
             ptr, idx = _inverse_lists(m, sizes[ax])
-            # the tiled adjoint kernel takes every element farther than the half width p from both faces
+            # the adjoint kernels take every element farther than the half width p from both faces
             # to have only its own padded cell (p + a); the padding modes put the others within p of a face
             inner = np.arange(p, sizes[ax] - p)
             assert np.all(np.diff(ptr)[inner] == 1) and np.all(idx[ptr[inner]] == inner + p)
@@ -117,6 +117,8 @@ class FilterConv(Module):
         self._cval = np.concatenate(vals)
         self._inv_ptr = np.concatenate(inv_ptr).astype(np.int32)
         self._inv_idx = np.concatenate(inv_idx).astype(np.int32)
+        # whether an element has more than its own padded cell (the adjoint then folds them through a workspace)
+        self._folds = any(int(np.diff(p).max()) > 1 for p in ptrs)
         self._dev = None
 
     def _device_data(self):
@@ -143,8 +145,13 @@ class FilterConv(Module):
         dy = _lib.as_device(dfdv).reshape(-1)
         w, _, _, ip, ii = self._device_data()
         dx = torch.empty_like(dy)
-        _lib.check(lib.pmt_filter_bwd(*self.nel3, *self.weights.shape, _lib.ptr(w), _lib.ptr(ip), _lib.ptr(ii),
-                                      _lib.ptr(dy), _lib.ptr(dx), _lib.stream()), "filter adjoint")
+        work = None
+        if self._folds or max(self.weights.shape) > 5:  # (the 3- and 5-wide kernels need none without folds)
+            work = torch.empty(lib.pmt_filter_work_size(*self.nel3, *self.weights.shape), dtype=torch.float64,
+                               device=dy.device)
+        _lib.check(lib.pmt_filter_bwd_work(*self.nel3, *self.weights.shape, _lib.ptr(w), _lib.ptr(ip), _lib.ptr(ii),
+                                           _lib.ptr(dy), _lib.ptr(dx), _lib.ptr(work), _lib.stream()),
+                   "filter adjoint")
         xs = self.sig_in[0].state
         return dx.cpu().numpy() if isinstance(xs, np.ndarray) else dx
 
