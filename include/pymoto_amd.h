@@ -89,6 +89,16 @@ int pmt_heaviside_bwd(long long n, double beta, double eta, const double* x, con
 int pmt_oc_update(long long n, const double* x, const double* dg, double xmin, double xmax, double move,
                   double lmid, double* xnew, double* sum_out, double* work, void* stream);
 
+/* The whole bisection of OC.step (optimizers.py:404-433) enqueued at once, without a host read between its
+ * steps: from [l1, l2], while l2 - l1 > tol, lmid = (l1 + l2) / 2 and l1 = lmid if sum(xnew(lmid)) - target
+ * > 0 else l2 = lmid; xnew receives the design of the last lmid (the same bits as pmt_oc_update step by
+ * step).  work: pmt_oc_work_size() doubles; on completion work[0..3] = l1, l2, the last lmid, max(dg) (NaN if
+ * dg has one).  l2 - l1 may still exceed tol where the halvings do not reach it (tol near the spacing of
+ * doubles); with l2 - l1 <= tol at the start xnew is unspecified. */
+int pmt_oc_work_size(void);
+int pmt_oc_step(long long n, const double* x, const double* dg, double xmin, double xmax, double move, double l1,
+                double l2, double tol, double target, double* xnew, double* work, void* stream);
+
 /* Vector kernels.  y = a*x + b*y (x may be NULL: y = b*y). */
 int pmt_axpby(long long n, double a, const double* x, double b, double* y, void* stream);
 /* *out = x.y, deterministic two-stage reduction; work holds pmt_reduce_work_size() doubles.

@@ -30,6 +30,8 @@ _SIGS = {
     "pmt_heaviside_fwd": (c_int, [c_ll, c_dbl, c_dbl, c_vp, c_vp, c_vp]),
     "pmt_heaviside_bwd": (c_int, [c_ll, c_dbl, c_dbl, c_vp, c_vp, c_vp, c_int, c_vp, c_vp]),
     "pmt_oc_update": (c_int, [c_ll, c_vp, c_vp, c_dbl, c_dbl, c_dbl, c_dbl, c_vp, c_vp, c_vp, c_vp]),
+    "pmt_oc_work_size": (c_int, []),
+    "pmt_oc_step": (c_int, [c_ll, c_vp, c_vp] + [c_dbl] * 7 + [c_vp, c_vp, c_vp]),
     "pmt_axpby": (c_int, [c_ll, c_dbl, c_vp, c_dbl, c_vp, c_vp]),
     "pmt_dot": (c_int, [c_ll, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "pmt_reduce_work_size": (c_int, []),

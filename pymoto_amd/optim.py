@@ -3,8 +3,8 @@
 ``OC.step`` follows the reference: positive sensitivities are clipped to zero, the move limits are
 max(xmin, x - move) and min(xmax, x + move), and the Lagrange multiplier is bisected on
 [l1init, l2init] until l2 - l1 <= l1l2tol, each trial design x*sqrt(-dg/lmid) clipped to the limits
-and its volume compared with maxvol * n (maxvol defaults to the initial mean density).  Every trial
-runs as one fused HIP kernel with a deterministic sum; the host reads 8 bytes per bisection step.
+and its volume compared with maxvol * n (maxvol defaults to the initial mean density).  The whole
+bisection runs on the device with deterministic sums; the host reads its result once.
 ``OC.optimize`` drives a ``Network`` the way ``Optimizer.optimize`` does (response, sensitivity,
 step, stopping on the relative design and objective change).
 """
@@ -35,17 +35,25 @@ class OC:
         n = x.numel()
         if self.maxvol is None:
             self.maxvol = float(x.sum().item()) / n
-        if float(dg.max().item()) > 1e-15:
-            warnings.warn("OC only works for negative sensitivities; clipping positive values.")
         lib = _lib.lib()
         xnew = torch.empty_like(x)
-        tot = torch.empty(1, dtype=torch.float64, device=x.device)
-        work = _lib.reduce_work()
         l1, l2 = self.l1init, self.l2init
+        maxdg = None
+        if n > 0 and l2 - l1 > self.l1l2tol:
+            work = torch.empty(lib.pmt_oc_work_size(), dtype=torch.float64, device=x.device)
+            _lib.check(lib.pmt_oc_step(n, _lib.ptr(x), _lib.ptr(dg), self.xmin, self.xmax, self.move, float(l1), float(l2),
+                                       float(self.l1l2tol), self.maxvol * n, _lib.ptr(xnew), _lib.ptr(work),
+                                       _lib.stream()), "OC step")
+            l1, l2, _, maxdg = work[:4].tolist()
+        if (float(dg.max().item()) if maxdg is None else maxdg) > 1e-15:
+            warnings.warn("OC only works for negative sensitivities; clipping positive values.")
+        # the steps left where the interval does not halve down to the tolerance
         while l2 - l1 > self.l1l2tol:
+            tot = torch.empty(1, dtype=torch.float64, device=x.device)
             lmid = 0.5 * (l1 + l2)
             _lib.check(lib.pmt_oc_update(n, _lib.ptr(x), _lib.ptr(dg), self.xmin, self.xmax, self.move, lmid,
-                                         _lib.ptr(xnew), _lib.ptr(tot), _lib.ptr(work), _lib.stream()), "OC update")
+                                         _lib.ptr(xnew), _lib.ptr(tot), _lib.ptr(_lib.reduce_work()), _lib.stream()),
+                       "OC update")
             if float(tot.item()) - self.maxvol * n > 0:
                 l1 = lmid
             else:
