@@ -385,162 +385,293 @@ __global__ void dense_from_stencil_kernel(GridDims g, const double* __restrict__
 }
 
 // ---------------- blocked Gauss-Jordan inversion (in place), block size GJB ----------------
+// Panel k: with P = A[K][K]^-1, the old row panel R = A[K][:] and column panel C = A[:][K],
+//   A[K][K] = P, A[K][j] = P R_j, A[i][K] = -C_i P, A[i][j] -= C_i (P R_j)   (no pivoting: the operator is SPD)
+// One launch per panel, a block per 64 x 64 tile: the panels are read from copies that the previous launch's
+// blocks of that row and column wrote beside the matrix, so the tiles are updated in place; P R_j is formed
+// again by every block of a column (the same work as the update, on compute units that would wait
+// otherwise); the block of the next diagonal tile inverts it at the end of its update, so its chain of
+// pivots runs beside the other tiles of the launch.
+// 24 us per panel at n = 847 (14 panels) and bound by that chain; four launches per panel (diagonal inverse, column
+// copy, row panel, update) took 76 us.  Above n = 1900 the tiles bound it: 25 ms at n = 6069 (45 ms before).
 constexpr int GJB = 64;
+constexpr int GJL = GJB + 2;  // LDS row stride: the 16 rows x 2 entries of a half wave's operand read lie in 64 banks
+typedef double gj_d4 __attribute__((ext_vector_type(4)));
 
-// invert the kk x kk diagonal block at (k0, k0) in LDS, write it to P (GJB x GJB, row-major).
-// 16 x 16 threads, each owning a 4 x 4 set of entries (rows tr + 16 i, columns tc + 16 j); the block
-// is padded with the identity beyond kk, so every pivot step is the same 16 multiply-adds per thread
-// between two barriers (in-place Gauss-Jordan, no pivoting: the Galerkin operator is SPD).
-__global__ void __launch_bounds__(1024) gj_diag_kernel(long long n, long long k0, int kk, const double* __restrict__ A,
-                                                        double* __restrict__ P) {
-  // 32 x 32 threads, each owning a 2 x 2 sub-block; two LDS copies of the block alternate between
-  // pivot steps, so one barrier separates a step's reads from the next step's writes
-  __shared__ double sM[2][GJB][GJB + 1];
-  const int tr = threadIdx.x / 32, tc = threadIdx.x % 32;
+// 1 / x to an ulp (a correctly rounded division is a longer dependent chain)
+__device__ inline double gj_rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
+// In-place inverse of a 64 x 64 tile held by 4 waves in the matrix-core result layout (a wave per 32 x 32
+// quadrant: entry r of m[a][b] is row 32 (wave / 2) + 16 a + 4 r + lane / 16, column 32 (wave % 2) + 16 b +
+// lane % 16): block Gauss-Jordan with 4 x 4 pivot blocks Q, 16 steps with one barrier each.  The pivot rows R
+// and columns C go through LDS (sh: two buffers); every thread inverts Q itself; the rest is
+// m -= (C Q^-1) R, one matrix operation per 16 x 16 tile.  The pivot rows are one register (r = s % 4) of
+// all lanes of a tile row and become Q^-1 R; in the pivot columns m counts as 0 and R as the identity.
+// 15 us, a chain of dependent FP64 operations.  (One pivot per step, the whole tile moving through LDS, took
+// 40 us; 4 x 4 entries per thread and the rank-4 update without the matrix cores 22 us.)
+constexpr int kGjShared = 2 * (256 + 256 + 16);  // doubles
+__device__ inline void gj_invert_tile(gj_d4 (&m)[2][2], double* sh, int tid) {
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  auto pick = [odd = (lq & 1) != 0, high = (lq & 2) != 0](double v0, double v1, double v2, double v3) {
+    const double lo = odd ? v1 : v0, hi = odd ? v3 : v2;  // by value: a select of array elements would index memory
+    return high ? hi : lo;
+  };
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int s = 0; s < 16; ++s) {
+    double* rows = sh + (s & 1) * kGjShared / 2;  // R [4][64], the identity in the pivot columns
+    double* cols = rows + 256;                    // C [64][4]
+    double* pivot = cols + 256;                   // Q [4][4]
+    const int ta = (s / 4) % 2;                   // tile of the pivot in its quadrant
+    const bool own_r = wr == (s / 8) * 32, own_c = wc == (s / 8) * 32;
+    const bool piv = own_c && l16 / 4 == s % 4;   // (of tile column ta)
+    if (own_r) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int r = tr + 32 * i, c = tc + 32 * j;
-      sM[0][r][c] = (r < kk && c < kk) ? A[(k0 + r) * n + k0 + c] : (r == c ? 1.0 : 0.0);
-    }
-  __syncthreads();
-  for (int p = 0; p < kk; ++p) {
-    double(*const src)[GJB + 1] = sM[p & 1];
-    double(*const dst)[GJB + 1] = sM[(p + 1) & 1];
-    const double inv = 1.0 / src[p][p];
-    double mrp[2], mpc[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) mrp[i] = src[tr + 32 * i][p];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) mpc[j] = src[p][tc + 32 * j];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = tr + 32 * i, c = tc + 32 * j;
-        const double m = src[r][c];
-        double v;
-        if (r == p)
-          v = c == p ? inv : m * inv;
-        else
-          v = c == p ? -mrp[i] * inv : m - mrp[i] * (mpc[j] * inv);
-        dst[r][c] = v;
+      for (int b = 0; b < 2; ++b) {
+        const double v = m[ta][b][s % 4], e = l16 % 4 == lq ? 1.0 : 0.0;
+        rows[lq * 64 + wc + 16 * b + l16] = b == ta && piv ? e : v;
+        if (b == ta && piv) pivot[lq * 4 + l16 % 4] = v;
       }
-    __syncthreads();
-  }
-  for (int q = threadIdx.x; q < GJB * GJB; q += blockDim.x) {  // zero outside kk x kk: consumers read full tiles
-    const int r = q / GJB, c = q % GJB;
-    P[q] = (r < kk && c < kk) ? sM[kk & 1][r][c] : 0.0;
-  }
-}
-
-// C[i][c] = A[i][k0+c] (old column panel), all rows i
-__global__ void gj_colcopy_kernel(long long n, long long k0, int kk, const double* __restrict__ A,
-                                  double* __restrict__ C) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n * kk) return;
-  const long long i = q / kk;
-  const int c = (int)(q % kk);
-  C[i * GJB + c] = A[i * n + k0 + c];
-}
-
-// row panel A[K][j] = P A[K][j] for j outside K.  Block = 16 columns, staged in LDS with P (the panel
-// is updated in place); thread = one column and 4 of the 64 rows (r, r + 16, r + 32, r + 48).
-constexpr int GJ_RP_COLS = 16;
-__global__ void __launch_bounds__(256) gj_rowpanel_kernel(long long n, long long k0, int kk, double* __restrict__ A,
-                                                           const double* __restrict__ P) {
-  __shared__ double sP[GJB][GJB + 1];
-  __shared__ double sA[GJB][GJ_RP_COLS + 1];
-  const int tid = threadIdx.x;
-  const long long j0 = (long long)blockIdx.x * GJ_RP_COLS;
-  for (int q = tid; q < GJB * GJB; q += blockDim.x) sP[q / GJB][q % GJB] = P[q];
-  for (int q = tid; q < GJB * GJ_RP_COLS; q += blockDim.x) {
-    const int r = q / GJ_RP_COLS, c = q % GJ_RP_COLS;
-    const long long j = j0 + c;
-    sA[r][c] = (r < kk && j < n) ? A[(k0 + r) * n + j] : 0.0;
-  }
-  __syncthreads();
-  const int jj = tid % GJ_RP_COLS, rg = tid / GJ_RP_COLS;
-  const long long j = j0 + jj;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int c = 0; c < kk; ++c) {
-    const double a = sA[c][jj];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = fma(sP[rg + 16 * i][c], a, acc[i]);
-  }
-  if (j >= n || (j >= k0 && j < k0 + kk)) return;  // the pivot columns are set by gj_update_kernel
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = rg + 16 * i;
-    if (r < kk) A[(k0 + r) * n + j] = acc[i];
-  }
-}
-
-// rank-kk update of all tiles outside the pivot row block:
-//   j outside K: A[i][j] -= C[i][:] A[K][j] ; j inside K: A[i][K] = -C[i][:] P ; pivot block = P
-__global__ void __launch_bounds__(256) gj_update_kernel(long long n, long long k0, int kk, double* __restrict__ A,
-                                                         const double* __restrict__ C, const double* __restrict__ P) {
-  __shared__ double sC[64][GJB + 1];
-  __shared__ double sR[GJB][64 + 1];
-  const long long i0 = (long long)blockIdx.y * 64, j0 = (long long)blockIdx.x * 64;
-  const int tid = threadIdx.x;
-  const bool rowK = (i0 == k0);  // tiles are aligned to GJB, so the pivot row block is one tile row
-  const bool colK = (j0 == k0);
-  if (rowK && !colK) return;  // already holds the new row panel
-  if (rowK && colK) {
-    for (int q = tid; q < kk * kk; q += blockDim.x) {
-      const int r = q / kk, c = q % kk;
-      A[(k0 + r) * n + k0 + c] = P[r * GJB + c];
     }
+    if (piv) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cols[(wr + 16 * a + 4 * r + lq) * 4 + l16 % 4] = m[a][ta][r];
+    }
+    __syncthreads();
+    double q[4][4], c[2][4], r1[2], rr[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[i][j] = pivot[i * 4 + j];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[a][k] = cols[(wr + 16 * a + l16) * 4 + k];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      r1[b] = rows[lq * 64 + wc + 16 * b + l16];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) rr[b][k] = rows[k * 64 + wc + 16 * b + l16];
+    }
+    const double keep = piv ? 0.0 : 1.0;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) m[a][ta] *= keep;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const double inv = gj_rcp(q[p][p]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[p][j] = j == p ? inv : q[p][j] * inv;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i == p) continue;
+        const double f = q[i][p];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[i][j] = j == p ? -f * inv : fma(-f, q[p][j], q[i][j]);
+      }
+    }
+    // this lane's column and row of Q^-1
+    double qc[4], qr[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      qc[k] = pick(q[k][0], q[k][1], q[k][2], q[k][3]);
+      qr[k] = pick(q[0][k], q[1][k], q[2][k], q[3][k]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      double x = c[a][0] * qc[0];
+#pragma unroll
+      for (int k = 1; k < 4; ++k) x = fma(c[a][k], qc[k], x);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) m[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x, r1[b], m[a][b], 0, 0, 0);
+    }
+    if (own_r) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        double w = qr[0] * rr[b][0];
+#pragma unroll
+        for (int k = 1; k < 4; ++k) w = fma(qr[k], rr[b][k], w);
+        m[ta][b][s % 4] = w;
+      }
+    }
+  }
+}
+
+// the inverse of a tile in that layout, its entries beyond kk x kk replaced by the identity, into P (zero
+// beyond kk x kk: the panel products read full tiles)
+__device__ inline void gj_invert_into(gj_d4 (&m)[2][2], double* sh, int kk, int tid, double* __restrict__ P) {
+  const int lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          f(a, b, r, (wave >> 1) * 32 + 16 * a + 4 * r + lq, (wave & 1) * 32 + 16 * b + l16);
+  };
+  each([&](int a, int b, int r, int row, int col) {
+    if (row >= kk || col >= kk) m[a][b][r] = row == col ? 1.0 : 0.0;
+  });
+  gj_invert_tile(m, sh, tid);
+  each([&](int a, int b, int r, int row, int col) {
+    P[row * GJB + col] = (row < kk && col < kk) ? m[a][b][r] : 0.0;
+  });
+}
+
+// Panel copies and inverse of the first diagonal tile: block 0 inverts, block 1 + t copies tile t of the row
+// panel, block 1 + nb + t tile t of the column panel.  C[i][c] = A[i][k0 + c], R[r][j] = A[k0 + r][j].
+__global__ void __launch_bounds__(256, 2) gj_first_kernel(long long n, int nb, const double* __restrict__ A,
+                                                       double* __restrict__ P, double* __restrict__ C,
+                                                       double* __restrict__ R) {
+  __shared__ double sh[kGjShared];
+  const int tid = threadIdx.x, kk = (int)(n < GJB ? n : GJB);
+  if (blockIdx.x == 0) {
+    gj_d4 m[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = (tid >> 7) * 32 + 16 * a + 4 * r + ((tid & 63) >> 4);
+          const int col = ((tid >> 6) & 1) * 32 + 16 * b + (tid & 15);
+          m[a][b][r] = (row < kk && col < kk) ? A[row * n + col] : 0.0;
+        }
+    gj_invert_into(m, sh, kk, tid, P);
     return;
   }
-  // stage C tile (64 x kk) and R tile (kk x 64): R = new row panel, or P for the pivot columns
-  for (int q = tid; q < 64 * GJB; q += blockDim.x) {
+  const bool col = (int)blockIdx.x > nb;
+  const long long o0 = (long long)((blockIdx.x - 1) % nb) * GJB;
+  for (int q = tid; q < GJB * GJB; q += 256) {
     const int r = q / GJB, c = q % GJB;
-    const long long i = i0 + r;
-    sC[r][c] = (i < n && c < kk) ? C[i * GJB + c] : 0.0;
+    const long long i = col ? o0 + r : r, j = col ? c : o0 + c;
+    const double v = (i < n && j < n) ? A[i * n + j] : 0.0;
+    if (col && i < n) C[i * GJB + c] = v;
+    if (!col && j < n) R[r * n + j] = v;
   }
-  for (int q = tid; q < GJB * 64; q += blockDim.x) {
-    const int r = q / 64, c = q % 64;
-    const long long j = j0 + c;
-    double v = 0.0;
-    if (r < kk && j < n) v = colK ? (c < kk ? P[r * GJB + c] : 0.0) : A[(k0 + r) * n + j];
-    sR[r][c] = v;
+}
+
+__global__ void __launch_bounds__(256, 2)
+gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double* __restrict__ P, double* __restrict__ Pn,
+               const double* __restrict__ C, double* __restrict__ Cn, const double* __restrict__ R,
+               double* __restrict__ Rn) {
+  __shared__ double sA[GJB * GJL];
+  __shared__ double sB[GJB * GJL];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  // the next diagonal tile, with the inversion after its update, goes first
+  int t = blockIdx.x;
+  if (k + 1 < nb) {
+    const int next = (k + 1) * nb + k + 1;
+    t = t == 0 ? next : t == next ? 0 : t;
   }
-  __syncthreads();
-  const int tr = (tid / 16) * 4, tc = (tid % 16) * 4;
-  double acc[4][4];
+  const int bi = t / nb, bj = t % nb;
+  const bool row_k = bi == k, col_k = bj == k;
+  const long long i0 = (long long)bi * GJB, j0 = (long long)bj * GJB;
+  // 64 x 64 tile of a row-major array, zero beyond rows x cols: all 16 loads of a thread in flight at once
+  constexpr int PER = GJB * GJB / 256;
+  auto fetch = [&](double (&d)[PER], const double* src, long long ld, long long rows, long long cols) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  for (int c = 0; c < kk; ++c) {
-    double cv[4], rv[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) cv[a] = sC[tr + a][c];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) rv[b] = sR[c][tc + b];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = fma(cv[a], rv[b], acc[a][b]);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const long long i = i0 + tr + a;
-    if (i >= n) continue;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const long long j = j0 + tc + b;
-      if (j >= n) continue;
-      if (colK) {
-        if (j < k0 + kk) A[i * n + j] = -acc[a][b];
-      } else {
-        A[i * n + j] -= acc[a][b];
-      }
+    for (int u = 0; u < PER; ++u) {
+      const int r = (tid + 256 * u) / GJB, c = tid % GJB;
+      d[u] = (r < rows && c < cols) ? src[r * ld + c] : 0.0;
     }
+  };
+  auto put = [&](double* dst, const double (&d)[PER]) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) dst[(tid + 256 * u) / GJB * GJL + tid % GJB] = d[u];
+  };
+  gj_d4 acc[2][2];
+  // acc = sA sB, a wave per 32 x 32 quadrant (A: row l16, entry lq; B: entry lq, column l16)
+  auto product = [&]() {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = gj_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int k4 = 0; k4 < GJB; k4 += 4) {
+      double x[2], y[2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a) x[a] = sA[(wr + 16 * a + l16) * GJL + k4 + lq];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) y[b] = sB[(k4 + lq) * GJL + wc + 16 * b + l16];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[a], y[b], acc[a][b], 0, 0, 0);
+    }
+  };
+  double tp[PER], tr[PER], tc[PER];
+  fetch(tp, P, GJB, GJB, GJB);
+  if (!col_k) fetch(tr, R + j0, n, GJB, n - j0);
+  // entry r of acc[a][b]: row wr + 16 a + 4 r + lq, column wc + 16 b + l16
+  gj_d4 v[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const long long i = i0 + wr + 16 * a + 4 * r + lq, j = j0 + wc + 16 * b + l16;
+        v[a][b][r] = (!row_k && !col_k && i < n && j < n) ? A[i * n + j] : 0.0;
+      }
+  if (!row_k) fetch(tc, C + i0 * GJB, GJB, n - i0, GJB);
+  if (!col_k) {
+    put(sA, tp);
+    put(sB, tr);
+    __syncthreads();
+    product();  // P R_j
+    __syncthreads();
   }
+  if (!row_k) {
+    put(sA, tc);
+    if (col_k) {
+      put(sB, tp);
+    } else {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sB[(wr + 16 * a + 4 * r + lq) * GJL + wc + 16 * b + l16] = acc[a][b][r];
+    }
+    __syncthreads();
+    product();
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) v[a][b] -= acc[a][b];
+  } else {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[a][b][r] = col_k ? P[(wr + 16 * a + 4 * r + lq) * GJB + wc + 16 * b + l16] : acc[a][b][r];
+  }
+  const bool next_row = bi == k + 1, next_col = bj == k + 1;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int lr = wr + 16 * a + 4 * r + lq, lc = wc + 16 * b + l16;
+        const long long i = i0 + lr, j = j0 + lc;
+        if (i < n && j < n) A[i * n + j] = v[a][b][r];
+        if (next_row && j < n) Rn[lr * n + j] = v[a][b][r];
+        if (next_col && i < n) Cn[i * GJB + lc] = v[a][b][r];
+      }
+  if (!(next_row && next_col)) return;
+  __syncthreads();  // sB was read by the last product
+  gj_invert_into(v, sB, (int)(n - i0 < GJB ? n - i0 : GJB), tid, Pn);
 }
 
 // y = A x, one 64-lane wave per row (T = double for the FP64 V-cycle, float for FP32)
@@ -666,20 +797,20 @@ int launch_dense_from_stencil(const GridDims& g, const double* S, double* A, hip
   return check_launch("dense_from_stencil_kernel");
 }
 
-int gj_invert(long long n, double* A, double* wsP, double* wsC, hipStream_t s) {
-  const long long nb = (n + GJB - 1) / GJB;
-  for (long long kb = 0; kb < nb; ++kb) {
-    const long long k0 = kb * GJB;
-    const int kk = (int)((n - k0) < GJB ? (n - k0) : GJB);
-    gj_diag_kernel<<<1, 1024, 0, s>>>(n, k0, kk, A, wsP);
-    PMT_TRY(check_launch("gj_diag_kernel"));
-    gj_colcopy_kernel<<<blocks_for(n * kk, 256), 256, 0, s>>>(n, k0, kk, A, wsC);
-    PMT_TRY(check_launch("gj_colcopy_kernel"));
-    gj_rowpanel_kernel<<<(unsigned)((n + GJ_RP_COLS - 1) / GJ_RP_COLS), 256, 0, s>>>(n, k0, kk, A, wsP);
-    PMT_TRY(check_launch("gj_rowpanel_kernel"));
-    dim3 grid((unsigned)nb, (unsigned)nb);
-    gj_update_kernel<<<grid, 256, 0, s>>>(n, k0, kk, A, wsC, wsP);
-    PMT_TRY(check_launch("gj_update_kernel"));
+int gj_invert(long long n, double* A, double* ws, hipStream_t s) {
+  const int nb = (int)((n + GJB - 1) / GJB);
+  double *P[2], *C[2], *R[2];
+  for (int h = 0; h < 2; ++h) {  // this panel's and the next one's
+    P[h] = ws + h * GJB * GJB;
+    C[h] = ws + 2 * GJB * GJB + h * n * GJB;
+    R[h] = ws + 2 * GJB * GJB + (2 + h) * n * GJB;
+  }
+  gj_first_kernel<<<1 + 2 * nb, 256, 0, s>>>(n, nb, A, P[0], C[0], R[0]);
+  PMT_TRY(check_launch("gj_first_kernel"));
+  for (int k = 0; k < nb; ++k) {
+    const int h = k & 1;
+    gj_step_kernel<<<nb * nb, 256, 0, s>>>(n, nb, k, A, P[h], P[1 - h], C[h], C[1 - h], R[h], R[1 - h]);
+    PMT_TRY(check_launch("gj_step_kernel"));
   }
   return PMT_OK;
 }

@@ -495,7 +495,7 @@ static int hex_coarse_stencils(pmt_mg* mg, hipStream_t s) {
     PMT_TRY(launch_stencil_from_moments(Lc.g, Lc.C, Lc.M, Lc.map, Lc.dK, target(lc), s));
   PMT_HIP(hipEventRecord(mg->ev_fork, s));
   // this stream's remaining work is enqueued first (a handful of launches), so it runs while the host
-  // enqueues the ~45 launches of the inversion
+  // enqueues the launches of the inversion
   if (mg->l1free)
     PMT_TRY(launch_coarse1_xhat(mg->L[0].g, L1.g, mg->xe, L1.cflag, L1.d.Xh, mg->prec != 64 ? L1.f.Xh : nullptr, s));
   if (lc > 1)
@@ -506,7 +506,7 @@ static int hex_coarse_stencils(pmt_mg* mg, hipStream_t s) {
   }
   PMT_HIP(hipStreamWaitEvent(mg->s2, mg->ev_fork, 0));
   PMT_TRY(launch_dense_from_stencil(Lc.g, Lc.d.S, mg->Ainv, mg->s2));
-  PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjP, mg->gjC, mg->s2));
+  PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjw, mg->s2));
   PMT_HIP(hipEventRecord(mg->ev_join, mg->s2));
   // joined by the first coarsest solve on each stream: the V-cycle descent before it hides the inversion
   mg->pending_join = true;
@@ -620,8 +620,7 @@ int pmt_mg_create(int nelx, int nely, int nelz, int nlevels, const double* omega
     }
   }
   ALLOC(mg->Ainv, mg->nc * mg->nc);
-  ALLOC(mg->gjP, 64 * 64);
-  ALLOC(mg->gjC, mg->nc * 64);
+  ALLOC(mg->gjw, gj_work_size(mg->nc));
   const long long n0 = mg->L[0].ndof;
   ALLOC(mg->p, n0);
   ALLOC(mg->q, n0);
@@ -745,7 +744,7 @@ int pmt_mg_update(pmt_mg* mg, const double* xe, const uint8_t* bcmask, double bc
   if (mg->dim != 3) {  // hex8: inverted on the second stream inside hex_coarse_stencils
     Level& Cl = mg->L[mg->nlev - 1];
     PMT_TRY(launch_dense_from_stencil(Cl.g, Cl.d.S, mg->Ainv, s));
-    PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjP, mg->gjC, s));
+    PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjw, s));
   }
   if (mg->smoother == 1) {
     for (int l = 0; l < mg->nlev - 1; ++l) {

@@ -93,8 +93,7 @@ struct pmt_mg {
   // streams that have waited since the last update are listed, so each waits once and none is skipped
   bool pending_join = false;
   std::vector<hipStream_t> joined;
-  double* gjP = nullptr;
-  double* gjC = nullptr;
+  double* gjw = nullptr;  // workspace of the coarsest inversion
   float* z32 = nullptr;  // FP32 V-cycle output on the fine grid
   double* p = nullptr;
   double* q = nullptr;

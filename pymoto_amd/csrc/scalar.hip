@@ -22,12 +22,6 @@
 
 namespace pmt {
 
-int gj_invert(long long n, double* A, double* wsP, double* wsC, hipStream_t s);
-template <typename T>
-int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s);
-int launch_dot(long long n, const double* x, const double* y, double* out, double* work, hipStream_t s);
-int launch_axpby(long long n, double a, const double* x, double b, double* y, hipStream_t s);
-
 namespace {
 
 constexpr int kScalarMaxLevels = 12;
@@ -405,8 +399,7 @@ struct pmt_smg {
   double* t[kScalarMaxLevels] = {};  // work
   double* P0 = nullptr;              // element matrix (device)
   double* Ainv = nullptr;            // coarsest inverse
-  double* gjP = nullptr;
-  double* gjC = nullptr;
+  double* gjw = nullptr;             // workspace of its inversion
   const double* xe = nullptr;
   const uint8_t* bcm = nullptr;
   double bcdiag = 0.0;
@@ -562,8 +555,7 @@ int pmt_smg_create(int nelx, int nely, int nelz, int nlevels, const double* omeg
     }
   }
   A(&h->Ainv, nc * nc);
-  A(&h->gjP, 64 * nc + 64 * 64);
-  A(&h->gjC, 64 * nc);
+  A(&h->gjw, gj_work_size(nc));
   const long long n0 = h->g[0].nnodes;
   A(&h->r, n0);
   A(&h->z, n0);
@@ -625,7 +617,7 @@ int pmt_smg_update(pmt_smg* h, const double* xe, const uint8_t* bcmask, double b
   else
     scalar_dense_kernel<2><<<blocks_for(nc, 128), 128, 0, s>>>(h->g[L], h->S[L], h->Ainv);
   PMT_TRY(check_launch("scalar_dense_kernel"));
-  PMT_TRY(gj_invert(nc, h->Ainv, h->gjP, h->gjC, s));
+  PMT_TRY(gj_invert(nc, h->Ainv, h->gjw, s));
   h->ready = true;
   return PMT_OK;
 }
