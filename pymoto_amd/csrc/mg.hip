@@ -185,6 +185,29 @@ static double first_sweep_factor(const pmt_mg* mg, int l) {
   return mg->smoother == 0 ? L.omega : 1.0 / (0.5 * (L.cheb_hi + L.cheb_lo));
 }
 
+// the coefficients of smooth()'s sweeps on level l (from zero the first one is a[0] D^-1 b)
+static Sweeps2 sweep_coefficients(const pmt_mg* mg, int l) {
+  const Level& L = mg->L[l];
+  Sweeps2 sw{};
+  sw.n = L.steps;
+  const double theta = 0.5 * (L.cheb_hi + L.cheb_lo), delta = 0.5 * (L.cheb_hi - L.cheb_lo);
+  const double sigma = theta / delta;
+  double rho_prev = 1.0 / sigma;
+  for (int k = 0; k < sw.n; ++k) {
+    if (mg->smoother == 0) {
+      sw.a[k] = L.omega;
+    } else if (k == 0) {
+      sw.a[k] = 1.0 / theta;
+    } else {
+      const double rho = 1.0 / (2.0 * sigma - rho_prev);
+      sw.a[k] = 2.0 * rho / delta;
+      sw.b[k] = rho * rho_prev;
+      rho_prev = rho;
+    }
+  }
+  return sw;
+}
+
 // out = V-cycle(b) on level l (GeometricMultigrid.solve with x0 = None, iterative.py:222-256)
 template <typename T>
 static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool first_done = false) {
@@ -193,6 +216,12 @@ static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool fir
   Level& C = mg->L[l + 1];
   LevelBuf<T>& B = L.buf<T>();
   LevelBuf<T>& CB = C.buf<T>();
+  if (v2_ok(mg, L.steps)) {  // Q4: all sweeps of a visit in one launch
+    const Sweeps2 sw = sweep_coefficients(mg, l);
+    PMT_TRY(launch_v2_down<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.b, s));
+    PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s));
+    return launch_v2_up<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.u, out, s);
+  }
   // 2*steps-1 out-of-place sweeps follow the first one: start in the buffer that ends in `out`
   T* cur = B.t;
   T* oth = out;

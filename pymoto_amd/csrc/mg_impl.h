@@ -124,6 +124,22 @@ struct pmt_mg {
 
 namespace pmt {
 
+// vcycle2d.hip: the smoothing sweeps of a Q4 level's visit in one launch.  Sweep k is
+// u + a[k] D^-1 (b - A u) + b[k] (u - u_prev), the first one of `down` from zero: u = a[0] D^-1 b.
+constexpr int kV2MaxSweeps = 10;
+struct Sweeps2 {
+  int n;
+  double a[kV2MaxSweeps], b[kV2MaxSweeps];
+};
+bool v2_ok(const pmt_mg* mg, int steps);
+// u = the sweeps from zero on level l, bc = R^T (b - A u)
+template <typename T>
+int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s);
+// uo = the sweeps from ui + R ec (uo must not be ui)
+template <typename T>
+int launch_v2_up(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, const T* ui, const T* ec, T* uo,
+                 hipStream_t s);
+
 // frees the block-CG workspace and graphs of a handle (blockcg.hip)
 void block_cg_release(pmt_mg* mg);
 // drops captured block-CG iterations (after an update or a change of precision or launch shapes)
