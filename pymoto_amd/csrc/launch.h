@@ -127,6 +127,12 @@ int launch_scale_rsqrt(long long n, const double* sc, int k, const double* z, do
 int launch_fill(long long n, double v, double* y, hipStream_t s);
 // host[0] = *v, then host[1] = seq (pinned host memory; the host polls host[1])
 int launch_publish(const double* v, double seq, double* host, hipStream_t s);
+// a sequence number unique in the process: pinned memory freed by another handle (with its last number still in
+// it) and handed out again can never look like the publish it is used for
+double publish_sequence();
+// polls host[1] for seq, then *v = host[0]; after 1 s without it, *v through the synchronising copy of *dev into
+// *pinned, so a value that never arrives cannot hang the caller
+int publish_wait(const double* host, double seq, const double* dev, double* pinned, double* v, hipStream_t s);
 int launch_to_double(long long n, const float* x, double* y, hipStream_t s);
 
 // coarse.hip

@@ -17,8 +17,6 @@
 // with BF16 operands and FP32 accumulation (hex8 only); the fine residual that is restricted to the
 // coarse grid stays FP32, so the coarse correction sees no BF16 rounding.
 #include <algorithm>
-#include <atomic>
-#include <chrono>
 #include <cmath>
 #include <limits>
 #include <new>
@@ -258,27 +256,13 @@ static int precondition(pmt_mg* mg, const double* r, double* z, hipStream_t s) {
   return launch_to_double(mg->L[0].ndof, mg->z32, z, s);
 }
 
-static int read_scalar(pmt_mg* mg, int k, double* v, hipStream_t s) {
-  PMT_HIP(hipMemcpyAsync(mg->host_sc + k, mg->sc + k, sizeof(double), hipMemcpyDeviceToHost, s));
-  PMT_HIP(hipStreamSynchronize(s));
-  *v = mg->host_sc[k];
-  return PMT_OK;
-}
-
 // The CG stopping test without a stream synchronisation (whose wake-up left the GPU idle for ~60 us per
 // iteration): a one-thread kernel (publish_scalar) stores sc[k] and then a fresh sequence number into
 // pinned memory, and the host polls for that sequence number (wait_published).  Work enqueued between
-// the two keeps the GPU busy.  After 1 s without it the host falls back to the synchronising read, so a
-// value that never arrives cannot hang the solve.
-static std::atomic<long long> g_publish_seq{0};
+// the two keeps the GPU busy.
 
-// the sequence number of the next publish (kept for wait_published); unique in the process: pinned memory
-// freed by another handle (with its last sequence number still in it) and handed out again here can
-// never look like this publish
-static double next_publish_seq(pmt_mg* mg) {
-  mg->pub_seq = (double)g_publish_seq.fetch_add(1, std::memory_order_relaxed) + 1.0;
-  return mg->pub_seq;
-}
+// the sequence number of the next publish (kept for wait_published)
+static double next_publish_seq(pmt_mg* mg) { return mg->pub_seq = publish_sequence(); }
 
 static int publish_scalar(pmt_mg* mg, int k, hipStream_t s) {
   const double seq = next_publish_seq(mg);
@@ -286,16 +270,7 @@ static int publish_scalar(pmt_mg* mg, int k, hipStream_t s) {
 }
 
 static int wait_published(pmt_mg* mg, int k, double* v, hipStream_t s) {
-  volatile double* h = mg->host_rr;
-  const double want = mg->pub_seq;
-  const auto t0 = std::chrono::steady_clock::now();
-  for (;;) {
-    if (h[1] == want) {
-      *v = h[0];
-      return PMT_OK;
-    }
-    if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) return read_scalar(mg, k, v, s);
-  }
+  return publish_wait(mg->host_rr, mg->pub_seq, mg->sc + k, mg->host_sc + k, v, s);
 }
 
 static int alloc_fp32(pmt_mg* mg) {

@@ -5,6 +5,8 @@
 // partials in a caller workspace, and a single-block second stage summing the partials in a
 // fixed order, so every dot product is bit-reproducible run to run.
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -507,6 +509,28 @@ int launch_cg_xr_update(long long n, const double* sc, const double* p, const do
   PMT_TRY(check_launch("cg_xr_update"));
   parts_stage2<<<1, kStage2Threads, 0, s>>>(work, parts, out_rr, seq, host);
   return check_launch("parts_stage2");
+}
+
+double publish_sequence() {
+  static std::atomic<long long> seq{0};
+  return (double)seq.fetch_add(1, std::memory_order_relaxed) + 1.0;
+}
+
+int publish_wait(const double* host, double seq, const double* dev, double* pinned, double* v, hipStream_t s) {
+  const volatile double* h = host;
+  const auto t0 = std::chrono::steady_clock::now();
+  for (;;) {
+    if (h[1] == seq) {
+      *v = h[0];
+      return PMT_OK;
+    }
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) {
+      PMT_HIP(hipMemcpyAsync(pinned, dev, sizeof(double), hipMemcpyDeviceToHost, s));
+      PMT_HIP(hipStreamSynchronize(s));
+      *v = *pinned;
+      return PMT_OK;
+    }
+  }
 }
 
 // v -> host-visible memory (pinned): host[0] = value, then (after a system-scope fence) host[1] = seq, so a
