@@ -615,41 +615,42 @@ __global__ void jacobi0_kernel(long long n, const T* __restrict__ dinv, const T*
   if (q < n) u[q] = omega * dinv[q] * b[q];
 }
 
-// rc = R^T rf : coarse node gathers the 3^D fine nodes around its fine image (weights 1, 1/2, 1/4, 1/8).
+// rc = R^T rf : coarse node gathers the 3^D fine nodes around its fine image (weights 1, 1/2, 1/4, 1/8), one thread
+// per dof.  Every lane reads 3^D values, a fine node outside the grid replaced by the centre with weight 0: a
+// branch around a load would wait for each in turn (8 us on the smallest grids; RESTR_FIG).
 // u0 (optional): also the coarse level's first smoothing sweep from zero, u0 = w0 D^-1 rc (the
 // expression of jacobi0_kernel, so the bits are the same as a separate launch)
 template <int DIM, typename T>
 __global__ void restrict_kernel(GridDims gf, GridDims gc, const T* __restrict__ rf, T* __restrict__ rc,
                                 const T* __restrict__ dinv, T w0, T* __restrict__ u0) {
-  const long long N = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (N >= gc.nnodes) return;
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= gc.nnodes * DIM) return;
+  const long long N = q / DIM;
+  const int d = (int)(q - N * DIM);
   const int I = (int)(N % gc.nx);
   const long long t = N / gc.nx;
   const int J = (int)(t % gc.ny);
   const int K = (int)(t / gc.ny);
-  T acc[DIM];
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) acc[d] = 0;
   constexpr int ZLO = DIM == 3 ? -1 : 0, ZHI = DIM == 3 ? 1 : 0;
+  const T* centre = rf + (((long long)(DIM == 3 ? 2 * K : 0) * gf.ny + 2 * J) * gf.nx + 2 * I) * DIM + d;
+  const long long sy = (long long)gf.nx * DIM, sz = sy * gf.ny;
+  // the axes' weights beside the centre, and its steps
+  const T wx[3] = {(T)(I > 0 ? 0.5 : 0.0), (T)1, (T)(2 * I + 1 < gf.nx ? 0.5 : 0.0)};
+  const T wy[3] = {(T)(J > 0 ? 0.5 : 0.0), (T)1, (T)(2 * J + 1 < gf.ny ? 0.5 : 0.0)};
+  const T wz[3] = {(T)(K > 0 ? 0.5 : 0.0), (T)1, (T)(2 * K + 1 < gf.nz ? 0.5 : 0.0)};
+  T acc = 0;
 #pragma unroll
   for (int dz = ZLO; dz <= ZHI; ++dz)
 #pragma unroll
     for (int dy = -1; dy <= 1; ++dy)
 #pragma unroll
       for (int dx = -1; dx <= 1; ++dx) {
-        const int fi = 2 * I + dx, fj = 2 * J + dy, fk = 2 * K + dz;
-        if (fi < 0 || fi >= gf.nx || fj < 0 || fj >= gf.ny || fk < 0 || fk >= gf.nz) continue;
-        const T w = (T)((dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0));
-        const long long m = ((long long)fk * gf.ny + fj) * gf.nx + fi;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) acc[d] = fma(w, rf[m * DIM + d], acc[d]);
+        const T w = wx[dx + 1] * wy[dy + 1] * wz[dz + 1];
+        const long long o = (wx[dx + 1] != 0 ? dx * DIM : 0) + (wy[dy + 1] != 0 ? dy * sy : 0) + (wz[dz + 1] != 0 ? dz * sz : 0);
+        acc = fma(w, centre[o], acc);
       }
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) rc[N * DIM + d] = acc[d];
-  if (u0) {
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) u0[N * DIM + d] = w0 * dinv[N * DIM + d] * acc[d];
-  }
+  rc[q] = acc;
+  if (u0) u0[q] = w0 * dinv[q] * acc;
 }
 
 // uf += R uc : fine node interpolates from the 1, 2, 4 or 8 coarse nodes around it.  Branch free: every
@@ -1010,7 +1011,7 @@ int launch_jacobi0(long long n, const T* dinv, const T* b, double omega, T* u, h
 template <typename T>
 int launch_restrict(const GridDims& gf, const GridDims& gc, const T* rf, T* rc, hipStream_t s, const T* dinv,
                     double w0, T* u0) {
-  dim3 grid(blocks_for(gc.nnodes, 256));
+  dim3 grid(blocks_for(gc.nnodes * gc.dim, 256));
   if (gf.dim == 3)
     restrict_kernel<3, T><<<grid, 256, 0, s>>>(gf, gc, rf, rc, dinv, (T)w0, u0);
   else
