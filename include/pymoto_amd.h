@@ -186,9 +186,9 @@ int pmt_k0_extend(int dim, const double* K0_host, double* ext_host);
  * PMT_TUNE_STREAM_PLANES: node planes per streamed column, 0 = chosen from the CU count (default).
  * PMT_TUNE_STREAM_TILE: streamed column shape, 0 = 32x8 (default), 1 = 64x4, 2 = 16x16 nodes.
  * PMT_TUNE_COARSE1: operator of the first coarse level of hex8 hierarchies, 1 = element by element in
- * the reflection basis from the transformed child densities, no stencil stored (default; used when
- * k0_pattern has PMT_K0_REFLECTION and the level is not the coarsest), 0 = half stencil.  Read by
- * pmt_mg_create: it applies to hierarchies created afterwards.
+ * the reflection basis from the transformed child densities, no stencil stored (used when k0_pattern has
+ * PMT_K0_REFLECTION and the level is not the coarsest), 0 = half stencil, 2 = 1 for levels of more than
+ * 100,000 nodes, else 0 (default).  Read by pmt_mg_create: it applies to hierarchies created afterwards.
  * PMT_TUNE_FILTER: FilterConv kernels for extents k x k x kz up to 15 whose box of outputs fits LDS, 1 = boxes
  * staged in LDS (default), 0 = one thread per element gathering through the caches; both sum the taps in
  * the same order.

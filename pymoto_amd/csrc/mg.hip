@@ -536,7 +536,15 @@ int pmt_mg_create(int nelx, int nely, int nelz, int nlevels, const double* omega
   mg->NE = (1 << mg->dim) * mg->dim;
   std::vector<double> K0ext(PMT_K0_EXT_LEN);
   mg->k0pat = pmt_k0_extend(mg->dim, K0_host, K0ext.data());
-  mg->l1free = mg->dim == 3 && nlevels >= 3 && (mg->k0pat & PMT_K0_REFLECTION) && get_tuning(PMT_TUNE_COARSE1) == 1;
+  // Level 1 of a hex8 hierarchy: applied from the child densities in the reflection basis (least memory and
+  // traffic), or as a stored half stencil where that many coefficients are fetched faster than the transforms
+  // run.  V-cycle of 2 + 2 sweeps, stencil-free / stored, FP64 and FP32: level 1 of 30,625 nodes 164 / 128 and
+  // 149 / 108 us, 70,785 nodes 235 / 219 and 190 / 170 us, 122,713 nodes 309 / 321 and 227 / 215 us, 213,689
+  // nodes 443 / 522 and 301 / 315 us, 545,025 nodes 989 / 1311 and 608 / 746 us.
+  const long long nodes1 = (nelx / 2 + 1LL) * (nely / 2 + 1) * (nelz / 2 + 1);
+  const int coarse1 = get_tuning(PMT_TUNE_COARSE1);
+  mg->l1free = mg->dim == 3 && nlevels >= 3 && (mg->k0pat & PMT_K0_REFLECTION) &&
+               (coarse1 == 2 ? nodes1 > kStoredLevel1Nodes : coarse1 == 1);
   mg->lmax_elem = element_lmax(mg->NE, K0_host);
   int ex = nelx, ey = nely, ez = nelz;
   for (int l = 0; l < nlevels; ++l) {

@@ -10,6 +10,8 @@ namespace pmt {
 constexpr int kMaxLevels = 12;
 struct BlockCG;
 
+constexpr long long kStoredLevel1Nodes = 100000;  // level-1 nodes up to which its half stencil is stored
+
 template <typename T>
 struct LevelBuf {
   T* dinv = nullptr;  // inverse diagonal (levels above the coarsest)

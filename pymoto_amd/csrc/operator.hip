@@ -598,6 +598,83 @@ stencil_half_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ u
   }
 }
 
+// Small grids of hex8 nodes: nine wavefronts per 64 nodes, wave r holding the row r of three neighbours,
+// so the 36 loads of a row are all in flight at once and the nine rows in parallel instead of one after the
+// other; the rows' sums meet in LDS and three waves (one per component) finish the nodes.  A sweep costs the
+// latency of one row (stencil_half_kernel that of nine): 225 to 9,537 nodes 4.6 us in FP32 (6.5 to 7.1), 4,225
+// nodes 4.9 us in FP64 (11.0), 70,785 nodes 12.4 us in FP32 (12.9).  Above that the coefficients stream from
+// memory and both run at its rate.
+constexpr long long kSplitNodes = 100000;
+
+template <int MODE, typename T>
+__global__ void __launch_bounds__(576)
+stencil_split_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ u, const T* __restrict__ b,
+                     const T* __restrict__ dinv, T omega, T* y, const T* up, T beta) {
+  constexpr int TS = (int)sizeof(T);
+  constexpr int C = Half<3>::C;
+  __shared__ T sum[9][3][64];
+  const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int nn = (int)g.nnodes;
+  const int n = (int)xcd_block() * 64 + lane;
+  const int i = n % g.nx, t = n / g.nx, j = t % g.ny, k = t / g.ny;
+  const int dy = r % 3 - 1, dz = r / 3 - 1;
+  const bool live = n < nn;
+  const __amdgpu_buffer_rsrc_t ru = plane_rsrc(u, 0, 3LL * nn, true);
+  // operands of the update, one wave per component
+  const int oq = live ? (3 * n + (r < 3 ? r : 0)) * TS : kOOB;
+  T uq = 0, bq = 0, dq = 0, pq = 0;
+  if (r < 3) {
+    if (MODE == MODE_JACOBI || MODE == MODE_CHEB) {
+      uq = bload(ru, oq, T());
+      dq = bload(plane_rsrc(dinv, 0, 3LL * nn, true), oq, T());
+    }
+    if (MODE != MODE_APPLY) bq = bload(plane_rsrc(b, 0, 3LL * nn, true), oq, T());
+    if (MODE == MODE_CHEB) pq = bload(plane_rsrc(up, 0, 3LL * nn, up != nullptr), oq, T());
+  }
+  T v[3][12];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int o = r * 3 + q;
+    const int ii = i + q - 1, jj = j + dy, kk = k + dz;
+    const bool in = live && ii >= 0 && ii < g.nx && jj >= 0 && jj < g.ny && kk >= 0 && kk < g.nz;
+    const int m = n + q - 1 + (dz * g.ny + dy) * g.nx;
+    // forward: block (n, m), stored at n; backward: transpose of m's block of the mirrored offset
+    const bool fwd = o >= C;
+    const int oh = in ? (fwd ? n : m) * TS : kOOB, ou = in ? 3 * m * TS : kOOB;
+    const int c0 = (fwd ? o - C : C - o) * 9, sd = fwd ? 3 : 1, sd2 = fwd ? 1 : 3;
+#pragma unroll
+    for (int d2 = 0; d2 < 3; ++d2) v[q][d2] = bload(ru, ou + d2 * TS, T());
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+      for (int d2 = 0; d2 < 3; ++d2)
+        v[q][3 + d * 3 + d2] = bload(plane_rsrc(H, (long long)(c0 + d * sd + d2 * sd2) * nn, nn, true), oh, T());
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    T acc = 0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int d2 = 0; d2 < 3; ++d2) acc = fma(v[q][3 + d * 3 + d2], v[q][d2], acc);
+    sum[r][d][lane] = acc;
+  }
+  __syncthreads();
+  if (r >= 3 || !live) return;
+  T out = 0;
+#pragma unroll
+  for (int w = 0; w < 9; ++w) out += sum[w][r][lane];
+  const long long q = 3LL * n + r;
+  if (MODE == MODE_APPLY)
+    y[q] = out;
+  else if (MODE == MODE_RESIDUAL)
+    y[q] = bq - out;
+  else if (MODE == MODE_JACOBI)
+    y[q] = uq + omega * dq * (bq - out);
+  else
+    y[q] = uq + omega * dq * (bq - out) + beta * (uq - pq);
+}
+
 template <int DIM, typename T>
 __global__ void stencil_diag_kernel(GridDims g, const double* __restrict__ S, T* __restrict__ dinv) {
   const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -754,7 +831,7 @@ extern int g_filter_tiled;  // filter.hip
 // Launch-shape tuning of the fine operator (set by pmt_set_tuning; read at every launch).
 static int g_fine_kernel = 2;  // 0 = 3D tiles, 1 = z-streamed columns, 2 = reflection basis (if available)
 static int g_refl_rows = 16;   // block shape of the reflection-basis kernel (node rows per block; 0 = by grid)
-static int g_coarse1 = 1;      // hex8 level 1 without a stencil (reflection basis), new hierarchies
+static int g_coarse1 = 2;      // hex8 level 1 of new hierarchies: 0 stored, 1 without a stencil, 2 by its size
 static int g_stream_nzc = 0;   // node planes per streamed block (0 = chosen from the CU count)
 static int g_stream_tile = 0;  // streamed column shape: 0 = 32x8, 1 = 64x4, 2 = 16x16 nodes
 
@@ -783,7 +860,7 @@ int set_tuning(int param, int value) {
     ++g_tuning_epoch;
     return 0;
   }
-  if (param == PMT_TUNE_COARSE1 && (value == 0 || value == 1)) {
+  if (param == PMT_TUNE_COARSE1 && value >= 0 && value <= 2) {
     g_coarse1 = value;
     ++g_tuning_epoch;
     return 0;
@@ -946,6 +1023,19 @@ int launch_stencil_half(int mode, const GridDims& g, const T* H, const T* u, con
   dim3 grid(xcd_blocks(g.nnodes, 256));
   const T om = (T)omega, be = (T)beta;
 #define PMT_HALF(D, M) stencil_half_kernel<D, M, T><<<grid, 256, 0, s>>>(g, H, u, b, dinv, om, y, up, be)
+#define PMT_SPLIT(M) stencil_split_kernel<M, T><<<xcd_blocks(g.nnodes, 64), 576, 0, s>>>(g, H, u, b, dinv, om, y, up, be)
+  if (g.dim == 3 && g.nnodes <= kSplitNodes) {
+    if (mode == MODE_APPLY)
+      PMT_SPLIT(MODE_APPLY);
+    else if (mode == MODE_RESIDUAL)
+      PMT_SPLIT(MODE_RESIDUAL);
+    else if (mode == MODE_JACOBI)
+      PMT_SPLIT(MODE_JACOBI);
+    else
+      PMT_SPLIT(MODE_CHEB);
+    return check_launch("stencil_split_kernel");
+  }
+#undef PMT_SPLIT
   if (g.dim == 3) {
     if (mode == MODE_APPLY)
       PMT_HALF(3, MODE_APPLY);

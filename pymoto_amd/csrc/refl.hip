@@ -697,7 +697,9 @@ static int refl_resident_blocks() {
 // Planes per block.  Every CU runs `resident` blocks at once; the launch takes
 // ceil(blocks / (CUs * resident)) rounds of (planes + 1) layers (one prologue layer per block).
 // Minimise that, among the chunkings that still give every CU at least two resident blocks (latency
-// hiding) whenever the grid allows it; ties go to the fewer blocks.
+// hiding) whenever the grid allows it; ties go to the fewer blocks.  One plane per block on grids that cannot
+// fill the CUs otherwise: level 1 of 30,625 nodes in FP64 12.0 us per sweep (two planes 15.3), of 70,785 nodes
+// in FP32 11.8 us (13.8).
 static int refl_planes(int nxy, int nz, int resident) {
   const long long cus = device_cu_count();
   const long long slots = cus * (resident > 0 ? resident : 1);
@@ -705,7 +707,7 @@ static int refl_planes(int nxy, int nz, int resident) {
   int best = 0;
   long long best_cost = -1;
   for (int pass = 0; pass < 2 && best == 0; ++pass)
-    for (int c = nz; c >= 2; --c) {
+    for (int c = nz; c >= 1; --c) {
       const long long blocks = (long long)nxy * ((nz + c - 1) / c);
       if (pass == 0 && blocks < want) continue;
       const long long cost = ((blocks + slots - 1) / slots) * (c + 1);
@@ -1002,7 +1004,7 @@ int launch_sens_stream(const GridDims& g, const double* tab, const uint8_t* bcm,
 //  1. coarse1_touched_kernel: thread = (listed element, corner); it lists the corner's node if no
 //     flagged element holding the node has a smaller index (the list's order is irrelevant);
 //  2. coarse1_tstencil_kernel: thread = (touched node, coefficient), T in [243][cap] layout;
-//  3. coarse1_tapply_kernel: four lanes per (touched node, component), 27 multiply-adds each.
+//  3. coarse1_tapply_kernel: nine wavefronts per 64 touched nodes, one row of three neighbours each.
 __global__ void __launch_bounds__(256)
 coarse1_touched_kernel(GridDims g, const int* __restrict__ list, const int* __restrict__ count,
                        const int* __restrict__ map, int* __restrict__ tnode, int* __restrict__ tcount) {
@@ -1052,45 +1054,53 @@ coarse1_tstencil_kernel(GridDims g, const int* __restrict__ tnode, int nt, long 
   T[(long long)c * cap + t] = v;
 }
 
-// Four lanes per (touched node, component): lane g < 3 sums the 9 neighbours of the z offset g - 1 (27
-// multiply-adds), the fourth idles, and the group (aligned in the wave) adds its three sums in order -
-// 4x the threads of one lane per output (latency: 81 dependent loads and multiply-adds per lane then).
+// Nine wavefronts per 64 touched nodes, wave r holding the row r of three neighbours: its 27 coefficients
+// (consecutive nodes in consecutive lanes) and 9 values are in flight together, the rows' sums meet in LDS and
+// three waves (one per component) add them in order.  The 1.9 KB of FP64 coefficients per node bound it: 8,450
+// nodes (16 MB) 7.4 us (four lanes per (node, component), fetching the coefficients in short pieces: 8.6 us).
 template <int MODE, typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(576)
 coarse1_tapply_kernel(GridDims g, const int* __restrict__ tnode, int nt, long long cap, const double* __restrict__ TS,
                       const T* __restrict__ u, const T* __restrict__ dinv, double omega, T* __restrict__ y) {
-  const long long q4 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int grp = (int)(q4 & 3);
-  const long long q = q4 >> 2;
-  const bool live = q < 3LL * nt;
-  const long long t = live ? q / 3 : 0;
-  const int d = (int)(q % 3);
-  const long long n = tnode[t];
-  const int I = (int)(n % g.nx);
-  const long long tt = n / g.nx;
-  const int J = (int)(tt % g.ny), K = (int)(tt / g.ny);
-  double acc = 0.0;
-  if (live && grp < 3) {
+  __shared__ double sum[9][3][64];
+  const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int t = (int)blockIdx.x * 64 + lane, tc = min(t, nt - 1);  // lanes past the end repeat the last node
+  const int n = tnode[tc];
+  const int I = n % g.nx, tt = n / g.nx, J = tt % g.ny, K = tt / g.ny;
+  const long long q = 3LL * n + (r < 3 ? r : 0);
+  const double y0 = r < 3 ? (double)y[q] : 0.0;
+  const double d0 = r < 3 && MODE == MODE_JACOBI ? (double)dinv[q] : 0.0;
+  // neighbours outside the grid have zero coefficients: read a clamped (valid) node instead
+  const int nj = min(max(J + r % 3 - 1, 0), g.ny - 1), nk = min(max(K + r / 3 - 1, 0), g.nz - 1);
+  double c[3][9];
+  T v[3][3];
 #pragma unroll
-    for (int oo = 0; oo < 9; ++oo) {
-      const int o = grp * 9 + oo;
-      // neighbours outside the grid have zero coefficients: read a clamped (valid) node instead
-      const int ni = min(max(I + o % 3 - 1, 0), g.nx - 1), nj = min(max(J + (o / 3) % 3 - 1, 0), g.ny - 1),
-                nk = min(max(K + o / 9 - 1, 0), g.nz - 1);
-      const long long m = ((long long)nk * g.ny + nj) * g.nx + ni;
+  for (int x = 0; x < 3; ++x) {
+    const long long m = ((long long)nk * g.ny + nj) * g.nx + min(max(I + x - 1, 0), g.nx - 1);
 #pragma unroll
-      for (int d2 = 0; d2 < 3; ++d2)
-        acc = fma(TS[(long long)((o * 3 + d) * 3 + d2) * cap + t], (double)u[m * 3 + d2], acc);
-    }
+    for (int d2 = 0; d2 < 3; ++d2) v[x][d2] = u[m * 3 + d2];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) c[x][k] = TS[(long long)((r * 3 + x) * 9 + k) * cap + tc];
   }
-  const double a1 = __shfl_down(acc, 1, 64), a2 = __shfl_down(acc, 2, 64);  // within the aligned group of 4
-  if (!live || grp != 0) return;
-  double f = (acc + a1) + a2;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    double acc = 0.0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+#pragma unroll
+      for (int d2 = 0; d2 < 3; ++d2) acc = fma(c[x][d * 3 + d2], (double)v[x][d2], acc);
+    sum[r][d][lane] = acc;
+  }
+  __syncthreads();
+  if (r >= 3 || t >= nt) return;
+  double f = 0.0;
+#pragma unroll
+  for (int w = 0; w < 9; ++w) f += sum[w][r][lane];
   if (MODE == MODE_RESIDUAL)
     f = -f;
-  else if (MODE == MODE_JACOBI || MODE == MODE_CHEB)
-    f = -omega * (double)dinv[n * 3 + d] * f;
-  y[n * 3 + d] = (T)((double)y[n * 3 + d] + f);
+  else if (MODE == MODE_JACOBI)
+    f = -omega * d0 * f;
+  y[q] = (T)(y0 + f);
 }
 
 int launch_coarse1_touched(const GridDims& g, const int* list, const int* map, int* tnode, int* tcount,
@@ -1121,13 +1131,13 @@ int launch_coarse1(int mode, const GridDims& g, int pattern, const double* G0ext
     launch_refl_shape<1, 16, 16, 0, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be);
   PMT_TRY(check_launch("fine_refl_kernel<coarse level 1>"));
   if (nt <= 0) return PMT_OK;
-  const unsigned blocks = (unsigned)blocks_for(12LL * nt, 256);  // 4 lanes per (node, component)
+  const unsigned blocks = (unsigned)blocks_for(nt, 64);
   if (mode == MODE_APPLY)
-    coarse1_tapply_kernel<MODE_APPLY, T><<<blocks, 256, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
+    coarse1_tapply_kernel<MODE_APPLY, T><<<blocks, 576, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
   else if (mode == MODE_RESIDUAL)
-    coarse1_tapply_kernel<MODE_RESIDUAL, T><<<blocks, 256, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
+    coarse1_tapply_kernel<MODE_RESIDUAL, T><<<blocks, 576, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
   else
-    coarse1_tapply_kernel<MODE_JACOBI, T><<<blocks, 256, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
+    coarse1_tapply_kernel<MODE_JACOBI, T><<<blocks, 576, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
   return check_launch("coarse1_tapply_kernel");
 }
 

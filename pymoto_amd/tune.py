@@ -39,8 +39,10 @@ def set_tuning(fine_kernel=None, stream_tile=None, stream_planes=None, refl_rows
 
 def set_coarse_level1(stencil_free=True):
     """Operator of the first coarse level of hex8 hierarchies created from now on: element by element in
-    the reflection basis of K0 (default) or the stored half stencil."""
-    _lib.check(_lib.lib().pmt_set_tuning(COARSE1, 1 if stencil_free else 0), "set tuning")
+    the reflection basis of K0 (True), the stored half stencil (False), or the faster one for the level's
+    size (None; what holds until this is called)."""
+    _lib.check(_lib.lib().pmt_set_tuning(COARSE1, 2 if stencil_free is None else 1 if stencil_free else 0),
+               "set tuning")
 
 
 def candidates(nz, reflection=True):
