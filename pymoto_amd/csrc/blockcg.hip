@@ -30,9 +30,11 @@ namespace pmt {
 
 constexpr int kMaxRhs = 8;
 
-struct VecSet {
-  const double* v[kMaxRhs];
+template <typename T>
+struct VecSetT {
+  const T* v[kMaxRhs];
 };
+using VecSet = VecSetT<double>;
 struct OutSet {
   double* v[kMaxRhs];
 };
@@ -75,6 +77,10 @@ struct BlockCG {
   // captured iterations: [0] operator + alpha + restart residual, [1] same with recurrence, [2] beta + orth
   hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   int graph_k = 0, graph_epoch = -1;
+  // vectors of the V-cycle of kcap columns in the precision `vec_prec` (64 or 32), null if they did not fit
+  void* vec = nullptr;
+  int vec_prec = 0;
+  float* z32 = nullptr;
   // captured work runs on a stream of the handle (the caller's may be the legacy default stream,
   // which cannot be captured), ordered after and before the caller's stream with two events
   hipStream_t cs = nullptr;
@@ -135,14 +141,14 @@ __device__ __forceinline__ void sum_entries(const double* __restrict__ partial, 
 }
 
 // partial sums of A^T B1 (entry a * K + b) and, NB == 2, of A^T B2 (entry K * K + a * K + b)
-template <int K, int NB>
+template <int K, int NB, typename T>
 __global__ void __launch_bounds__(256)
-gram_kernel(long long n, VecSet A, VecSet B1, VecSet B2, double* __restrict__ partial) {
+gram_kernel(long long n, VecSet A, VecSetT<T> B1, VecSetT<T> B2, double* __restrict__ partial) {
   double acc[NB * K * K];
 #pragma unroll
   for (int e = 0; e < NB * K * K; ++e) acc[e] = 0.0;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-    double va[K], vb[NB][K];
+    double va[K], vb[NB][K];  // (T float: the preconditioner's result, widened)
 #pragma unroll
     for (int a = 0; a < K; ++a) va[a] = A.v[a][i];
 #pragma unroll
@@ -314,9 +320,9 @@ bcg_check_kernel(int k, int init, const double* __restrict__ partial, int nb, do
 // column, in one pass over the columns left instead of one per pair.
 
 // w_j = z_j (+ sum_a p_a beta[a][j]) to column j of P; sums w_j . w_j (entries 0..) and w_0 . w_j (entries K..)
-template <int K, bool COMBINE>
+template <int K, bool COMBINE, typename T>
 __global__ void __launch_bounds__(256)
-orth_first_kernel(long long n, int k, VecSet P, VecSet Z, const double* __restrict__ beta, OutSet out,
+orth_first_kernel(long long n, int k, VecSet P, VecSetT<T> Z, const double* __restrict__ beta, OutSet out,
                   double* __restrict__ partial) {
   __shared__ double c[K * kMaxRhs];
   if (COMBINE)
@@ -414,9 +420,10 @@ orth_last_kernel(long long n, int j, int normalize, const double* __restrict__ p
 // host side
 // ------------------------------------------------------------------------------------------------
 
-static VecSet vset(const double* base, long long n, int k, const double* zero) {
-  VecSet s;
-  for (int j = 0; j < kMaxRhs; ++j) s.v[j] = j < k ? base + (long long)j * n : zero;
+template <typename T>
+static VecSetT<T> vset(const T* base, long long n, int k, const double* zero) {
+  VecSetT<T> s;
+  for (int j = 0; j < kMaxRhs; ++j) s.v[j] = j < k ? base + (long long)j * n : (const T*)zero;
   return s;
 }
 static OutSet oset(double* base, long long n, int k) {  // nullptr: not written
@@ -477,20 +484,25 @@ static void orth_passes(BlockCG* w, int k, int normalize, const VecSet& p, const
   }
 }
 
+// is M R left in z32, in FP32, instead of Z?
+static bool z_is_f32(const pmt_mg* mg, const BlockCG* w, int k) { return k > 1 && w->vec && mg->prec != 64; }
+
 // P = orth(Z), or orth(Z + P beta) (iterative.py:259-292)
-static int orth_into_P(BlockCG* w, int k, bool initial, hipStream_t s) {
+template <typename T>
+static int orth_into_P(BlockCG* w, int k, bool initial, const T* Z, hipStream_t s) {
   const long long n = w->n;
   const unsigned nb = sum_blocks(n);
-  const VecSet p = vset(w->P, n, k, w->zero), z = vset(w->Z, n, k, w->zero);
+  const VecSet p = vset(w->P, n, k, w->zero);
+  const VecSetT<T> z = vset(Z, n, k, w->zero);
   const OutSet po = oset(w->P, n, k);
   const double* beta = w->sm + Small::BETA;
   const int nz = initial ? 1 : 0;
   with_k(k, [&](auto kk) {
     constexpr int K = decltype(kk)::value;
     if (initial)
-      orth_first_kernel<K, false><<<nb, 256, 0, s>>>(n, k, p, z, beta, po, w->partial);
+      orth_first_kernel<K, false, T><<<nb, 256, 0, s>>>(n, k, p, z, beta, po, w->partial);
     else
-      orth_first_kernel<K, true><<<nb, 256, 0, s>>>(n, k, p, z, beta, po, w->partial);
+      orth_first_kernel<K, true, T><<<nb, 256, 0, s>>>(n, k, p, z, beta, po, w->partial);
     orth_passes<K, 1>(w, k, nz, p, po, s);
     double* half = w->partial + (long long)kSumBlocks * kMaxRhs * kMaxRhs;
     const double* last = k % 2 ? w->partial : half;  // where pass k - 1 left its sums
@@ -502,6 +514,14 @@ static int orth_into_P(BlockCG* w, int k, bool initial, hipStream_t s) {
   return check_launch("orth kernels");
 }
 
+// Z = M R, in reduced precision left in z32: one V-cycle of all columns (the launches of a V-cycle are mostly short: k columns at once cost little
+// more than one, and share the coefficients of the stored levels); column by column without its vectors
+static int precondition_columns(pmt_mg* mg, BlockCG* w, int k, hipStream_t s) {
+  if (k > 1 && w->vec) return mg_precondition_columns(mg, w->R, w->Z, w->z32, s, k);
+  for (int j = 0; j < k; ++j) PMT_TRY(mg_precondition(mg, col(w->R, w->n, j), col(w->Z, w->n, j), s));
+  return PMT_OK;
+}
+
 // iteration part 1: Q = A P, alpha, X += P alpha, R update, convergence test
 static int iter_part1(pmt_mg* mg, BlockCG* w, int k, bool restart_now, hipStream_t s) {
   const long long n = w->n;
@@ -510,14 +530,14 @@ static int iter_part1(pmt_mg* mg, BlockCG* w, int k, bool restart_now, hipStream
                x = vset(w->X, n, k, w->zero);
   const OutSet xo = oset(w->X, n, k), ro = oset(w->R, n, k);
   const double* alpha = w->sm + Small::ALPHA;
-  for (int j = 0; j < k; ++j) PMT_TRY(mg_level_apply(mg, 0, MODE_APPLY, col(w->P, n, j), nullptr, col(w->Q, n, j), s));
+  PMT_TRY(mg_level_apply(mg, 0, MODE_APPLY, w->P, nullptr, w->Q, s, k));
   with_k(k, [&](auto kk) {
     constexpr int K = decltype(kk)::value;
     if constexpr (K < 8) {
-      gram_kernel<K, 2><<<nb, 256, 0, s>>>(n, p, q, r, w->partial);
+      gram_kernel<K, 2, double><<<nb, 256, 0, s>>>(n, p, q, r, w->partial);
     } else {  // 128 sums per thread would not stay in registers
-      gram_kernel<K, 1><<<nb, 256, 0, s>>>(n, p, q, q, w->partial);
-      gram_kernel<K, 1><<<nb, 256, 0, s>>>(n, p, r, r, w->partial + (long long)K * K * nb);
+      gram_kernel<K, 1, double><<<nb, 256, 0, s>>>(n, p, q, q, w->partial);
+      gram_kernel<K, 1, double><<<nb, 256, 0, s>>>(n, p, r, r, w->partial + (long long)K * K * nb);
     }
     bcg_alpha_kernel<K><<<1, 1024, 0, s>>>(w->partial, (int)nb, w->sm);
     if (restart_now)
@@ -527,26 +547,32 @@ static int iter_part1(pmt_mg* mg, BlockCG* w, int k, bool restart_now, hipStream
   });
   PMT_TRY(check_launch("block CG update"));
   if (restart_now) {
-    for (int j = 0; j < k; ++j)
-      PMT_TRY(mg_level_apply(mg, 0, MODE_RESIDUAL, col(w->X, n, j), col(w->B, n, j), col(w->R, n, j), s));
+    PMT_TRY(mg_level_apply(mg, 0, MODE_RESIDUAL, w->X, w->B, w->R, s, k));
     PMT_TRY(launch_norms(w, k, w->R, 0, s));
   }
   return launch_check(w, k, false, s);
 }
 
-// iteration part 2: Z = M R, beta, P = orth(Z + P beta)
-static int iter_part2(pmt_mg* mg, BlockCG* w, int k, hipStream_t s) {
+// beta and P = orth(Z + P beta)
+template <typename T>
+static int next_directions(BlockCG* w, int k, const T* Z, hipStream_t s) {
   const long long n = w->n;
   const unsigned nb = sum_blocks(n);
-  for (int j = 0; j < k; ++j) PMT_TRY(mg_precondition(mg, col(w->R, n, j), col(w->Z, n, j), s));
-  const VecSet q = vset(w->Q, n, k, w->zero), z = vset(w->Z, n, k, w->zero);
+  const VecSet q = vset(w->Q, n, k, w->zero);
+  const VecSetT<T> z = vset(Z, n, k, w->zero);
   with_k(k, [&](auto kk) {
     constexpr int K = decltype(kk)::value;
-    gram_kernel<K, 1><<<nb, 256, 0, s>>>(n, q, z, z, w->partial);
+    gram_kernel<K, 1, T><<<nb, 256, 0, s>>>(n, q, z, z, w->partial);
     bcg_beta_kernel<K><<<1, 1024, 0, s>>>(w->partial, (int)nb, w->sm);
   });
   PMT_TRY(check_launch("block CG beta"));
-  return orth_into_P(w, k, false, s);
+  return orth_into_P<T>(w, k, false, Z, s);
+}
+
+// iteration part 2: Z = M R, beta, P = orth(Z + P beta)
+static int iter_part2(pmt_mg* mg, BlockCG* w, int k, hipStream_t s) {
+  PMT_TRY(precondition_columns(mg, w, k, s));
+  return z_is_f32(mg, w, k) ? next_directions<float>(w, k, w->z32, s) : next_directions<double>(w, k, w->Z, s);
 }
 
 static void drop_graphs(BlockCG* w) {
@@ -558,8 +584,56 @@ static void drop_graphs(BlockCG* w) {
   w->graph_epoch = -1;
 }
 
+// the levels' vectors for a V-cycle of kcap columns, in one allocation: u, t, b, r per level (FP32: and the
+// result of the fine level).  Without the memory for them the columns go one by one.  Four loads on
+// 128x64x64: a V-cycle of 4 columns 0.42 ms (one by one 4 x 0.21 ms).
+template <typename T>
+static void level_columns(pmt_mg* mg, BlockCG* w) {
+  long long total = 0;
+  T* base = nullptr;
+  auto carve = [&] {
+    T* p = base;
+    auto take = [&](T** v, long long n) {
+      if (base) *v = p;
+      p += n * w->kcap;
+      total += n * w->kcap;
+    };
+    for (int l = 0; l < mg->nlev; ++l) {
+      Level& L = mg->L[l];
+      LevelCols<T>& c = L.cols<T>();
+      if (l > 0) take(&c.u, L.ndof);
+      if (l > 0 || sizeof(T) == 4) take(&c.b, L.ndof);
+      if (l < mg->nlev - 1) take(&c.t, L.ndof);
+      if (l < mg->nlev - 1) take(&c.r, L.ndof);
+    }
+    if (sizeof(T) == 4) take((T**)&w->z32, w->n);
+  };
+  carve();
+  if (hipMalloc(&w->vec, (size_t)total * sizeof(T)) != hipSuccess) {
+    (void)hipGetLastError();
+    w->vec = nullptr;
+    return;
+  }
+  base = (T*)w->vec;
+  carve();
+}
+
+static void ensure_columns(pmt_mg* mg, BlockCG* w) {
+  const int prec = mg->prec == 64 ? 64 : 32;
+  if (w->vec_prec == prec) return;
+  if (w->vec) (void)hipFree(w->vec);
+  w->vec = nullptr;
+  w->vec_prec = prec;
+  drop_graphs(w);
+  if (prec == 64)
+    level_columns<double>(mg, w);
+  else
+    level_columns<float>(mg, w);
+}
+
 static void free_workspace(BlockCG* w) {
   drop_graphs(w);
+  if (w->vec) (void)hipFree(w->vec);
   if (w->mem) (void)hipFree(w->mem);
   if (w->host) (void)hipHostFree(w->host);
   if (w->ev_in) (void)hipEventDestroy(w->ev_in);
@@ -671,6 +745,7 @@ int pmt_block_pcg_solve(pmt_mg* mg, int k, const double* B, double* X, int x0_is
   hipStream_t caller = (hipStream_t)stream;
   PMT_TRY(ensure_workspace(mg, k, caller));
   BlockCG* w = mg->bcg;
+  if (k > 1) ensure_columns(mg, w);
   // all work on the handle's stream, after what the caller queued before this call
   hipStream_t s = w->cs;
   PMT_HIP(hipEventRecord(w->ev_in, caller));
@@ -684,8 +759,7 @@ int pmt_block_pcg_solve(pmt_mg* mg, int k, const double* B, double* X, int x0_is
     PMT_HIP(hipMemcpyAsync(w->R, B, bytes, hipMemcpyDeviceToDevice, s));
   } else {
     PMT_HIP(hipMemcpyAsync(w->X, X, bytes, hipMemcpyDeviceToDevice, s));
-    for (int j = 0; j < k; ++j)
-      PMT_TRY(mg_level_apply(mg, 0, MODE_RESIDUAL, col(w->X, n, j), col(w->B, n, j), col(w->R, n, j), s));
+    PMT_TRY(mg_level_apply(mg, 0, MODE_RESIDUAL, w->X, w->B, w->R, s, k));
   }
   // numbers of this solve's convergence tests: past any that an earlier, failed solve may still publish
   w->seq += 2.0;
@@ -712,8 +786,11 @@ int pmt_block_pcg_solve(pmt_mg* mg, int k, const double* B, double* X, int x0_is
   int it = 0;
   if (!done) {
     // P = orth(Z, normalize=True), Z = M R
-    for (int j = 0; j < k; ++j) PMT_TRY(mg_precondition(mg, col(w->R, n, j), col(w->Z, n, j), s));
-    PMT_TRY(orth_into_P(w, k, true, s));
+    PMT_TRY(precondition_columns(mg, w, k, s));
+    if (z_is_f32(mg, w, k))
+      PMT_TRY(orth_into_P<float>(w, k, true, w->z32, s));
+    else
+      PMT_TRY(orth_into_P<double>(w, k, true, w->Z, s));
     const bool graphs = use_graph != 0;
     if (graphs && (w->graph_k != k || w->graph_epoch != tuning_epoch())) {
       drop_graphs(w);

@@ -677,39 +677,61 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
 // y = A x, one 64-lane wave per row, FP64 sums; IO double, or float (the FP64 coarsest inverse applied to an FP32
 // right-hand side: the widening, the product and the rounding in one).  Each lane has 8 entries of its row in
 // flight.  1911 unknowns: 7.1 us (12.3 us with the loads left to the loop), 847: 3.7 (6.6).
-template <typename T, typename IO>
-__global__ void __launch_bounds__(256) gemv_kernel(long long n, const T* __restrict__ A, const IO* __restrict__ x,
-                                                    IO* __restrict__ y) {
+// Up to NC of the `cols` columns x, y per block share a row's entries.
+template <typename T, typename IO, int NC>
+__global__ void __launch_bounds__(256) gemv_kernel(long long n, int cols, const T* __restrict__ A,
+                                                   const IO* __restrict__ x, IO* __restrict__ y) {
   const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= n) return;
+  const int col0 = (int)blockIdx.y * NC;
   const T* a = A + row * n;
-  T s = 0;
+  const IO* xc[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) xc[k] = x + n * min(col0 + k, cols - 1);
+  T s[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) s[k] = 0;
   long long c = lane;
   for (; c + 7 * 64 < n; c += 8 * 64) {
     T v[8];
-    IO w[8];
+    IO w[NC][8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       v[u] = a[c + 64 * u];
-      w[u] = x[c + 64 * u];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) w[k][u] = xc[k][c + 64 * u];
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) s = fma(v[u], (T)w[u], s);
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s[k] = fma(v[u], (T)w[k][u], s[k]);
   }
   T v[7];
-  IO w[7];
+  IO w[NC][7];
 #pragma unroll
   for (int u = 0; u < 7; ++u) {
     const bool in = c + 64 * u < n;
     v[u] = in ? a[c + 64 * u] : (T)0;
-    w[u] = in ? x[c + 64 * u] : (IO)0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) w[k][u] = in ? xc[k][c + 64 * u] : (IO)0;
   }
 #pragma unroll
-  for (int u = 0; u < 7; ++u)
-    if (c + 64 * u < n) s = fma(v[u], (T)w[u], s);
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) y[row] = (IO)s;
+  for (int k = 0; k < NC; ++k) {
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+      if (c + 64 * u < n) s[k] = fma(v[u], (T)w[k][u], s[k]);
+    for (int off = 32; off > 0; off >>= 1) s[k] += __shfl_down(s[k], off, 64);
+    if (lane == 0 && col0 + k < cols) y[n * (col0 + k) + row] = (IO)s[k];
+  }
+}
+
+template <typename T, typename IO>
+static void launch_gemv_t(long long n, const T* A, const IO* x, IO* y, int cols, hipStream_t s) {
+  if (cols == 1)
+    gemv_kernel<T, IO, 1><<<blocks_for(n, 4), 256, 0, s>>>(n, cols, A, x, y);
+  else
+    gemv_kernel<T, IO, 4><<<dim3(blocks_for(n, 4), (cols + 3) / 4), 256, 0, s>>>(n, cols, A, x, y);
 }
 
 // y = (float) x
@@ -826,15 +848,15 @@ int gj_invert(long long n, double* A, double* ws, hipStream_t s) {
 }
 
 template <typename T>
-int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s) {
-  gemv_kernel<T, T><<<blocks_for(n, 4), 256, 0, s>>>(n, A, x, y);
+int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s, int cols) {
+  launch_gemv_t<T, T>(n, A, x, y, cols, s);
   return check_launch("gemv_kernel");
 }
-template int launch_gemv<double>(long long, const double*, const double*, double*, hipStream_t);
-template int launch_gemv<float>(long long, const float*, const float*, float*, hipStream_t);
+template int launch_gemv<double>(long long, const double*, const double*, double*, hipStream_t, int);
+template int launch_gemv<float>(long long, const float*, const float*, float*, hipStream_t, int);
 
-int launch_gemv_f32io(long long n, const double* A, const float* x, float* y, hipStream_t s) {
-  gemv_kernel<double, float><<<blocks_for(n, 4), 256, 0, s>>>(n, A, x, y);
+int launch_gemv_f32io(long long n, const double* A, const float* x, float* y, hipStream_t s, int cols) {
+  launch_gemv_t<double, float>(n, A, x, y, cols, s);
   return check_launch("gemv_kernel<double, float>");
 }
 
@@ -844,16 +866,17 @@ __global__ void to_float_first_kernel(long long n, const double* __restrict__ x,
                                       const float* __restrict__ dinv, float w, float* __restrict__ u1) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
-    const float v = (float)x[i];
-    y[i] = v;
-    u1[i] = w * dinv[i] * v;
+    const long long c = blockIdx.y * n + i;
+    const float v = (float)x[c];
+    y[c] = v;
+    u1[c] = w * dinv[i] * v;
   }
 }
 
 int launch_to_float_first(long long n, const double* x, float* y, const float* dinv, float w, float* u1,
-                          hipStream_t s) {
+                          hipStream_t s, int cols) {
   if (n <= 0) return PMT_OK;
-  to_float_first_kernel<<<blocks_for(n, 256), 256, 0, s>>>(n, x, y, dinv, w, u1);
+  to_float_first_kernel<<<dim3(blocks_for(n, 256), cols), 256, 0, s>>>(n, x, y, dinv, w, u1);
   return check_launch("to_float_first_kernel");
 }
 

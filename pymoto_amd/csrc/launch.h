@@ -21,10 +21,11 @@ int launch_coarse_correct(long long n, int m, const double* W, const double* AW,
 enum { MODE_APPLY = 0, MODE_RESIDUAL = 1, MODE_JACOBI = 2, MODE_CHEB = 3, MODE_APPLY_DOTS = 4 };
 
 // operator.hip (level kernels exist for T = double and T = float)
+// cols (here and below): vectors u, b, y, up (rf, rc, ...) of `cols` columns, a column the level's dofs
 template <typename T>
 int launch_fine(int mode, const GridDims& g, const double* K0, int k0_pattern, const T* xe, const uint8_t* bcm,
                 double bcdiag, const T* u, const T* b, const T* dinv, double omega, T* y, hipStream_t s,
-                const T* up = nullptr, double beta = 0.0);
+                const T* up = nullptr, double beta = 0.0, int cols = 1);
 int k0_matches_pattern(int dim, const double* K0_host);
 // refl.hip: hex8 operator in the mid-plane reflection basis (K0ext = pmt_k0_extend layout)
 constexpr int kK0ReflOffset64 = 576;  // 72 FP64 block entries after K0
@@ -45,13 +46,13 @@ int launch_coarse1_tstencil(const GridDims& g, const int* tnode, int nt, long lo
 template <typename T>
 int launch_coarse1(int mode, const GridDims& g, int pattern, const double* G0ext, const T* Xh, const int* tnode, int nt,
                    long long cap, const double* TS, const T* u, const T* b, const T* dinv, double omega, T* y,
-                   hipStream_t s, const T* up = nullptr, double beta = 0.0);
+                   hipStream_t s, const T* up = nullptr, double beta = 0.0, int cols = 1);
 template <typename T>
 int launch_fine_refl(int mode, const GridDims& g, int planes /* 0 = from the occupancy */, int rows,
                      int pattern /* K0 has the box class pattern: skip its structural zeros */, const double* K0ext,
                      const T* xe,
                      const uint8_t* bcm, double bcdiag, const T* u, const T* b, const T* dinv, double omega, T* y,
-                     hipStream_t s, const T* up, double beta);
+                     hipStream_t s, const T* up, double beta, int cols = 1);
 // q = A p on the fine grid with out[0] = p.q and out[1] = p.r (deterministic two-stage sums; ws holds
 // 2 * ws_parts doubles).  Returns PMT_ERR_STATE (nothing launched) when the reflection kernel is not the
 // fine operator or the launch needs more partial sums than ws holds; the caller then runs K.u and
@@ -89,15 +90,15 @@ template <typename T>
 int launch_stencil_compress(const GridDims& g, const double* S, T* H, hipStream_t s);
 template <typename T>
 int launch_stencil_half(int mode, const GridDims& g, const T* H, const T* u, const T* b, const T* dinv, double omega,
-                        T* y, hipStream_t s, const T* up = nullptr, double beta = 0.0);
+                        T* y, hipStream_t s, const T* up = nullptr, double beta = 0.0, int cols = 1);
 template <typename T>
-int launch_jacobi0(long long n, const T* dinv, const T* b, double omega, T* u, hipStream_t s);
+int launch_jacobi0(long long n, const T* dinv, const T* b, double omega, T* u, hipStream_t s, int cols = 1);
 template <typename T>
 // u0 (optional): also u0 = w0 D^-1 rc (dinv of the coarse level), its first smoothing sweep from zero
 int launch_restrict(const GridDims& gf, const GridDims& gc, const T* rf, T* rc, hipStream_t s, const T* dinv = nullptr,
-                    double w0 = 0.0, T* u0 = nullptr);
+                    double w0 = 0.0, T* u0 = nullptr, int cols = 1);
 template <typename T>
-int launch_prolong(const GridDims& gf, const GridDims& gc, const T* uc, T* uf, hipStream_t s);
+int launch_prolong(const GridDims& gf, const GridDims& gc, const T* uc, T* uf, hipStream_t s, int cols = 1);
 
 // mfma.hip (hex8 only; BF16 operands, FP32 accumulation and vectors)
 int launch_fine_mfma(int mode, const GridDims& g, const double* K0, const float* xe, const uint8_t* bcm,
@@ -170,10 +171,10 @@ int launch_dense_from_stencil(const GridDims& g, const double* S, double* A, hip
 inline long long gj_work_size(long long n) { return 2 * 64 * 64 + 4 * 64 * n; }
 int gj_invert(long long n, double* A, double* ws, hipStream_t s);
 template <typename T>
-int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s);
-int launch_gemv_f32io(long long n, const double* A, const float* x, float* y, hipStream_t s);
+int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s, int cols = 1);
+int launch_gemv_f32io(long long n, const double* A, const float* x, float* y, hipStream_t s, int cols = 1);
 int launch_to_float_first(long long n, const double* x, float* y, const float* dinv, float w, float* u1,
-                          hipStream_t s);
+                          hipStream_t s, int cols = 1);
 int launch_to_float(long long n, const double* x, float* y, hipStream_t s);
 
 }  // namespace pmt

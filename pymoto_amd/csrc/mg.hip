@@ -83,32 +83,37 @@ const float* fine_x<float>(pmt_mg* mg) {
 // convert in and out: the coarsest solve stays FP64 (an FP32 copy of the inverse of this badly
 // conditioned operator loses the smooth components the coarse correction exists for).
 template <typename T>
-static int coarse_solve(pmt_mg* mg, const T* b, T* out, hipStream_t s);
+static int coarse_solve(pmt_mg* mg, const T* b, T* out, hipStream_t s, int cols);
 template <>
-int coarse_solve<double>(pmt_mg* mg, const double* b, double* out, hipStream_t s) {
+int coarse_solve<double>(pmt_mg* mg, const double* b, double* out, hipStream_t s, int cols) {
   PMT_TRY(mg_join(mg, s));
-  return launch_gemv<double>(mg->nc, mg->Ainv, b, out, s);
+  return launch_gemv<double>(mg->nc, mg->Ainv, b, out, s, cols);
 }
 template <>
-int coarse_solve<float>(pmt_mg* mg, const float* b, float* out, hipStream_t s) {
+int coarse_solve<float>(pmt_mg* mg, const float* b, float* out, hipStream_t s, int cols) {
   PMT_TRY(mg_join(mg, s));
-  return launch_gemv_f32io(mg->nc, mg->Ainv, b, out, s);  // FP64 inverse and sums, FP32 in and out
+  return launch_gemv_f32io(mg->nc, mg->Ainv, b, out, s, cols);  // FP64 inverse and sums, FP32 in and out
 }
 
 // level operator in `mode`; Jacobi / Chebyshev sweeps use `omega` (and `up`, `beta`)
 template <typename T>
 static int level_apply(pmt_mg* mg, int l, int mode, const T* u, const T* b, T* y, hipStream_t s, double omega,
-                       const T* up = nullptr, double beta = 0.0) {
+                       const T* up = nullptr, double beta = 0.0, int cols = 1) {
   Level& L = mg->L[l];
   LevelBuf<T>& B = L.buf<T>();
   if constexpr (std::is_same<T, float>::value) {
-    if (l == 0 && mg->prec == 16 && (mode == MODE_JACOBI || mode == MODE_CHEB))
-      return launch_fine_mfma(mode, L.g, mg->K0, fine_x<T>(mg), mg->bcm, mg->bcdiag, u, b, B.dinv, omega, y, s, up,
-                              beta);
+    if (l == 0 && mg->prec == 16 && (mode == MODE_JACOBI || mode == MODE_CHEB)) {
+      for (int c = 0; c < cols; ++c) {
+        const long long o = c * L.ndof;
+        PMT_TRY(launch_fine_mfma(mode, L.g, mg->K0, fine_x<T>(mg), mg->bcm, mg->bcdiag, u + o, b + o, B.dinv, omega,
+                                 y + o, s, up ? up + o : up, beta));
+      }
+      return PMT_OK;
+    }
   }
   if (l == 0)
     return launch_fine<T>(mode, L.g, mg->K0, mg->k0pat, fine_x<T>(mg), mg->bcm, mg->bcdiag, u, b, B.dinv, omega, y,
-                          s, up, beta);
+                          s, up, beta, cols);
   if (l == mg->nlev - 1) {  // coarsest: only its full FP64 stencil exists (it is solved directly)
     if constexpr (std::is_same<T, double>::value)
       if (mode != MODE_CHEB) return launch_stencil<double>(mode, L.g, L.d.S, u, b, B.dinv, omega, y, s);
@@ -116,13 +121,13 @@ static int level_apply(pmt_mg* mg, int l, int mode, const T* u, const T* b, T* y
   }
   if (l == 1 && mg->l1free)
     return launch_coarse1<T>(mode, L.g, mg->g0pat, mg->G0ext, B.Xh, L.tnode, mg->host_counts[0],
-                             L.t_cap, L.TS, u, b, B.dinv, omega, y, s, up, beta);
-  return launch_stencil_half<T>(mode, L.g, B.H, u, b, B.dinv, omega, y, s, up, beta);
+                             L.t_cap, L.TS, u, b, B.dinv, omega, y, s, up, beta, cols);
+  return launch_stencil_half<T>(mode, L.g, B.H, u, b, B.dinv, omega, y, s, up, beta, cols);
 }
 
 template <typename T>
-static int level_apply(pmt_mg* mg, int l, int mode, const T* u, const T* b, T* y, hipStream_t s) {
-  return level_apply<T>(mg, l, mode, u, b, y, s, mg->L[l].omega);
+static int level_apply(pmt_mg* mg, int l, int mode, const T* u, const T* b, T* y, hipStream_t s, int cols = 1) {
+  return level_apply<T>(mg, l, mode, u, b, y, s, mg->L[l].omega, nullptr, 0.0, cols);
 }
 
 // `steps` smoothing sweeps on level l, from zero or from cur.  Damped Jacobi: u += omega D^-1 (b - A u)
@@ -134,18 +139,18 @@ static int level_apply(pmt_mg* mg, int l, int mode, const T* u, const T* b, T* y
 // The ping-pong buffers cur/oth swap after every sweep; a Chebyshev sweep overwrites u_{k-1} in place.
 template <typename T>
 static int smooth(pmt_mg* mg, int l, const T* b, T*& cur, T*& oth, bool from_zero, hipStream_t s,
-                  bool first_done = false) {
+                  bool first_done = false, int cols = 1) {
   Level& L = mg->L[l];
   LevelBuf<T>& B = L.buf<T>();
   if (mg->smoother == 0) {
     int it0 = 0;
     if (from_zero) {
       // first_done: cur already holds omega D^-1 b (written by the CG update)
-      if (!first_done) PMT_TRY(launch_jacobi0<T>(L.ndof, B.dinv, b, L.omega, cur, s));
+      if (!first_done) PMT_TRY(launch_jacobi0<T>(L.ndof, B.dinv, b, L.omega, cur, s, cols));
       it0 = 1;
     }
     for (int it = it0; it < L.steps; ++it) {
-      PMT_TRY(level_apply<T>(mg, l, MODE_JACOBI, cur, b, oth, s, L.omega));
+      PMT_TRY(level_apply<T>(mg, l, MODE_JACOBI, cur, b, oth, s, L.omega, nullptr, 0.0, cols));
       T* tmp = cur;
       cur = oth;
       oth = tmp;
@@ -157,9 +162,9 @@ static int smooth(pmt_mg* mg, int l, const T* b, T*& cur, T*& oth, bool from_zer
   double rho_prev = 1.0 / sigma;
   if (from_zero) {
     // first_done: cur already holds D^-1 b / theta (written by the CG update)
-    if (!first_done) PMT_TRY(launch_jacobi0<T>(L.ndof, B.dinv, b, 1.0 / theta, cur, s));
+    if (!first_done) PMT_TRY(launch_jacobi0<T>(L.ndof, B.dinv, b, 1.0 / theta, cur, s, cols));
   } else {
-    PMT_TRY(level_apply<T>(mg, l, MODE_JACOBI, cur, b, oth, s, 1.0 / theta));
+    PMT_TRY(level_apply<T>(mg, l, MODE_JACOBI, cur, b, oth, s, 1.0 / theta, nullptr, 0.0, cols));
     T* tmp = cur;
     cur = oth;
     oth = tmp;
@@ -167,7 +172,7 @@ static int smooth(pmt_mg* mg, int l, const T* b, T*& cur, T*& oth, bool from_zer
   for (int it = 1; it < L.steps; ++it) {
     const double rho = 1.0 / (2.0 * sigma - rho_prev);
     const T* up = (from_zero && it == 1) ? nullptr : oth;  // u_{k-1} (zero before the first sweep)
-    PMT_TRY(level_apply<T>(mg, l, MODE_CHEB, cur, b, oth, s, 2.0 * rho / delta, up, rho * rho_prev));
+    PMT_TRY(level_apply<T>(mg, l, MODE_CHEB, cur, b, oth, s, 2.0 * rho / delta, up, rho * rho_prev, cols));
     rho_prev = rho;
     T* tmp = cur;
     cur = oth;
@@ -206,53 +211,68 @@ static Sweeps2 sweep_coefficients(const pmt_mg* mg, int l) {
   return sw;
 }
 
-// out = V-cycle(b) on level l (GeometricMultigrid.solve with x0 = None, iterative.py:222-256)
+// the vectors of level l for a V-cycle of `cols` columns
 template <typename T>
-static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool first_done = false) {
-  if (l == mg->nlev - 1) return coarse_solve<T>(mg, b, out, s);
+static LevelCols<T> level_vectors(pmt_mg* mg, int l, int cols) {
+  if (cols > 1) return mg->L[l].cols<T>();
+  LevelBuf<T>& B = mg->L[l].buf<T>();
+  LevelCols<T> v;
+  v.u = B.u;
+  v.t = B.t;
+  v.b = B.b;
+  v.r = B.r;
+  return v;
+}
+
+// out = V-cycle(b) on level l (GeometricMultigrid.solve with x0 = None, iterative.py:222-256), for `cols` columns
+// of the level's dofs at once
+template <typename T>
+static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool first_done = false, int cols = 1) {
+  if (l == mg->nlev - 1) return coarse_solve<T>(mg, b, out, s, cols);
   Level& L = mg->L[l];
   Level& C = mg->L[l + 1];
-  LevelBuf<T>& B = L.buf<T>();
-  LevelBuf<T>& CB = C.buf<T>();
+  const LevelCols<T> B = level_vectors<T>(mg, l, cols), CB = level_vectors<T>(mg, l + 1, cols);
   if (v2_ok(mg, L.steps)) {  // Q4: all sweeps of a visit in one launch
     const Sweeps2 sw = sweep_coefficients(mg, l);
-    PMT_TRY(launch_v2_down<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.b, s));
-    PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s));
-    return launch_v2_up<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.u, out, s);
+    PMT_TRY(launch_v2_down<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.b, s, cols));
+    PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s, false, cols));
+    return launch_v2_up<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.u, out, s, cols);
   }
   // 2*steps-1 out-of-place sweeps follow the first one: start in the buffer that ends in `out`
   T* cur = B.t;
   T* oth = out;
-  PMT_TRY(smooth<T>(mg, l, b, cur, oth, true, s, first_done));
-  PMT_TRY(level_apply<T>(mg, l, MODE_RESIDUAL, cur, b, B.r, s));
+  PMT_TRY(smooth<T>(mg, l, b, cur, oth, true, s, first_done, cols));
+  PMT_TRY(level_apply<T>(mg, l, MODE_RESIDUAL, cur, b, B.r, s, cols));
   // a smoothed coarse level starts from zero: the restriction also writes its first sweep into the
   // buffer that sweep would write (CB.t), with the factor the smoother would use
   const bool fuse = l + 1 < mg->nlev - 1;
   const double w0 = first_sweep_factor(mg, l + 1);
-  PMT_TRY(launch_restrict<T>(L.g, C.g, B.r, CB.b, s, fuse ? CB.dinv : nullptr, w0, fuse ? CB.t : nullptr));
-  PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s, fuse));
-  PMT_TRY(launch_prolong<T>(L.g, C.g, CB.u, cur, s));
-  PMT_TRY(smooth<T>(mg, l, b, cur, oth, false, s));
+  PMT_TRY(launch_restrict<T>(L.g, C.g, B.r, CB.b, s, fuse ? C.buf<T>().dinv : nullptr, w0, fuse ? CB.t : nullptr, cols));
+  PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s, fuse, cols));
+  PMT_TRY(launch_prolong<T>(L.g, C.g, CB.u, cur, s, cols));
+  PMT_TRY(smooth<T>(mg, l, b, cur, oth, false, s, false, cols));
   if (cur != out) return arg_error("vcycle: internal buffer parity error");
   return PMT_OK;
 }
 
 // reduced-precision V-cycles: z32 = M r, from r rounded to FP32 (already in the fine level's FP32 right-hand
 // side when r32_ready: the CG update wrote it)
-static int precondition_f32(pmt_mg* mg, const double* r, bool r32_ready, hipStream_t s, bool first_done = false) {
+static int precondition_f32(pmt_mg* mg, const double* r, float* z32, bool r32_ready, hipStream_t s,
+                            bool first_done = false, int cols = 1) {
   Level& F = mg->L[0];
+  const LevelCols<float> B = level_vectors<float>(mg, 0, cols);
   if (!r32_ready) {
     // the rounding also writes the first fine sweep from zero (the CG update does the same in the loop)
-    PMT_TRY(launch_to_float_first(F.ndof, r, F.f.b, F.f.dinv, (float)first_sweep_factor(mg, 0), F.f.t, s));
+    PMT_TRY(launch_to_float_first(F.ndof, r, B.b, F.f.dinv, (float)first_sweep_factor(mg, 0), B.t, s, cols));
     first_done = true;
   }
-  return vcycle<float>(mg, 0, F.f.b, mg->z32, s, first_done);
+  return vcycle<float>(mg, 0, B.b, z32, s, first_done, cols);
 }
 
 // the preconditioner as CG sees it: FP64 in, FP64 out
 static int precondition(pmt_mg* mg, const double* r, double* z, hipStream_t s) {
   if (mg->prec == 64) return vcycle<double>(mg, 0, r, z, s);
-  PMT_TRY(precondition_f32(mg, r, false, s));
+  PMT_TRY(precondition_f32(mg, r, mg->z32, false, s));
   return launch_to_double(mg->L[0].ndof, mg->z32, z, s);
 }
 
@@ -377,11 +397,16 @@ static double element_lmax(int ne, const double* K0) {
   return lam;
 }
 
-int mg_level_apply(pmt_mg* mg, int l, int mode, const double* u, const double* b, double* y, hipStream_t s) {
-  return level_apply<double>(mg, l, mode, u, b, y, s);
+int mg_level_apply(pmt_mg* mg, int l, int mode, const double* u, const double* b, double* y, hipStream_t s, int cols) {
+  return level_apply<double>(mg, l, mode, u, b, y, s, cols);
 }
 
 int mg_precondition(pmt_mg* mg, const double* r, double* z, hipStream_t s) { return precondition(mg, r, z, s); }
+
+int mg_precondition_columns(pmt_mg* mg, const double* r, double* z, float* z32, hipStream_t s, int cols) {
+  if (mg->prec == 64) return vcycle<double>(mg, 0, r, z, s, false, cols);
+  return precondition_f32(mg, r, z32, false, s, false, cols);
+}
 
 // Every stream that reads the coarsest inverse after an update waits for its inversion once: the handle
 // lists the streams that have waited since the update (a stream ordered after a joined stream is not
@@ -902,7 +927,7 @@ int pmt_pcg_solve(pmt_mg* mg, const double* b, double* x, int x0_is_zero, double
     // z = M r, sc[3] = q.z, p = z + beta p: reads r and q, writes only z, sc[3] and p (no result)
     auto next_direction = [&]() -> int {
       if (mixed) {
-        PMT_TRY(precondition_f32(mg, mg->r, r32_ready, s, r32_ready && first));
+        PMT_TRY(precondition_f32(mg, mg->r, mg->z32, r32_ready, s, r32_ready && first));
         if (mg->cs_m == 0) {
           PMT_TRY(launch_dot_flat(n, mg->q, mg->z32, sc + 3, mg->rwork, s));
           PMT_TRY(launch_cg_p_update(n, sc, mg->z32, mg->p, s, x_pending ? x : nullptr));

@@ -24,6 +24,15 @@ struct LevelBuf {
   T* Xh = nullptr;    // hex8 level 1 without a stencil: transformed child densities [layer][8][element]
 };
 
+// the vectors of a level that a V-cycle of several columns writes (LevelBuf's for one column)
+template <typename T>
+struct LevelCols {
+  T* u = nullptr;
+  T* t = nullptr;
+  T* b = nullptr;
+  T* r = nullptr;
+};
+
 struct Level {
   GridDims g;
   long long ndof = 0;
@@ -48,8 +57,12 @@ struct Level {
   double* C = nullptr;
   LevelBuf<double> d;
   LevelBuf<float> f;
+  LevelCols<double> dcols;  // block CG's columns (its workspace; null without one)
+  LevelCols<float> fcols;
   template <typename T>
   LevelBuf<T>& buf();
+  template <typename T>
+  LevelCols<T>& cols();
 };
 template <>
 inline LevelBuf<double>& Level::buf<double>() {
@@ -58,6 +71,14 @@ inline LevelBuf<double>& Level::buf<double>() {
 template <>
 inline LevelBuf<float>& Level::buf<float>() {
   return f;
+}
+template <>
+inline LevelCols<double>& Level::cols<double>() {
+  return dcols;
+}
+template <>
+inline LevelCols<float>& Level::cols<float>() {
+  return fcols;
 }
 
 }  // namespace pmt
@@ -136,21 +157,26 @@ struct Sweeps2 {
 bool v2_ok(const pmt_mg* mg, int steps);
 // u = the sweeps from zero on level l, bc = R^T (b - A u)
 template <typename T>
-int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s);
+int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s,
+                   int cols);
 // uo = the sweeps from ui + R ec (uo must not be ui)
 template <typename T>
 int launch_v2_up(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, const T* ui, const T* ec, T* uo,
-                 hipStream_t s);
+                 hipStream_t s, int cols);
 
 // frees the block-CG workspace and graphs of a handle (blockcg.hip)
 void block_cg_release(pmt_mg* mg);
 // drops captured block-CG iterations (after an update or a change of precision or launch shapes)
 void block_cg_invalidate(pmt_mg* mg);
 
-// y = A_l u (mode apply), b - A_l u (residual) or a damped-Jacobi sweep on level l, FP64
-int mg_level_apply(pmt_mg* mg, int l, int mode, const double* u, const double* b, double* y, hipStream_t s);
+// y = A_l u (mode apply), b - A_l u (residual) or a damped-Jacobi sweep on level l, FP64, `cols` columns
+int mg_level_apply(pmt_mg* mg, int l, int mode, const double* u, const double* b, double* y, hipStream_t s,
+                   int cols = 1);
 // z = M r: one V-cycle in the handle's precision, FP64 in and out
 int mg_precondition(pmt_mg* mg, const double* r, double* z, hipStream_t s);
+// the same for `cols` columns at once, with the Level::cols vectors of the handle's precision; the result in z
+// (FP64 V-cycles) or in z32 (reduced precision)
+int mg_precondition_columns(pmt_mg* mg, const double* r, double* z, float* z32, hipStream_t s, int cols);
 // device allocation owned (and freed) by the handle
 int mg_alloc(pmt_mg* mg, void** p, long long bytes);
 // make stream s wait for the coarsest inverse of the last update (no-op once joined); callers that

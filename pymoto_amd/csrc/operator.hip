@@ -519,6 +519,11 @@ template <int DIM, int MODE, typename T>
 __global__ void __launch_bounds__(256)
 stencil_half_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ u, const T* __restrict__ b,
                     const T* __restrict__ dinv, T omega, T* y, const T* up, T beta) {
+  const long long column = DIM * (long long)blockIdx.y * g.nnodes;
+  u += column;
+  y += column;
+  b = b ? b + column : b;
+  up = up ? up + column : up;
   const long long n = (long long)xcd_block() * blockDim.x + threadIdx.x;
   if (n >= g.nnodes) return;
   const int i = (int)(n % g.nx);
@@ -600,38 +605,47 @@ stencil_half_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ u
 
 // Small grids of hex8 nodes: nine wavefronts per 64 nodes, wave r holding the row r of three neighbours,
 // so the 36 loads of a row are all in flight at once and the nine rows in parallel instead of one after the
-// other; the rows' sums meet in LDS and three waves (one per component) finish the nodes.  A sweep costs the
+// other; the rows' sums meet in LDS and one wave per component finishes the nodes.  A sweep costs the
 // latency of one row (stencil_half_kernel that of nine): 225 to 9,537 nodes 4.6 us in FP32 (6.5 to 7.1), 4,225
 // nodes 4.9 us in FP64 (11.0), 70,785 nodes 12.4 us in FP32 (12.9).  Above that the coefficients stream from
 // memory and both run at its rate.
+// NC columns share the coefficients in registers: four columns of 70,785 nodes in FP32 18.9 us, one 11.4.
 constexpr long long kSplitNodes = 100000;
 
-template <int MODE, typename T>
+template <int MODE, int NC, typename T>
 __global__ void __launch_bounds__(576)
-stencil_split_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ u, const T* __restrict__ b,
+stencil_split_kernel(GridDims g, int cols, const T* __restrict__ H, const T* __restrict__ u, const T* __restrict__ b,
                      const T* __restrict__ dinv, T omega, T* y, const T* up, T beta) {
   constexpr int TS = (int)sizeof(T);
   constexpr int C = Half<3>::C;
-  __shared__ T sum[9][3][64];
+  constexpr int FIN = (3 * NC + 8) / 9;  // (column, component) pairs a wave finishes
+  __shared__ T sum[NC][9][3][64];
   const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int nn = (int)g.nnodes;
   const int n = (int)xcd_block() * 64 + lane;
   const int i = n % g.nx, t = n / g.nx, j = t % g.ny, k = t / g.ny;
   const int dy = r % 3 - 1, dz = r / 3 - 1;
   const bool live = n < nn;
-  const __amdgpu_buffer_rsrc_t ru = plane_rsrc(u, 0, 3LL * nn, true);
-  // operands of the update, one wave per component
-  const int oq = live ? (3 * n + (r < 3 ? r : 0)) * TS : kOOB;
-  T uq = 0, bq = 0, dq = 0, pq = 0;
-  if (r < 3) {
-    if (MODE == MODE_JACOBI || MODE == MODE_CHEB) {
-      uq = bload(ru, oq, T());
-      dq = bload(plane_rsrc(dinv, 0, 3LL * nn, true), oq, T());
+  const int col0 = (int)blockIdx.y * NC;
+  auto column = [&](const T* v, int c, bool valid) {  // columns past the last one are empty: they read 0
+    return plane_rsrc(v, 3LL * nn * (col0 + c), 3LL * nn, valid && col0 + c < cols);
+  };
+  // operands of the updates
+  T uq[FIN], bq[FIN], dq[FIN], pq[FIN];
+#pragma unroll
+  for (int f = 0; f < FIN; ++f) {
+    const int pr = r + 9 * f, c = pr / 3, oq = live ? (3 * n + pr % 3) * TS : kOOB;
+    uq[f] = bq[f] = dq[f] = pq[f] = 0;
+    if (pr < 3 * NC) {
+      if (MODE == MODE_JACOBI || MODE == MODE_CHEB) {
+        uq[f] = bload(column(u, c, true), oq, T());
+        dq[f] = bload(plane_rsrc(dinv, 0, 3LL * nn, true), oq, T());
+      }
+      if (MODE != MODE_APPLY) bq[f] = bload(column(b, c, true), oq, T());
+      if (MODE == MODE_CHEB) pq[f] = bload(column(up, c, up != nullptr), oq, T());
     }
-    if (MODE != MODE_APPLY) bq = bload(plane_rsrc(b, 0, 3LL * nn, true), oq, T());
-    if (MODE == MODE_CHEB) pq = bload(plane_rsrc(up, 0, 3LL * nn, up != nullptr), oq, T());
   }
-  T v[3][12];
+  T h[3][9], v[NC][3][3];
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     const int o = r * 3 + q;
@@ -643,36 +657,44 @@ stencil_split_kernel(GridDims g, const T* __restrict__ H, const T* __restrict__ 
     const int oh = in ? (fwd ? n : m) * TS : kOOB, ou = in ? 3 * m * TS : kOOB;
     const int c0 = (fwd ? o - C : C - o) * 9, sd = fwd ? 3 : 1, sd2 = fwd ? 1 : 3;
 #pragma unroll
-    for (int d2 = 0; d2 < 3; ++d2) v[q][d2] = bload(ru, ou + d2 * TS, T());
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int d2 = 0; d2 < 3; ++d2) v[c][q][d2] = bload(column(u, c, true), ou + d2 * TS, T());
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
       for (int d2 = 0; d2 < 3; ++d2)
-        v[q][3 + d * 3 + d2] = bload(plane_rsrc(H, (long long)(c0 + d * sd + d2 * sd2) * nn, nn, true), oh, T());
+        h[q][d * 3 + d2] = bload(plane_rsrc(H, (long long)(c0 + d * sd + d2 * sd2) * nn, nn, true), oh, T());
   }
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    T acc = 0;
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
+    for (int d = 0; d < 3; ++d) {
+      T acc = 0;
 #pragma unroll
-      for (int d2 = 0; d2 < 3; ++d2) acc = fma(v[q][3 + d * 3 + d2], v[q][d2], acc);
-    sum[r][d][lane] = acc;
-  }
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int d2 = 0; d2 < 3; ++d2) acc = fma(h[q][d * 3 + d2], v[c][q][d2], acc);
+      sum[c][r][d][lane] = acc;
+    }
   __syncthreads();
-  if (r >= 3 || !live) return;
-  T out = 0;
 #pragma unroll
-  for (int w = 0; w < 9; ++w) out += sum[w][r][lane];
-  const long long q = 3LL * n + r;
-  if (MODE == MODE_APPLY)
-    y[q] = out;
-  else if (MODE == MODE_RESIDUAL)
-    y[q] = bq - out;
-  else if (MODE == MODE_JACOBI)
-    y[q] = uq + omega * dq * (bq - out);
-  else
-    y[q] = uq + omega * dq * (bq - out) + beta * (uq - pq);
+  for (int f = 0; f < FIN; ++f) {
+    const int pr = r + 9 * f, c = pr / 3, d = pr % 3;
+    if (pr >= 3 * NC || col0 + c >= cols || !live) return;
+    T out = 0;
+#pragma unroll
+    for (int w = 0; w < 9; ++w) out += sum[c][w][d][lane];
+    const long long q = 3LL * nn * (col0 + c) + 3LL * n + d;
+    if (MODE == MODE_APPLY)
+      y[q] = out;
+    else if (MODE == MODE_RESIDUAL)
+      y[q] = bq[f] - out;
+    else if (MODE == MODE_JACOBI)
+      y[q] = uq[f] + omega * dq[f] * (bq[f] - out);
+    else
+      y[q] = uq[f] + omega * dq[f] * (bq[f] - out) + beta * (uq[f] - pq[f]);
+  }
 }
 
 template <int DIM, typename T>
@@ -688,8 +710,8 @@ __global__ void stencil_diag_kernel(GridDims g, const double* __restrict__ S, T*
 template <typename T>
 __global__ void jacobi0_kernel(long long n, const T* __restrict__ dinv, const T* __restrict__ b,
                                T omega, T* __restrict__ u) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < n) u[q] = omega * dinv[q] * b[q];
+  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y * n + q;
+  if (q < n) u[c] = omega * dinv[q] * b[c];
 }
 
 // rc = R^T rf : coarse node gathers the 3^D fine nodes around its fine image (weights 1, 1/2, 1/4, 1/8), one thread
@@ -702,6 +724,9 @@ __global__ void restrict_kernel(GridDims gf, GridDims gc, const T* __restrict__ 
                                 const T* __restrict__ dinv, T w0, T* __restrict__ u0) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= gc.nnodes * DIM) return;
+  rf += (long long)blockIdx.y * gf.nnodes * DIM;
+  rc += (long long)blockIdx.y * gc.nnodes * DIM;
+  u0 = u0 ? u0 + (long long)blockIdx.y * gc.nnodes * DIM : u0;
   const long long N = q / DIM;
   const int d = (int)(q - N * DIM);
   const int I = (int)(N % gc.nx);
@@ -737,6 +762,8 @@ template <int DIM, typename T>
 __global__ void prolong_kernel(GridDims gf, GridDims gc, const T* __restrict__ uc, T* __restrict__ uf) {
   const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= gf.nnodes) return;
+  uc += (long long)blockIdx.y * gc.nnodes * DIM;
+  uf += (long long)blockIdx.y * gf.nnodes * DIM;
   const int i = (int)(n % gf.nx);
   const long long t = n / gf.nx;
   const int j = (int)(t % gf.ny);
@@ -953,12 +980,17 @@ static void launch_stream_t(int mode, const GridDims& g, const double* K0, const
 template <typename T>
 int launch_fine(int mode, const GridDims& g, const double* K0, int k0_pattern, const T* xe, const uint8_t* bcm,
                 double bcdiag, const T* u, const T* b, const T* dinv, double omega, T* y, hipStream_t s, const T* up,
-                double beta) {
+                double beta, int cols) {
   const T bd = (T)bcdiag, om = (T)omega, be = (T)beta;
   const bool cls = (k0_pattern & PMT_K0_CLASS_PATTERN) != 0;
   if (g.dim == 3 && g_fine_kernel == 2 && (k0_pattern & PMT_K0_REFLECTION)) {
     return launch_fine_refl<T>(mode, g, g_stream_nzc, g_refl_rows, refl_pattern(k0_pattern), K0, xe, bcm, bcdiag, u,
-                               b, dinv, omega, y, s, up, beta);
+                               b, dinv, omega, y, s, up, beta, cols);
+  }
+  for (int c = 1; c < cols; ++c) {  // the other kernels take a column per launch
+    const long long o = c * g.nnodes * g.dim;
+    PMT_TRY(launch_fine<T>(mode, g, K0, k0_pattern, xe, bcm, bcdiag, u + o, b ? b + o : b, dinv, omega, y + o, s,
+                           up ? up + o : up, beta));
   }
   if (g.dim == 3 && g_fine_kernel >= 1) {
     if (cls)
@@ -1019,11 +1051,20 @@ int launch_stencil_compress(const GridDims& g, const double* S, T* H, hipStream_
 
 template <typename T>
 int launch_stencil_half(int mode, const GridDims& g, const T* H, const T* u, const T* b, const T* dinv, double omega,
-                        T* y, hipStream_t s, const T* up, double beta) {
-  dim3 grid(xcd_blocks(g.nnodes, 256));
+                        T* y, hipStream_t s, const T* up, double beta, int cols) {
+  dim3 grid(xcd_blocks(g.nnodes, 256), cols);
   const T om = (T)omega, be = (T)beta;
 #define PMT_HALF(D, M) stencil_half_kernel<D, M, T><<<grid, 256, 0, s>>>(g, H, u, b, dinv, om, y, up, be)
-#define PMT_SPLIT(M) stencil_split_kernel<M, T><<<xcd_blocks(g.nnodes, 64), 576, 0, s>>>(g, H, u, b, dinv, om, y, up, be)
+#define PMT_SPLIT(M)                                                                                              \
+  do {                                                                                                            \
+    const unsigned nb = (unsigned)xcd_blocks(g.nnodes, 64);                                                       \
+    if (cols == 1)                                                                                                \
+      stencil_split_kernel<M, 1, T><<<nb, 576, 0, s>>>(g, cols, H, u, b, dinv, om, y, up, be);                     \
+    else if (cols == 2)                                                                                           \
+      stencil_split_kernel<M, 2, T><<<nb, 576, 0, s>>>(g, cols, H, u, b, dinv, om, y, up, be);                     \
+    else                                                                                                          \
+      stencil_split_kernel<M, 4, T><<<dim3(nb, (cols + 3) / 4), 576, 0, s>>>(g, cols, H, u, b, dinv, om, y, up, be); \
+  } while (0)
   if (g.dim == 3 && g.nnodes <= kSplitNodes) {
     if (mode == MODE_APPLY)
       PMT_SPLIT(MODE_APPLY);
@@ -1093,15 +1134,15 @@ int launch_stencil_dinv(const GridDims& g, const double* S, T* dinv, hipStream_t
 }
 
 template <typename T>
-int launch_jacobi0(long long n, const T* dinv, const T* b, double omega, T* u, hipStream_t s) {
-  jacobi0_kernel<T><<<blocks_for(n, 256), 256, 0, s>>>(n, dinv, b, (T)omega, u);
+int launch_jacobi0(long long n, const T* dinv, const T* b, double omega, T* u, hipStream_t s, int cols) {
+  jacobi0_kernel<T><<<dim3(blocks_for(n, 256), cols), 256, 0, s>>>(n, dinv, b, (T)omega, u);
   return check_launch("jacobi0_kernel");
 }
 
 template <typename T>
 int launch_restrict(const GridDims& gf, const GridDims& gc, const T* rf, T* rc, hipStream_t s, const T* dinv,
-                    double w0, T* u0) {
-  dim3 grid(blocks_for(gc.nnodes * gc.dim, 256));
+                    double w0, T* u0, int cols) {
+  dim3 grid(blocks_for(gc.nnodes * gc.dim, 256), cols);
   if (gf.dim == 3)
     restrict_kernel<3, T><<<grid, 256, 0, s>>>(gf, gc, rf, rc, dinv, (T)w0, u0);
   else
@@ -1110,8 +1151,8 @@ int launch_restrict(const GridDims& gf, const GridDims& gc, const T* rf, T* rc, 
 }
 
 template <typename T>
-int launch_prolong(const GridDims& gf, const GridDims& gc, const T* uc, T* uf, hipStream_t s) {
-  dim3 grid(blocks_for(gf.nnodes, 256));
+int launch_prolong(const GridDims& gf, const GridDims& gc, const T* uc, T* uf, hipStream_t s, int cols) {
+  dim3 grid(blocks_for(gf.nnodes, 256), cols);
   if (gf.dim == 3)
     prolong_kernel<3, T><<<grid, 256, 0, s>>>(gf, gc, uc, uf);
   else
@@ -1119,18 +1160,18 @@ int launch_prolong(const GridDims& gf, const GridDims& gc, const T* uc, T* uf, h
   return check_launch("prolong_kernel");
 }
 
-#define PMT_INSTANTIATE_LEVEL(T)                                                                                   \
+#define PMT_INSTANTIATE_LEVEL(T)                                                                                    \
   template int launch_fine<T>(int, const GridDims&, const double*, int, const T*, const uint8_t*, double, const T*, \
-                              const T*, const T*, double, T*, hipStream_t, const T*, double);                      \
-  template int launch_stencil<T>(int, const GridDims&, const T*, const T*, const T*, const T*, double, T*,         \
-                                 hipStream_t);                                                                     \
-  template int launch_stencil_dinv<T>(const GridDims&, const double*, T*, hipStream_t);                            \
-  template int launch_stencil_compress<T>(const GridDims&, const double*, T*, hipStream_t);                        \
-  template int launch_stencil_half<T>(int, const GridDims&, const T*, const T*, const T*, const T*, double, T*,    \
-                                      hipStream_t, const T*, double);                                              \
-  template int launch_jacobi0<T>(long long, const T*, const T*, double, T*, hipStream_t);                          \
-  template int launch_restrict<T>(const GridDims&, const GridDims&, const T*, T*, hipStream_t, const T*, double, T*); \
-  template int launch_prolong<T>(const GridDims&, const GridDims&, const T*, T*, hipStream_t);
+                              const T*, const T*, double, T*, hipStream_t, const T*, double, int);                  \
+  template int launch_stencil<T>(int, const GridDims&, const T*, const T*, const T*, const T*, double, T*,          \
+                                 hipStream_t);                                                                      \
+  template int launch_stencil_dinv<T>(const GridDims&, const double*, T*, hipStream_t);                             \
+  template int launch_stencil_compress<T>(const GridDims&, const double*, T*, hipStream_t);                         \
+  template int launch_stencil_half<T>(int, const GridDims&, const T*, const T*, const T*, const T*, double, T*,     \
+                                      hipStream_t, const T*, double, int);                                          \
+  template int launch_jacobi0<T>(long long, const T*, const T*, double, T*, hipStream_t, int);                      \
+  template int launch_restrict<T>(const GridDims&, const GridDims&, const T*, T*, hipStream_t, const T*, double, T*, int);\
+  template int launch_prolong<T>(const GridDims&, const GridDims&, const T*, T*, hipStream_t, int);
 PMT_INSTANTIATE_LEVEL(double)
 PMT_INSTANTIATE_LEVEL(float)
 #undef PMT_INSTANTIATE_LEVEL

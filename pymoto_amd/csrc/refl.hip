@@ -322,6 +322,11 @@ fine_refl_kernel(GridDims g, int tiles_x, int ntiles_xy, int nzc, int nwork, con
 
   const int work = (int)xcd_block();
   if (work >= nwork) return;  // whole block leaves together (grid padded for the XCD remap)
+  const long long column = 3 * (long long)blockIdx.y * g.nnodes;
+  u += column;
+  y += column;
+  b = b ? b + column : b;
+  up = up ? up + column : up;
   const int txy = work % ntiles_xy;
   const int tid = threadIdx.x, tx = tid % RX, ty = tid / RX;
   // PAT 2 (isotropic cube): the 8 block numbers, read once and kept in scalar registers
@@ -722,17 +727,17 @@ static int refl_planes(int nxy, int nz, int resident) {
 template <int OP, int RX, int SY, int PAT, typename T>
 static void launch_refl_shape(int mode, const GridDims& g, int planes, const T* tab, const T* xe, const uint8_t* bcm,
                               T bcdiag, const T* u, const T* b, const T* dinv, T omega, T* y, hipStream_t s,
-                              const T* up, T beta, double* partial = nullptr, int* nwork_out = nullptr) {
+                              const T* up, T beta, double* partial = nullptr, int* nwork_out = nullptr, int cols = 1) {
   const int tx = (g.nx + RX - 3) / (RX - 2);
   const int ty = (g.ny + SY - 3) / (SY - 2);
   const int nxy = tx * ty;
 #define PMT_REFL(M)                                                                                             \
   do {                                                                                                          \
     const int nzc = planes > 0 ? (planes < g.nz ? planes : g.nz)                                               \
-                               : refl_planes(nxy, g.nz, refl_resident_blocks<OP, RX, SY, M, PAT, T>());         \
+                               : refl_planes(nxy * cols, g.nz, refl_resident_blocks<OP, RX, SY, M, PAT, T>());         \
     const int nwork = nxy * ((g.nz + nzc - 1) / nzc);                                                          \
     if (nwork_out) *nwork_out = nwork;                                                                          \
-    fine_refl_kernel<OP, RX, SY, M, PAT, T><<<(unsigned)((nwork + 7) & ~7), RX * SY, 0, s>>>(                  \
+    fine_refl_kernel<OP, RX, SY, M, PAT, T><<<dim3((unsigned)((nwork + 7) & ~7), cols), RX * SY, 0, s>>>(                  \
         g, tx, nxy, nzc, nwork, tab, 0, xe, bcm, bcdiag, u, b, dinv, omega, y, up, beta, partial);               \
   } while (0)
   if (mode == MODE_APPLY_DOTS) {
@@ -776,38 +781,42 @@ int refl_auto_rows(const GridDims& g) {
 template <int OP, int PAT, typename T>
 static void launch_refl_rows(int rows, int mode, const GridDims& g, int planes, const T* tab, const T* xe,
                              const uint8_t* bcm, T bcdiag, const T* u, const T* b, const T* dinv, T omega, T* y,
-                             hipStream_t s, const T* up, T beta, double* partial = nullptr, int* nwork_out = nullptr) {
+                             hipStream_t s, const T* up, T beta, double* partial = nullptr, int* nwork_out = nullptr,
+                             int cols = 1) {
   switch (rows > 0 ? rows : refl_auto_rows(g)) {
     case 12:
       launch_refl_shape<OP, 32, 12, PAT, T>(mode, g, planes, tab, xe, bcm, bcdiag, u, b, dinv, omega, y, s, up, beta,
-                                            partial, nwork_out);
+                                            partial, nwork_out, cols);
       break;
     case 24:
       launch_refl_shape<OP, 16, 24, PAT, T>(mode, g, planes, tab, xe, bcm, bcdiag, u, b, dinv, omega, y, s, up, beta,
-                                            partial, nwork_out);
+                                            partial, nwork_out, cols);
       break;
     case 32:
       launch_refl_shape<OP, 16, 32, PAT, T>(mode, g, planes, tab, xe, bcm, bcdiag, u, b, dinv, omega, y, s, up, beta,
-                                            partial, nwork_out);
+                                            partial, nwork_out, cols);
       break;
     default:
       launch_refl_shape<OP, 16, 16, PAT, T>(mode, g, planes, tab, xe, bcm, bcdiag, u, b, dinv, omega, y, s, up, beta,
-                                            partial, nwork_out);
+                                            partial, nwork_out, cols);
   }
 }
 
 template <typename T>
 int launch_fine_refl(int mode, const GridDims& g, int planes, int rows, int pattern, const double* K0ext, const T* xe,
                      const uint8_t* bcm, double bcdiag, const T* u, const T* b, const T* dinv, double omega, T* y,
-                     hipStream_t s, const T* up, double beta) {
+                     hipStream_t s, const T* up, double beta, int cols) {
   const T* tab = sizeof(T) == 8 ? (const T*)(K0ext + kK0ReflOffset64) : (const T*)(K0ext + kK0ReflOffset32);
   const T bd = (T)bcdiag, om = (T)omega, be = (T)beta;
   if (pattern == 2)
-    launch_refl_rows<0, 2, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be);
+    launch_refl_rows<0, 2, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be, nullptr,
+                              nullptr, cols);
   else if (pattern == 1)
-    launch_refl_rows<0, 1, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be);
+    launch_refl_rows<0, 1, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be, nullptr,
+                              nullptr, cols);
   else
-    launch_refl_rows<0, 0, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be);
+    launch_refl_rows<0, 0, T>(rows, mode, g, planes, tab, xe, bcm, bd, u, b, dinv, om, y, s, up, be, nullptr,
+                              nullptr, cols);
   return check_launch("fine_refl_kernel");
 }
 
@@ -1067,6 +1076,8 @@ coarse1_tapply_kernel(GridDims g, const int* __restrict__ tnode, int nt, long lo
   const int t = (int)blockIdx.x * 64 + lane, tc = min(t, nt - 1);  // lanes past the end repeat the last node
   const int n = tnode[tc];
   const int I = n % g.nx, tt = n / g.nx, J = tt % g.ny, K = tt / g.ny;
+  u += 3 * (long long)blockIdx.y * g.nnodes;
+  y += 3 * (long long)blockIdx.y * g.nnodes;
   const long long q = 3LL * n + (r < 3 ? r : 0);
   const double y0 = r < 3 ? (double)y[q] : 0.0;
   const double d0 = r < 3 && MODE == MODE_JACOBI ? (double)dinv[q] : 0.0;
@@ -1120,18 +1131,21 @@ int launch_coarse1_tstencil(const GridDims& g, const int* tnode, int nt, long lo
 template <typename T>
 int launch_coarse1(int mode, const GridDims& g, int pattern, const double* G0ext, const T* Xh, const int* tnode, int nt,
                    long long cap, const double* TS, const T* u, const T* b, const T* dinv, double omega, T* y,
-                   hipStream_t s, const T* up, double beta) {
+                   hipStream_t s, const T* up, double beta, int cols) {
   const T* tab = sizeof(T) == 8 ? (const T*)G0ext : (const T*)(G0ext + 576);
   const T om = (T)omega, be = (T)beta;
   if (pattern == 2)
-    launch_refl_shape<1, 16, 16, 2, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be);
+    launch_refl_shape<1, 16, 16, 2, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be, nullptr,
+                                       nullptr, cols);
   else if (pattern == 1)
-    launch_refl_shape<1, 16, 16, 1, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be);
+    launch_refl_shape<1, 16, 16, 1, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be, nullptr,
+                                       nullptr, cols);
   else
-    launch_refl_shape<1, 16, 16, 0, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be);
+    launch_refl_shape<1, 16, 16, 0, T>(mode, g, 0, tab, Xh, nullptr, (T)0, u, b, dinv, om, y, s, up, be, nullptr,
+                                       nullptr, cols);
   PMT_TRY(check_launch("fine_refl_kernel<coarse level 1>"));
   if (nt <= 0) return PMT_OK;
-  const unsigned blocks = (unsigned)blocks_for(nt, 64);
+  const dim3 blocks((unsigned)blocks_for(nt, 64), cols);
   if (mode == MODE_APPLY)
     coarse1_tapply_kernel<MODE_APPLY, T><<<blocks, 576, 0, s>>>(g, tnode, nt, cap, TS, u, dinv, omega, y);
   else if (mode == MODE_RESIDUAL)
@@ -1183,16 +1197,16 @@ int launch_coarse1_xhat(const GridDims& gf, const GridDims& gc, const double* xe
 
 template int launch_fine_refl<double>(int, const GridDims&, int, int, int, const double*, const double*, const uint8_t*,
                                       double, const double*, const double*, const double*, double, double*,
-                                      hipStream_t, const double*, double);
+                                      hipStream_t, const double*, double, int);
 template int launch_fine_refl<float>(int, const GridDims&, int, int, int, const double*, const float*, const uint8_t*,
                                      double, const float*, const float*, const float*, double, float*, hipStream_t,
-                                     const float*, double);
+                                     const float*, double, int);
 template int launch_coarse1<double>(int, const GridDims&, int, const double*, const double*, const int*, int,
                                     long long, const double*, const double*, const double*, const double*, double,
-                                    double*, hipStream_t, const double*, double);
+                                    double*, hipStream_t, const double*, double, int);
 template int launch_coarse1<float>(int, const GridDims&, int, const double*, const float*, const int*, int, long long,
                                    const double*, const float*, const float*, const float*, double, float*, hipStream_t,
-                                   const float*, double);
+                                   const float*, double, int);
 
 // Zero pattern the level-1 kernel may skip for a table (coarse1_table layout): 2 when K0 has the box class
 // pattern and every entry outside the numerical pattern is below 1e-14 of the largest, 1 with the class

@@ -137,6 +137,9 @@ v2_down_kernel(GridDims gf, GridDims gc, V2Op<T> op, Sweeps2 sw, int ct, const T
   const int i = 2 * I0 - 1 - sw.n + tx, j = 2 * J0 - 1 - sw.n + ty;
   const bool in = i >= 0 && i < gf.nx && j >= 0 && j < gf.ny;
   const long long n = (long long)j * gf.nx + i;
+  b += 2 * (long long)blockIdx.z * gf.nnodes;  // column
+  uo += 2 * (long long)blockIdx.z * gf.nnodes;
+  bc += 2 * (long long)blockIdx.z * gc.nnodes;
   for (int q = ty * blockDim.x + tx; q < 2 * row * row; q += blockDim.x * blockDim.x) buf[q] = {(T)0, (T)0};
   T A[9][2][2];
   v2_row<T, FINE>(op, gf, i, j, A);
@@ -179,6 +182,10 @@ v2_up_kernel(GridDims gf, GridDims gc, V2Op<T> op, Sweeps2 sw, int t, const T* _
   const int i = blockIdx.x * t - sw.n + tx, j = blockIdx.y * t - sw.n + ty;
   const bool in = i >= 0 && i < gf.nx && j >= 0 && j < gf.ny;
   const long long n = (long long)j * gf.nx + i;
+  b += 2 * (long long)blockIdx.z * gf.nnodes;  // column
+  ui += 2 * (long long)blockIdx.z * gf.nnodes;
+  uo += 2 * (long long)blockIdx.z * gf.nnodes;
+  ec += 2 * (long long)blockIdx.z * gc.nnodes;
   for (int q = ty * blockDim.x + tx; q < 2 * row * row; q += blockDim.x * blockDim.x) buf[q] = {(T)0, (T)0};
   T A[9][2][2];
   v2_row<T, FINE>(op, gf, i, j, A);
@@ -222,13 +229,13 @@ bool v2_ok(const pmt_mg* mg, int steps) { return mg->dim == 2 && steps <= kV2Max
 // compute unit.  A sweep is bound by the LDS reads of a block's wavefronts, so while the blocks do not fill
 // the chip small ones are faster, although most of their nodes are halo; beyond, large ones compute less.
 template <typename F>
-int v2_side(int nx, int ny, F out) {
+int v2_side(int nx, int ny, int cols, F out) {
   int best = kV2W;
   long long cost = 0;
   for (int w = kV2W; w >= 12; w -= 2) {
     const int t = out(w);
     if (t < 1) break;
-    const long long blocks = (long long)((nx + t - 1) / t) * ((ny + t - 1) / t);
+    const long long blocks = (long long)cols * ((nx + t - 1) / t) * ((ny + t - 1) / t);
     const long long c = (blocks + device_cu_count() - 1) / device_cu_count() * ((w * w + 63) / 64);
     if (w == kV2W || c < cost) {
       cost = c;
@@ -244,12 +251,13 @@ size_t v2_lds(int w) {
 }
 
 template <typename T>
-int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s) {
+int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s,
+                   int cols) {
   Level& L = mg->L[l];
   const GridDims& gc = mg->L[l + 1].g;
   auto coarse = [&](int w) { return (w - 2 - 2 * sw.n) / 2; };  // 2 ct + 1 residuals per side and the halo
-  const int w = v2_side(gc.nx, gc.ny, coarse), ct = coarse(w);
-  const dim3 grid((gc.nx + ct - 1) / ct, (gc.ny + ct - 1) / ct), block(w, w);
+  const int w = v2_side(gc.nx, gc.ny, cols, coarse), ct = coarse(w);
+  const dim3 grid((gc.nx + ct - 1) / ct, (gc.ny + ct - 1) / ct, cols), block(w, w);
   const V2Op<T> op = v2_op<T>(mg, L, L.buf<T>(), l == 0, xe);
   if (l == 0)
     v2_down_kernel<T, true><<<grid, block, v2_lds<T>(w), s>>>(L.g, gc, op, sw, ct, b, u, bc);
@@ -260,11 +268,11 @@ int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b
 
 template <typename T>
 int launch_v2_up(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, const T* ui, const T* ec, T* uo,
-                 hipStream_t s) {
+                 hipStream_t s, int cols) {
   Level& L = mg->L[l];
   auto nodes = [&](int w) { return w - 2 * sw.n; };
-  const int w = v2_side(L.g.nx, L.g.ny, nodes), t = nodes(w);
-  const dim3 grid((L.g.nx + t - 1) / t, (L.g.ny + t - 1) / t), block(w, w);
+  const int w = v2_side(L.g.nx, L.g.ny, cols, nodes), t = nodes(w);
+  const dim3 grid((L.g.nx + t - 1) / t, (L.g.ny + t - 1) / t, cols), block(w, w);
   const V2Op<T> op = v2_op<T>(mg, L, L.buf<T>(), l == 0, xe);
   if (l == 0)
     v2_up_kernel<T, true><<<grid, block, v2_lds<T>(w), s>>>(L.g, mg->L[l + 1].g, op, sw, t, b, ui, ec, uo);
@@ -274,8 +282,9 @@ int launch_v2_up(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, 
 }
 
 #define PMT_V2_INST(T)                                                                                              \
-  template int launch_v2_down<T>(pmt_mg*, int, const T*, const Sweeps2&, const T*, T*, T*, hipStream_t);             \
-  template int launch_v2_up<T>(pmt_mg*, int, const T*, const Sweeps2&, const T*, const T*, const T*, T*, hipStream_t);
+  template int launch_v2_down<T>(pmt_mg*, int, const T*, const Sweeps2&, const T*, T*, T*, hipStream_t, int);        \
+  template int launch_v2_up<T>(pmt_mg*, int, const T*, const Sweeps2&, const T*, const T*, const T*, T*,             \
+                               hipStream_t, int);
 PMT_V2_INST(double)
 PMT_V2_INST(float)
 #undef PMT_V2_INST

@@ -62,3 +62,30 @@ def test_dependent_columns(gpu_lib, k):
     X = cg.solve(B)
     assert cg.iterations < 300 and true_residual(K, X, B) < 2e-10
     assert float((X[:, k - 1] + 3.0 * X[:, 0]).abs().max() / X.abs().max()) < 1e-7
+
+
+@pytest.mark.parametrize("k", [2, 5])
+def test_columns_through_every_level_operator(gpu_lib, k):
+    """The same solve through each operator that takes several columns: level 1 stored or stencil-free, the fine
+    grid's kernels (all columns in one launch or one each) and the matrix-core sweeps.  A wrong column would
+    cost the preconditioner its effect: the iteration counts agree (two more with BF16 sweeps)."""
+    from pymoto_amd import tune
+    d, K, B = problem((24, 16, 8), k, 7)
+    its = {}
+    try:
+        for free in (False, True):
+            for kernel in (0, 1, 2):
+                for prec in ("fp64", "fp32", "bf16"):
+                    tune.set_coarse_level1(free)
+                    tune.set_tuning(fine_kernel=kernel)
+                    mg = pm.solvers.build_hierarchy(d, 3, omega=0.4, smooth_steps=2, precision=prec)
+                    cg = pm.solvers.CG(preconditioner=mg, tol=1e-10, maxit=300)
+                    cg.update(K)
+                    X = cg.solve(B)
+                    assert true_residual(K, X, B) < 2e-10
+                    its[free, kernel, prec] = cg.iterations
+    finally:
+        tune.set_coarse_level1(None)
+        tune.set_tuning(**tune.DEFAULT)
+    base = its[False, 0, "fp64"]
+    assert all(abs(n - base) <= (2 if key[2] == "bf16" else 1) for key, n in its.items()), its
