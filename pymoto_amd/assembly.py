@@ -293,8 +293,10 @@ class AssembleGeneral(Module):
             raise NotImplementedError("the device assembly back-propagates DyadicMatrix sensitivities only")
         g, lib = self.grid, _lib.lib()
         xs = self.sig_in[0].state
-        dx = torch.zeros(self.nel, dtype=torch.float64, device=_lib.device())
-        for k, (u, v, fac) in enumerate(dgdmat.terms()):
+        terms = list(dgdmat.terms())
+        # the first term's contraction writes every element, the others add to it
+        dx = (torch.empty if terms else torch.zeros)(self.nel, dtype=torch.float64, device=_lib.device())
+        for k, (u, v, fac) in enumerate(terms):
             if g.scalar:
                 rc = lib.pmt_scalar_sens_contract(*g.nel3, _lib.ptr(g.K0_dev), _lib.ptr(g.bcmask_dev), _lib.ptr(u),
                                                   _lib.ptr(v), float(fac), _lib.ptr(dx), int(k > 0), _lib.stream())
