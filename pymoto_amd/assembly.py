@@ -19,7 +19,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .core import Module
+from .core import Module, returns_new_arrays
 from .domain import VoxelDomain
 from .dyadic import DyadicMatrix
 
@@ -286,6 +286,7 @@ class AssembleGeneral(Module):
             raise ValueError(f"Input vector wrong size ({xe.numel()}), must be equal to #nel ({self.nel})")
         return StiffnessMatrix(self.grid, xe.reshape(-1))
 
+    @returns_new_arrays
     def _sensitivity(self, dgdmat):
         if dgdmat is None:
             return [None]

@@ -118,6 +118,15 @@ def _zeros_like(state: Any) -> Any:
         raise TypeError(f"cannot create a zero sensitivity for a state of type {type(state).__name__}") from None
 
 
+def returns_new_arrays(f):
+    """Marks a ``_sensitivity`` whose results are newly allocated, distinct, and kept by nobody: the first term
+    of a signal's sensitivity is then taken over instead of copied (the copy of a 192x96x96 density vector took 5.6 us
+    on the device and 13 us per module with its launch).  The mark belongs to the function: an override without it
+    goes back to copies."""
+    f.returns_new_arrays = True
+    return f
+
+
 # --------------------------------------------------------------------------------------------
 # signals
 
@@ -353,8 +362,14 @@ class Module(metaclass=_ModuleMeta):
             d_in = list(d_in) if isinstance(d_in, (list, tuple)) else [d_in]
             if len(d_in) != len(self.sig_in):
                 raise TypeError(f"_sensitivity returned {len(d_in)} values for {len(self.sig_in)} inputs")
+            fresh = getattr(self._sensitivity, "returns_new_arrays", False)
             for s, d in zip(self.sig_in, d_in):
-                if _is_signal(s):
+                if not _is_signal(s):
+                    continue
+                if fresh and d is not None and getattr(s.add_sensitivity, "__func__", None) is Signal.add_sensitivity \
+                        and s.sensitivity is None:
+                    s.sensitivity = d  # nobody else holds it: no private copy needed
+                else:
                     s.add_sensitivity(d)
         except Exception as e:
             _rethrow(e, self._describe())

@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .core import Module
+from .core import Module, returns_new_arrays
 from .domain import VoxelDomain
 
 
@@ -140,6 +140,7 @@ class FilterConv(Module):
                                       _lib.ptr(xd), _lib.ptr(y), _lib.stream()), "filter forward")
         return y
 
+    @returns_new_arrays
     def _sensitivity(self, dfdv):
         lib = _lib.lib()
         dy = _lib.as_device(dfdv).reshape(-1)
@@ -192,6 +193,7 @@ class DensityFilter(Module):
         xd = _lib.as_device(x)
         return self._apply(xd, so=self._scale(xd))
 
+    @returns_new_arrays
     def _sensitivity(self, dfdy):
         dy = _lib.as_device(dfdy)
         dx = self._apply(dy, si=self._scale(dy))

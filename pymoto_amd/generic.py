@@ -15,7 +15,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .core import Module
+from .core import Module, returns_new_arrays
 
 
 def _printed_float(v) -> float:
@@ -138,6 +138,7 @@ class MathExpression(Module):
                    "power law")
         return y
 
+    @returns_new_arrays
     def _sensitivity(self, df_dy):
         x = _lib.as_device(self.sig_in[0].state)
         dy = _lib.as_device(df_dy)
@@ -216,6 +217,7 @@ class EinSum(Module):
         ut, vt = u.t().contiguous(), v.t().contiguous()  # column j contiguous
         return torch.cat([self._dot(ut[j], vt[j]) for j in range(ut.shape[0])])
 
+    @returns_new_arrays
     def _sensitivity(self, df_in):
         inps = self.get_input_states(as_list=True)
         if len(inps) == 1:
