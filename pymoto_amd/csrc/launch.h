@@ -54,7 +54,8 @@ int launch_fine_refl(int mode, const GridDims& g, int planes /* 0 = from the occ
                      const uint8_t* bcm, double bcdiag, const T* u, const T* b, const T* dinv, double omega, T* y,
                      hipStream_t s, const T* up, double beta, int cols = 1);
 // q = A p on the fine grid with out[0] = p.q and out[1] = p.r (deterministic two-stage sums; ws holds
-// 2 * ws_parts doubles).  Returns PMT_ERR_STATE (nothing launched) when the reflection kernel is not the
+// 2 * ws_parts doubles).  parts (optional): if the sums' partials are few they are left in ws (*parts of p.q, then
+// of p.r) for the caller to add, else *parts = 0.  Returns PMT_ERR_STATE (nothing launched) when the reflection kernel is not the
 // fine operator or the launch needs more partial sums than ws holds; the caller then runs K.u and
 // the dot products separately.
 // element product of the fine reflection-basis kernel: 2 = the isotropic cube's 8 numbers, 1 = the box
@@ -65,7 +66,7 @@ inline int refl_pattern(int k0_pattern) {
 }
 int launch_fine_apply_dots(const GridDims& g, const double* K0ext, int k0_pattern, const double* xe,
                            const uint8_t* bcm, double bcdiag, const double* p, const double* r, double* q,
-                           double* ws, long long ws_parts, double* out, hipStream_t s);
+                           double* ws, long long ws_parts, double* out, hipStream_t s, int* parts = nullptr);
 long long fine_apply_dots_parts(const GridDims& g);  // a sufficient ws_parts for the grid
 // refl.hip: dx = alpha u_e^T K0 v_e (accumulate: dx += ...) in the reflection basis over z-streamed node
 // columns; tab = the FP64 block entries behind K0; hex8 only
@@ -111,19 +112,28 @@ int launch_dot(long long n, const double* x, const float* y, double* out, double
 int launch_dot2(long long n, const double* a0, const double* b0, const double* a1, const double* b1, double* out,
                 double* work, hipStream_t s);
 int launch_axpby(long long n, double a, const double* x, double b, double* y, hipStream_t s);
-// x = nullptr: r only (the x update deferred to launch_cg_p_update).  work: cg_xr_parts(n) partial sums
 long long cg_xr_parts(long long n);
+// np partials (few enough) are added by the kernels that need their sum instead of by a launch
+bool cg_sums_inline(long long np);
 // x.y in one flat pass, work: cg_xr_parts(n) partials (the CG loop's dots; bits differ from launch_dot's)
 template <typename Y>
 int launch_dot_flat(long long n, const double* x, const Y* y, double* out, double* work, hipStream_t s);
-int launch_cg_xr_update(long long n, const double* sc, const double* p, const double* q, double* x, double* r,
-                        double* work, double* out_rr, hipStream_t s, float* r32 = nullptr,
-                        const float* dinv32 = nullptr, float omega32 = 0.0f, float* u1 = nullptr,
-                        double* host = nullptr, double seq = 0.0);  // host: also publish r.r (launch_publish)
+// the partials of a0.b0 and, behind them, of a1.b1 (cg_xr_parts(n) each) in work
+int launch_dot2_flat(long long n, const double* a0, const double* b0, const double* a1, const double* b1,
+                     double* work, hipStream_t s);
+// r -= alpha q and the sum of r.r, alpha = sc[1] / sc[0]; dots (optional): the np partials of p.q and behind them those
+// of p.r, whose sums go to sc[0], sc[1] first.  (x += alpha p: launch_cg_beta_update.)  work: cg_xr_parts(n)
+// partial sums
+template <typename U>
+int launch_cg_xr_update(long long n, double* sc, const double* dots, long long np, const double* q, double* r,
+                        double* work, double* out_rr, hipStream_t s, float* r32 = nullptr, const U* dinv = nullptr,
+                        double omega = 0.0, U* u1 = nullptr, double* host = nullptr, double seq = 0.0);  // host: also publish r.r (launch_publish)
 int launch_cg_x_update(long long n, const double* sc, const double* p, double* x, hipStream_t s);
-// x (optional): also x += (sc[1]/sc[0]) p_old first, the update a cg_xr_update with x = nullptr deferred
-int launch_cg_p_update(long long n, const double* sc, const double* z, double* p, hipStream_t s, double* x = nullptr);
-int launch_cg_p_update(long long n, const double* sc, const float* z, double* p, hipStream_t s, double* x = nullptr);
+// p = z - (q.z / sc[0]) p; x (optional): also x += (sc[1]/sc[0]) p_old first, the update that launch_cg_xr_update
+// left out.  work: cg_xr_parts(n) partial sums; sc[3] is scratch
+template <typename Z>
+int launch_cg_beta_update(long long n, double* sc, const double* q, const Z* z, double* p, double* work, double* x,
+                          hipStream_t s);
 int launch_scale_rsqrt(long long n, const double* sc, int k, const double* z, double* p, hipStream_t s);
 int launch_fill(long long n, double v, double* y, hipStream_t s);
 // host[0] = *v, then host[1] = seq (pinned host memory; the host polls host[1])

@@ -665,7 +665,7 @@ int pmt_mg_create(int nelx, int nely, int nelz, int nlevels, const double* omega
   ALLOC(mg->r, n0);
   ALLOC(mg->sc, 16);
   ALLOC(mg->work, 2 * kReduceBlocks);
-  ALLOC(mg->rwork, cg_xr_parts(n0));
+  ALLOC(mg->rwork, 3 * cg_xr_parts(n0));  // r.r or q.z, then p.q and p.r
   ALLOC(mg->cs_buf, 4 + 4 * kReduceBlocks);
   if (hex && (mg->k0pat & PMT_K0_REFLECTION)) {
     mg->dotws_parts = fine_apply_dots_parts(mg->L[0].g);
@@ -889,48 +889,62 @@ int pmt_pcg_solve(pmt_mg* mg, const double* b, double* x, int x0_is_zero, double
   double tprev = 0.0;  // the relative residual one iteration before tval (0: none yet)
   bool x_pending = false;  // x lacks this iteration's alpha p (added by the p update or after the loop)
   for (i = 0; i < maxit; ++i) {
-    // q = A p, sc[0] = p.q, sc[1] = p.r: fused into the reflection-basis operator when it is the fine
-    // operator, else K.u and one two-dot pass
+    // q = A p with the partials of p.q and p.r (dots, np each): fused into the reflection-basis operator when it
+    // is the fine operator, else K.u and one two-dot pass.  The r update adds them if they are few; a restart
+    // (which updates x instead) and larger problems have them added to sc[0], sc[1] here
+    const bool restart_now = i % restart == 0;
+    const double* dots = nullptr;
+    int np = 0;
     const int frc = mg->dotws ? launch_fine_apply_dots(F.g, mg->K0, mg->k0pat, mg->xe, mg->bcm, mg->bcdiag, mg->p,
-                                                       mg->r, mg->q, mg->dotws, mg->dotws_parts, sc, s)
+                                                       mg->r, mg->q, mg->dotws, mg->dotws_parts, sc, s,
+                                                       restart_now ? nullptr : &np)
                               : PMT_ERR_STATE;
     if (frc == PMT_ERR_STATE) {
       PMT_TRY(level_apply<double>(mg, 0, MODE_APPLY, mg->p, nullptr, mg->q, s));
-      PMT_TRY(launch_dot2(n, mg->p, mg->q, mg->p, mg->r, sc, mg->work, s));
+      if (!restart_now && cg_sums_inline(cg_xr_parts(n))) {
+        np = (int)cg_xr_parts(n);
+        PMT_TRY(launch_dot2_flat(n, mg->p, mg->q, mg->p, mg->r, mg->rwork + np, s));
+        dots = mg->rwork + np;
+      } else {
+        PMT_TRY(launch_dot2(n, mg->p, mg->q, mg->p, mg->r, sc, mg->work, s));
+      }
     } else {
       PMT_TRY(frc);
+      dots = np > 0 ? mg->dotws : nullptr;
     }
     // reduced-precision V-cycles: the update also writes r in FP32 (the V-cycle's input), and z stays
     // FP32 (q.z and p = z + beta p widen it exactly: the same sums as through an FP64 copy)
     const bool mixed = mg->prec != 64;
     // the update also writes the V-cycle's first fine sweep from zero into the fine level's work vector:
-    // omega D^-1 r32 (damped Jacobi) or D^-1 r32 / theta (Chebyshev), the same FP32 expression as the
-    // sweep kernel
-    const bool first = mixed && (mg->smoother == 0 || mg->smoother == 1);
+    // omega D^-1 r (damped Jacobi) or D^-1 r / theta (Chebyshev) in the V-cycle's precision, the expression
+    // of the sweep kernel
+    const bool first = !v2_ok(mg, F.steps);  // (the Q4 V-cycle starts from r)
     const double first_factor = first_sweep_factor(mg, 0);
-    bool r32_ready = false;
+    bool r_ready = false;  // the V-cycle's input (and first sweep) are written
     bool published = false;  // r.r already on its way to the host (with the r update's reduction)
-    if (i % restart == 0) {
+    if (restart_now) {
       PMT_TRY(launch_cg_x_update(n, sc, mg->p, x, s));
       PMT_TRY(level_apply<double>(mg, 0, MODE_RESIDUAL, x, b, mg->r, s));
       PMT_TRY(launch_dot(n, mg->r, mg->r, sc + 2, mg->work, s));
     } else {
       // x += alpha p is deferred to the p update, which reads p anyway (x_pending until it runs)
       const double seq = next_publish_seq(mg);
-      PMT_TRY(launch_cg_xr_update(n, sc, mg->p, mg->q, nullptr, mg->r, mg->rwork, sc + 2, s, mixed ? F.f.b : nullptr,
-                                  first ? F.f.dinv : nullptr, (float)first_factor, first ? F.f.t : nullptr,
-                                  mg->host_rr, seq));
-      r32_ready = mixed;
+      if (mixed)
+        PMT_TRY(launch_cg_xr_update<float>(n, sc, dots, np, mg->q, mg->r, mg->rwork, sc + 2, s, F.f.b,
+                                           F.f.dinv, first_factor, first ? F.f.t : nullptr, mg->host_rr, seq));
+      else
+        PMT_TRY(launch_cg_xr_update<double>(n, sc, dots, np, mg->q, mg->r, mg->rwork, sc + 2, s, nullptr,
+                                            F.d.dinv, first_factor, first ? F.d.t : nullptr, mg->host_rr, seq));
+      r_ready = true;
       x_pending = true;
       published = true;
     }
     // z = M r, sc[3] = q.z, p = z + beta p: reads r and q, writes only z, sc[3] and p (no result)
     auto next_direction = [&]() -> int {
       if (mixed) {
-        PMT_TRY(precondition_f32(mg, mg->r, mg->z32, r32_ready, s, r32_ready && first));
+        PMT_TRY(precondition_f32(mg, mg->r, mg->z32, r_ready, s, r_ready && first));
         if (mg->cs_m == 0) {
-          PMT_TRY(launch_dot_flat(n, mg->q, mg->z32, sc + 3, mg->rwork, s));
-          PMT_TRY(launch_cg_p_update(n, sc, mg->z32, mg->p, s, x_pending ? x : nullptr));
+          PMT_TRY(launch_cg_beta_update(n, sc, mg->q, mg->z32, mg->p, mg->rwork, x_pending ? x : nullptr, s));
           x_pending = false;
           return PMT_OK;
         }
@@ -938,11 +952,10 @@ int pmt_pcg_solve(pmt_mg* mg, const double* b, double* x, int x0_is_zero, double
         // along W of relative size 1e-7 in every direction, and CG would stall at that level
         PMT_TRY(launch_to_double(n, mg->z32, mg->z, s));
       } else {
-        PMT_TRY(precondition(mg, mg->r, mg->z, s));
+        PMT_TRY(vcycle<double>(mg, 0, mg->r, mg->z, s, r_ready && first));
       }
       PMT_TRY(launch_coarse_correct(n, mg->cs_m, mg->cs_W, mg->cs_AW, mg->cs_Einv, mg->cs_buf, mg->z, s));
-      PMT_TRY(launch_dot_flat(n, mg->q, mg->z, sc + 3, mg->rwork, s));
-      PMT_TRY(launch_cg_p_update(n, sc, mg->z, mg->p, s, x_pending ? x : nullptr));
+      PMT_TRY(launch_cg_beta_update(n, sc, mg->q, mg->z, mg->p, mg->rwork, x_pending ? x : nullptr, s));
       x_pending = false;
       return PMT_OK;
     };

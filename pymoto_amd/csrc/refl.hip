@@ -846,7 +846,7 @@ __global__ void __launch_bounds__(256) sum_parts_kernel(const double* __restrict
 
 int launch_fine_apply_dots(const GridDims& g, const double* K0ext, int k0_pattern, const double* xe,
                            const uint8_t* bcm, double bcdiag, const double* p, const double* r, double* q,
-                           double* ws, long long ws_parts, double* out, hipStream_t s) {
+                           double* ws, long long ws_parts, double* out, hipStream_t s, int* parts) {
   if (g.dim != 3 || get_tuning(PMT_TUNE_FINE_KERNEL) != 2 || !(k0_pattern & PMT_K0_REFLECTION) ||
       ws_parts < fine_apply_dots_parts(g))
     return PMT_ERR_STATE;
@@ -864,6 +864,8 @@ int launch_fine_apply_dots(const GridDims& g, const double* K0ext, int k0_patter
     launch_refl_rows<0, 0, double>(rows, MODE_APPLY_DOTS, g, tuned_stream_planes(), tab, xe, bcm, bcdiag, p, r,
                                    nullptr, 0.0, q, s, nullptr, 0.0, ws, &nwork);
   PMT_TRY(check_launch("fine_refl_kernel<apply + dots>"));
+  if (parts) *parts = cg_sums_inline(nwork) ? nwork : 0;
+  if (parts && *parts > 0) return PMT_OK;
   sum_parts_kernel<<<1, 256, 0, s>>>(ws, nwork, out);
   return check_launch("sum_parts_kernel");
 }

@@ -900,8 +900,11 @@ int pmt_smg_pcg_solve(pmt_smg* h, const double* b, double* x, int x0_is_zero, do
   bool x_pending = false;  // x lacks this iteration's alpha p (added by the p update or after the loop)
   for (it = 0; it < maxit; ++it) {
     PMT_TRY(smg_apply(h, 0, h->p, h->q, s, h->r));
-    scalar_sum2_kernel<<<1, 512, 0, s>>>(nparts, h->parts, sc);
-    PMT_TRY(check_launch("scalar_sum2_kernel"));
+    const bool inline_sums = it % restart != 0 && cg_sums_inline(nparts);  // the r update adds the partials
+    if (!inline_sums) {
+      scalar_sum2_kernel<<<1, 512, 0, s>>>(nparts, h->parts, sc);
+      PMT_TRY(check_launch("scalar_sum2_kernel"));
+    }
     const double seq = publish_sequence();
     if (it % restart == 0) {
       PMT_TRY(launch_cg_x_update(n, sc, h->p, x, s));
@@ -909,15 +912,14 @@ int pmt_smg_pcg_solve(pmt_smg* h, const double* b, double* x, int x0_is_zero, do
       PMT_TRY(launch_dot(n, h->r, h->r, sc + 2, h->work, s));
       PMT_TRY(launch_publish(sc + 2, seq, h->host, s));
     } else {
-      PMT_TRY(launch_cg_xr_update(n, sc, h->p, h->q, nullptr, h->r, h->work, sc + 2, s, nullptr, nullptr, 0.0f, nullptr,
-                                  h->host, seq));
+      PMT_TRY(launch_cg_xr_update<double>(n, sc, inline_sums ? h->parts : nullptr, nparts, h->q, h->r,
+                                          h->work, sc + 2, s, nullptr, nullptr, 0.0, nullptr, h->host, seq));
       x_pending = true;
     }
     // z = M r, beta = -(q.z) / (p.q), p = z + beta p
     auto next_direction = [&]() -> int {
       PMT_TRY(smg_vcycle(h, 0, h->r, h->z, s));
-      PMT_TRY(launch_dot_flat(n, h->q, h->z, sc + 3, h->work, s));
-      PMT_TRY(launch_cg_p_update(n, sc, h->z, h->p, s, x_pending ? x : nullptr));
+      PMT_TRY(launch_cg_beta_update(n, sc, h->q, h->z, h->p, h->work, x_pending ? x : nullptr, s));
       x_pending = false;
       return PMT_OK;
     };

@@ -372,46 +372,122 @@ int launch_dot2(long long n, const double* a0, const double* b0, const double* a
   return check_launch("dot_stage2<2>");
 }
 
-// CG: x += alpha p (WITHX; else the caller adds it later, in cg_p_update), r -= alpha q, partial ||r||^2;
-// alpha = sc[1]/sc[0] read on device; r32 (optional): the new r rounded to FP32, the input of a
-// reduced-precision preconditioner; u1 (optional, with r32): omega * D^-1 * r32, the preconditioner's
-// first sweep from zero (same FP32 expression as jacobi0_kernel).  One pass over the vectors: a block
+// CG: r -= alpha q, partial ||r||^2 (x += alpha p comes later, with the p update); alpha = sc[1]/sc[0] read on
+// device; r32 (optional): the new r rounded to FP32, the input of a
+// reduced-precision preconditioner; u1 (optional): omega * D^-1 * r, the preconditioner's first sweep from zero
+// in its precision (the expression of jacobi0_kernel).  One pass over the vectors: a block
 // owns kXrPer * 256 consecutive entries (strided by 256 per step, so every step is coalesced and the
 // steps' loads are independent) and writes its sum of r^2 to partial[block]; the fixed-order second
 // stage is parts_stage2.  At 12.8M dofs: 71 us (4 per thread) for the 461 MB of the mixed-precision
 // update, where the fixed 1024-block grid-stride loop of the dots took 84 us.
 constexpr int kXrPer = 4;
+constexpr long long kMaxParts = 2048;
 
 long long cg_xr_parts(long long n) { return (n + 256LL * kXrPer - 1) / (256LL * kXrPer); }
 
-template <bool WITHX>
-__global__ void __launch_bounds__(kReduceThreads)
-cg_xr_update(long long n, const double* __restrict__ sc, const double* __restrict__ p, const double* __restrict__ q,
-             double* __restrict__ x, double* __restrict__ r, double* __restrict__ partial, float* __restrict__ r32,
-             const float* __restrict__ dinv32, float omega32, float* __restrict__ u1) {
-  const double alpha = sc[1] / sc[0];
-  double s = 0.0;
-  const long long base = (long long)blockIdx.x * (256 * kXrPer) + threadIdx.x;
-  auto step = [&](long long i) {
-    if (WITHX) x[i] = fma(alpha, p[i], x[i]);
-    const double rv = fma(-alpha, q[i], r[i]);
-    r[i] = rv;
-    if (r32) {
-      const float rf = (float)rv;
-      r32[i] = rf;
-      if (u1) u1[i] = omega32 * dinv32[i] * rf;
+// The sums of NOUT sets of np <= kMaxParts partials (set o at partial + o * np), in a fixed order, in every thread
+// of a block of 256: a kernel that needs them adds them itself, all loads in flight, instead of waiting for a
+// launch that does (3 to 4 us each on the chain of a small problem's iteration; 1 us here).  An iteration on
+// 96x48x48 (FP64) so took 15 us less of 180; on 256x128x128 (760 partials, 12,530 blocks that add them) the same.
+template <int NOUT>
+__device__ inline void block_parts(const double* __restrict__ partial, int np, double (&out)[NOUT]) {
+  constexpr int PER = (int)(kMaxParts / kReduceThreads);
+  __shared__ double sh[NOUT][kReduceThreads / 64];
+  double v[NOUT][PER];
+#pragma unroll
+  for (int o = 0; o < NOUT; ++o)
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int b = threadIdx.x + k * kReduceThreads;
+      v[o][k] = b < np ? partial[o * np + b] : 0.0;
     }
-    s = fma(rv, rv, s);
+#pragma unroll
+  for (int o = 0; o < NOUT; ++o) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) t += v[o][k];
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[o][threadIdx.x >> 6] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int o = 0; o < NOUT; ++o) {
+    out[o] = 0.0;
+    for (int w = 0; w < kReduceThreads / 64; ++w) out[o] += sh[o][w];
+  }
+}
+
+// dots (np > 0): the partials of p.q and p.r, added here; block 0 leaves the sums in sc[0], sc[1]
+template <bool PARTS, typename U>
+__global__ void __launch_bounds__(kReduceThreads)
+cg_xr_update(long long n, double* __restrict__ sc, const double* __restrict__ dots, int np,
+             const double* __restrict__ q, double* __restrict__ r, double* __restrict__ partial,
+             float* __restrict__ r32, const U* __restrict__ dinv, U omega, U* __restrict__ u1) {
+  const long long base = (long long)blockIdx.x * (256 * kXrPer) + threadIdx.x;
+  double qv[kXrPer], rv[kXrPer];
+  U dv[kXrPer];
+  if constexpr (PARTS) {  // the entries' loads are in flight during the sums
+#pragma unroll
+    for (int k = 0; k < kXrPer; ++k) {
+      const long long i = base + 256LL * k < n ? base + 256LL * k : n - 1;
+      qv[k] = q[i];
+      rv[k] = r[i];
+      dv[k] = u1 ? dinv[i] : (U)0;
+    }
+  }
+  double alpha;
+  if constexpr (PARTS) {
+    double pq[2];
+    block_parts<2>(dots, np, pq);
+    alpha = pq[1] / pq[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      sc[0] = pq[0];
+      sc[1] = pq[1];
+    }
+  } else {
+    alpha = sc[1] / sc[0];
+  }
+  double s = 0.0;
+  auto step = [&](int k) {
+    const long long i = base + 256LL * k;
+    const double v = PARTS ? fma(-alpha, qv[k], rv[k]) : fma(-alpha, q[i], r[i]);
+    r[i] = v;
+    const U rf = (U)v;
+    if (r32) r32[i] = (float)v;
+    if (u1) u1[i] = omega * (PARTS ? dv[k] : dinv[i]) * rf;
+    s = fma(v, v, s);
   };
   if (base + 256LL * (kXrPer - 1) < n) {  // every block but the last: no bounds test between the steps
 #pragma unroll
-    for (int k = 0; k < kXrPer; ++k) step(base + 256LL * k);
+    for (int k = 0; k < kXrPer; ++k) step(k);
   } else {
+#pragma unroll
     for (int k = 0; k < kXrPer; ++k)
-      if (base + 256LL * k < n) step(base + 256LL * k);
+      if (base + 256LL * k < n) step(k);
   }
   double t = block_sum(s);
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
+// partials of a0.b0 (entry 0..) and a1.b1 (entry np..), blocks as dot_flat
+__global__ void __launch_bounds__(kReduceThreads)
+dot2_flat(long long n, const double* __restrict__ a0, const double* __restrict__ b0, const double* __restrict__ a1,
+          const double* __restrict__ b1, double* __restrict__ partial) {
+  double s0 = 0.0, s1 = 0.0;
+  const long long base = (long long)blockIdx.x * (256 * kXrPer) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kXrPer; ++k) {
+    const long long i = base + 256LL * k;
+    if (i < n) {
+      s0 = fma(a0[i], b0[i], s0);
+      s1 = fma(a1[i], b1[i], s1);
+    }
+  }
+  const double t0 = block_sum(s0), t1 = block_sum(s1);
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = t0;
+    partial[gridDim.x + blockIdx.x] = t1;
+  }
 }
 
 // x.y in one flat pass (the cg_xr_update blocking: kXrPer * 256 entries per block, partial[block]); its
@@ -442,7 +518,7 @@ __global__ void cg_x_update(long long n, const double* __restrict__ sc, const do
 
 // CG: p = z + beta p with beta = -sc[3]/sc[0]   (iterative.py:394-395); z FP64 or the FP32 output of a
 // reduced-precision preconditioner (widened exactly).  x (optional): first the x update the iteration's
-// cg_xr_update<false> left out, x += alpha p with alpha = sc[1]/sc[0] and the old p - the same
+// cg_xr_update left out, x += alpha p with alpha = sc[1]/sc[0] and the old p - the same
 // expression, so the iterates are bitwise those of the undeferred update, for one read of p fewer
 template <typename Z, bool WITHX>
 __global__ void cg_p_update(long long n, const double* __restrict__ sc, const Z* __restrict__ z,
@@ -453,6 +529,32 @@ __global__ void cg_p_update(long long n, const double* __restrict__ sc, const Z*
     const double pv = p[i];
     if (WITHX) x[i] = fma(sc[1] / sc[0], pv, x[i]);
     p[i] = fma(beta, pv, (double)z[i]);
+  }
+}
+
+// the same with q.z from its np partials (few blocks of kXrPer entries per thread: each adds them)
+template <typename Z, bool WITHX>
+__global__ void __launch_bounds__(kReduceThreads)
+cg_p_update_parts(long long n, const double* __restrict__ sc, const double* __restrict__ parts, int np,
+                  const Z* __restrict__ z, double* __restrict__ p, double* __restrict__ x) {
+  double qz[1], pv[kXrPer], zv[kXrPer], xv[kXrPer];
+  const double pq = sc[0], alpha = WITHX ? sc[1] / pq : 0.0;
+  const long long base = (long long)blockIdx.x * (256 * kXrPer) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kXrPer; ++k) {
+    const long long i = base + 256LL * k < n ? base + 256LL * k : n - 1;  // loads in flight during the sum
+    pv[k] = p[i];
+    zv[k] = (double)z[i];
+    xv[k] = WITHX ? x[i] : 0.0;
+  }
+  block_parts<1>(parts, np, qz);
+  const double beta = -qz[0] / pq;
+#pragma unroll
+  for (int k = 0; k < kXrPer; ++k) {
+    const long long i = base + 256LL * k;
+    if (i >= n) return;
+    if (WITHX) x[i] = fma(alpha, pv[k], xv[k]);
+    p[i] = fma(beta, pv[k], zv[k]);
   }
 }
 
@@ -497,18 +599,34 @@ int launch_axpby(long long n, double a, const double* x, double b, double* y, hi
   return check_launch("axpby_kernel");
 }
 
-int launch_cg_xr_update(long long n, const double* sc, const double* p, const double* q, double* x, double* r,
-                        double* work, double* out_rr, hipStream_t s, float* r32, const float* dinv32, float omega32,
-                        float* u1, double* host, double seq) {
+bool cg_sums_inline(long long np) { return np <= kMaxParts; }
+
+template <typename U>
+int launch_cg_xr_update(long long n, double* sc, const double* dots, long long np, const double* q, double* r,
+                        double* work, double* out_rr, hipStream_t s, float* r32, const U* dinv, double omega, U* u1,
+                        double* host, double seq) {
   if (n <= 0) return PMT_OK;
   const long long parts = cg_xr_parts(n);
-  if (x)
-    cg_xr_update<true><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, p, q, x, r, work, r32, dinv32, omega32, u1);
+  if (dots)
+    cg_xr_update<true, U><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, dots, (int)np, q, r, work, r32, dinv,
+                                                                    (U)omega, u1);
   else
-    cg_xr_update<false><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, p, q, x, r, work, r32, dinv32, omega32, u1);
+    cg_xr_update<false, U><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, nullptr, 0, q, r, work, r32, dinv,
+                                                                     (U)omega, u1);
   PMT_TRY(check_launch("cg_xr_update"));
   parts_stage2<<<1, kStage2Threads, 0, s>>>(work, parts, out_rr, seq, host);
   return check_launch("parts_stage2");
+}
+template int launch_cg_xr_update<double>(long long, double*, const double*, long long, const double*, double*, double*,
+                                         double*, hipStream_t, float*, const double*, double, double*, double*, double);
+template int launch_cg_xr_update<float>(long long, double*, const double*, long long, const double*, double*, double*,
+                                        double*, hipStream_t, float*, const float*, double, float*, double*, double);
+
+int launch_dot2_flat(long long n, const double* a0, const double* b0, const double* a1, const double* b1,
+                     double* work, hipStream_t s) {
+  if (n <= 0) return PMT_OK;
+  dot2_flat<<<(unsigned)cg_xr_parts(n), kReduceThreads, 0, s>>>(n, a0, b0, a1, b1, work);
+  return check_launch("dot2_flat");
 }
 
 double publish_sequence() {
@@ -568,21 +686,31 @@ int launch_cg_x_update(long long n, const double* sc, const double* p, double* x
   return check_launch("cg_x_update");
 }
 
-int launch_cg_p_update(long long n, const double* sc, const double* z, double* p, hipStream_t s, double* x) {
+template <typename Z>
+int launch_cg_beta_update(long long n, double* sc, const double* q, const Z* z, double* p, double* work, double* x,
+                          hipStream_t s) {
+  if (n <= 0) return PMT_OK;
+  const long long parts = cg_xr_parts(n);
+  if (!cg_sums_inline(parts)) {
+    PMT_TRY(launch_dot_flat(n, q, z, sc + 3, work, s));
+    if (x)
+      cg_p_update<Z, true><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, x);
+    else
+      cg_p_update<Z, false><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, nullptr);
+    return check_launch("cg_p_update");
+  }
+  dot_flat<Z><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, q, z, work);
+  PMT_TRY(check_launch("dot_flat"));
   if (x)
-    cg_p_update<double, true><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, x);
+    cg_p_update_parts<Z, true><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, work, (int)parts, z, p, x);
   else
-    cg_p_update<double, false><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, x);
-  return check_launch("cg_p_update");
+    cg_p_update_parts<Z, false><<<(unsigned)parts, kReduceThreads, 0, s>>>(n, sc, work, (int)parts, z, p, nullptr);
+  return check_launch("cg_p_update_parts");
 }
-
-int launch_cg_p_update(long long n, const double* sc, const float* z, double* p, hipStream_t s, double* x) {
-  if (x)
-    cg_p_update<float, true><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, x);
-  else
-    cg_p_update<float, false><<<blocks_for(n, 256), 256, 0, s>>>(n, sc, z, p, x);
-  return check_launch("cg_p_update<float>");
-}
+template int launch_cg_beta_update<double>(long long, double*, const double*, const double*, double*, double*, double*,
+                                           hipStream_t);
+template int launch_cg_beta_update<float>(long long, double*, const double*, const float*, double*, double*, double*,
+                                          hipStream_t);
 
 int launch_scale_rsqrt(long long n, const double* sc, int k, const double* z, double* p, hipStream_t s) {
   scale_rsqrt<<<blocks_for(n, 256), 256, 0, s>>>(n, sc, k, z, p);
