@@ -392,7 +392,7 @@ __global__ void dense_from_stencil_kernel(GridDims g, const double* __restrict__
 // again by every block of a column (the same work as the update, on compute units that would wait
 // otherwise); the block of the next diagonal tile inverts it at the end of its update, so its chain of
 // pivots runs beside the other tiles of the launch.
-// 24 us per panel at n = 847 (14 panels) and bound by that chain; four launches per panel (diagonal inverse, column
+// 21 us per panel at n = 847 (14 panels) and bound by that chain; four launches per panel (diagonal inverse, column
 // copy, row panel, update) took 76 us.  Above n = 1900 the tiles bound it: 25 ms at n = 6069 (45 ms before).
 constexpr int GJB = 64;
 constexpr int GJL = GJB + 2;  // LDS row stride: the 16 rows x 2 entries of a half wave's operand read lie in 64 banks
@@ -408,19 +408,17 @@ __device__ inline double gj_rcp(double x) {
 // In-place inverse of a 64 x 64 tile held by 4 waves in the matrix-core result layout (a wave per 32 x 32
 // quadrant: entry r of m[a][b] is row 32 (wave / 2) + 16 a + 4 r + lane / 16, column 32 (wave % 2) + 16 b +
 // lane % 16): block Gauss-Jordan with 4 x 4 pivot blocks Q, 16 steps with one barrier each.  The pivot rows R
-// and columns C go through LDS (sh: two buffers); every thread inverts Q itself; the rest is
-// m -= (C Q^-1) R, one matrix operation per 16 x 16 tile.  The pivot rows are one register (r = s % 4) of
+// and columns C go through LDS (sh: two buffers); every thread solves for the row of Q^-1 that it needs; the
+// rest is m -= C (Q^-1 R), one matrix operation per 16 x 16 tile.  The pivot rows are one register (r = s % 4) of
 // all lanes of a tile row and become Q^-1 R; in the pivot columns m counts as 0 and R as the identity.
-// 15 us, a chain of dependent FP64 operations.  (One pivot per step, the whole tile moving through LDS, took
-// 40 us; 4 x 4 entries per thread and the rank-4 update without the matrix cores 22 us.)
+// 12 us, a chain of dependent FP64 operations.  (With the whole of Q inverted by every thread, for (C Q^-1) R,
+// 15 us; 4 x 4 entries per thread and the rank-4 update without the matrix cores 22 us; one pivot per step, the
+// whole tile moving through LDS, 40 us.)
 constexpr int kGjShared = 2 * (256 + 256 + 16);  // doubles
 __device__ inline void gj_invert_tile(gj_d4 (&m)[2][2], double* sh, int tid) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  auto pick = [odd = (lq & 1) != 0, high = (lq & 2) != 0](double v0, double v1, double v2, double v3) {
-    const double lo = odd ? v1 : v0, hi = odd ? v3 : v2;  // by value: a select of array elements would index memory
-    return high ? hi : lo;
-  };
+  const double unit[4] = {lq == 0 ? 1.0 : 0.0, lq == 1 ? 1.0 : 0.0, lq == 2 ? 1.0 : 0.0, lq == 3 ? 1.0 : 0.0};
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
     double* rows = sh + (s & 1) * kGjShared / 2;  // R [4][64], the identity in the pivot columns
@@ -444,60 +442,49 @@ __device__ inline void gj_invert_tile(gj_d4 (&m)[2][2], double* sh, int tid) {
         for (int r = 0; r < 4; ++r) cols[(wr + 16 * a + 4 * r + lq) * 4 + l16 % 4] = m[a][ta][r];
     }
     __syncthreads();
-    double q[4][4], c[2][4], r1[2], rr[2][4];
+    double q[4][4], c[2], rr[2][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) q[i][j] = pivot[i * 4 + j];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2; ++a) c[a] = cols[(wr + 16 * a + l16) * 4 + lq];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) c[a][k] = cols[(wr + 16 * a + l16) * 4 + k];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      r1[b] = rows[lq * 64 + wc + 16 * b + l16];
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int k = 0; k < 4; ++k) rr[b][k] = rows[k * 64 + wc + 16 * b + l16];
-    }
     const double keep = piv ? 0.0 : 1.0;
 #pragma unroll
     for (int a = 0; a < 2; ++a) m[a][ta] *= keep;
+    // this lane's row y of Q^-1: y Q = e, Q = L U with the unit diagonal in L, y U first, along with the elimination
+    double y[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = unit[j];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const double inv = gj_rcp(q[p][p]);
+      y[p] *= inv;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) q[p][j] = j == p ? inv : q[p][j] * inv;
+      for (int j = p + 1; j < 4; ++j) y[j] = fma(-y[p], q[p][j], y[j]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (i == p) continue;
-        const double f = q[i][p];
+      for (int i = p + 1; i < 4; ++i) {
+        q[i][p] *= inv;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) q[i][j] = j == p ? -f * inv : fma(-f, q[p][j], q[i][j]);
+        for (int j = p + 1; j < 4; ++j) q[i][j] = fma(-q[i][p], q[p][j], q[i][j]);
       }
     }
-    // this lane's column and row of Q^-1
-    double qc[4], qr[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      qc[k] = pick(q[k][0], q[k][1], q[k][2], q[k][3]);
-      qr[k] = pick(q[0][k], q[1][k], q[2][k], q[3][k]);
-    }
+    for (int p = 3; p > 0; --p)
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      double x = c[a][0] * qc[0];
+      for (int j = 0; j < p; ++j) y[j] = fma(-y[p], q[p][j], y[j]);
 #pragma unroll
-      for (int k = 1; k < 4; ++k) x = fma(c[a][k], qc[k], x);
+    for (int b = 0; b < 2; ++b) {
+      double w = y[0] * rr[b][0];  // row lq of Q^-1 R
 #pragma unroll
-      for (int b = 0; b < 2; ++b) m[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x, r1[b], m[a][b], 0, 0, 0);
-    }
-    if (own_r) {
+      for (int k = 1; k < 4; ++k) w = fma(y[k], rr[b][k], w);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        double w = qr[0] * rr[b][0];
-#pragma unroll
-        for (int k = 1; k < 4; ++k) w = fma(qr[k], rr[b][k], w);
-        m[ta][b][s % 4] = w;
-      }
+      for (int a = 0; a < 2; ++a) m[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(-c[a], w, m[a][b], 0, 0, 0);
+      if (own_r) m[ta][b][s % 4] = w;
     }
   }
 }
