@@ -13,6 +13,10 @@
 // Coarsest level: dense matrix from the stencil, explicit inverse by blocked Gauss-Jordan
 // (no pivoting; the Galerkin operator is SPD), applied as a dense GEMV in every V-cycle -
 // the direct solve of auto_determine_solver (iterative.py:174-176).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
 #include "launch.h"
 
 namespace pmt {
@@ -390,10 +394,14 @@ __global__ void dense_from_stencil_kernel(GridDims g, const double* __restrict__
 // One launch per panel, a block per 64 x 64 tile: the panels are read from copies that the previous launch's
 // blocks of that row and column wrote beside the matrix, so the tiles are updated in place; P R_j is formed
 // again by every block of a column (the same work as the update, on compute units that would wait
-// otherwise); the block of the next diagonal tile inverts it at the end of its update, so its chain of
+// otherwise).  Of a symmetric matrix only the tiles on and above the diagonal are kept: its processed and its
+// remaining part stay symmetric and the entries between them change sign when mirrored, so the row panel is the
+// column panel transposed, negated for the processed columns; the last panel's launch writes the other half.
+// The block of the next diagonal tile inverts it at the end of its update, so its chain of
 // pivots runs beside the other tiles of the launch.
 // 21 us per panel at n = 847 (14 panels) and bound by that chain; four launches per panel (diagonal inverse, column
-// copy, row panel, update) took 76 us.  Above n = 1900 the tiles bound it: 25 ms at n = 6069 (45 ms before).
+// copy, row panel, update) took 76 us.  From n = 1900 on the tiles bound it: 12.9 ms at n = 6069 (24 ms for all
+// tiles, 49 ms in four launches per panel).
 constexpr int GJB = 64;
 constexpr int GJL = GJB + 2;  // LDS row stride: the 16 rows x 2 entries of a half wave's operand read lie in 64 banks
 typedef double gj_d4 __attribute__((ext_vector_type(4)));
@@ -544,6 +552,10 @@ __global__ void __launch_bounds__(256, 2) gj_first_kernel(long long n, int nb, c
   }
 }
 
+// index of the first tile of row bi among the tiles on and above the diagonal
+__device__ inline int gj_row_start(int bi, int nb) { return bi * nb - bi * (bi - 1) / 2; }
+
+template <bool SYM>
 __global__ void __launch_bounds__(256, 2)
 gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double* __restrict__ P, double* __restrict__ Pn,
                const double* __restrict__ C, double* __restrict__ Cn, const double* __restrict__ R,
@@ -555,10 +567,17 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
   // the next diagonal tile, with the inversion after its update, goes first
   int t = blockIdx.x;
   if (k + 1 < nb) {
-    const int next = (k + 1) * nb + k + 1;
+    const int next = SYM ? gj_row_start(k + 1, nb) : (k + 1) * nb + k + 1;
     t = t == 0 ? next : t == next ? 0 : t;
   }
-  const int bi = t / nb, bj = t % nb;
+  int bi = t / nb, bj = t % nb;
+  if (SYM) {  // the largest row that starts at or before t
+    bi = (int)((2 * nb + 1 - sqrtf((float)((2 * nb + 1) * (2 * nb + 1) - 8 * t))) * 0.5f);
+    bi = max(0, min(bi, nb - 1));
+    while (bi > 0 && gj_row_start(bi, nb) > t) --bi;
+    while (bi + 1 < nb && gj_row_start(bi + 1, nb) <= t) ++bi;
+    bj = bi + t - gj_row_start(bi, nb);
+  }
   const bool row_k = bi == k, col_k = bj == k;
   const long long i0 = (long long)bi * GJB, j0 = (long long)bj * GJB;
   // 64 x 64 tile of a row-major array, zero beyond rows x cols: all 16 loads of a thread in flight at once
@@ -575,8 +594,8 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
     for (int u = 0; u < PER; ++u) dst[(tid + 256 * u) / GJB * GJL + tid % GJB] = d[u];
   };
   gj_d4 acc[2][2];
-  // acc = sA sB, a wave per 32 x 32 quadrant (A: row l16, entry lq; B: entry lq, column l16)
-  auto product = [&]() {
+  // acc = sA sB, a wave per 32 x 32 quadrant (A: row l16, entry lq; B: entry lq, column l16; transposed: sB holds B^T)
+  auto product = [&](auto transposed) {
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -587,7 +606,8 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
 #pragma unroll
       for (int a = 0; a < 2; ++a) x[a] = sA[(wr + 16 * a + l16) * GJL + k4 + lq];
 #pragma unroll
-      for (int b = 0; b < 2; ++b) y[b] = sB[(k4 + lq) * GJL + wc + 16 * b + l16];
+      for (int b = 0; b < 2; ++b)
+        y[b] = transposed ? sB[(wc + 16 * b + l16) * GJL + k4 + lq] : sB[(k4 + lq) * GJL + wc + 16 * b + l16];
 #pragma unroll
       for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -596,7 +616,12 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
   };
   double tp[PER], tr[PER], tc[PER];
   fetch(tp, P, GJB, GJB, GJB);
-  if (!col_k) fetch(tr, R + j0, n, GJB, n - j0);
+  if (!col_k) {
+    if (SYM)
+      fetch(tr, C + j0 * GJB, GJB, n - j0, GJB);
+    else
+      fetch(tr, R + j0, n, GJB, n - j0);
+  }
   // entry r of acc[a][b]: row wr + 16 a + 4 r + lq, column wc + 16 b + l16
   gj_d4 v[2][2];
 #pragma unroll
@@ -613,7 +638,7 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
     put(sA, tp);
     put(sB, tr);
     __syncthreads();
-    product();  // P R_j
+    product(std::integral_constant<bool, SYM>());  // P R_j (SYM: up to the sign)
     __syncthreads();
   }
   if (!row_k) {
@@ -629,11 +654,12 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
           for (int r = 0; r < 4; ++r) sB[(wr + 16 * a + 4 * r + lq) * GJL + wc + 16 * b + l16] = acc[a][b][r];
     }
     __syncthreads();
-    product();
+    product(std::false_type());
+    const double sign = SYM && bj < k ? 1.0 : -1.0;
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) v[a][b] -= acc[a][b];
+      for (int b = 0; b < 2; ++b) v[a][b] += sign * acc[a][b];
   } else {
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -653,8 +679,14 @@ gj_step_kernel(long long n, int nb, int k, double* __restrict__ A, const double*
         const int lr = wr + 16 * a + 4 * r + lq, lc = wc + 16 * b + l16;
         const long long i = i0 + lr, j = j0 + lc;
         if (i < n && j < n) A[i * n + j] = v[a][b][r];
-        if (next_row && j < n) Rn[lr * n + j] = v[a][b][r];
-        if (next_col && i < n) Cn[i * GJB + lc] = v[a][b][r];
+        if (SYM) {
+          if (next_col && i < n) Cn[i * GJB + lc] = v[a][b][r];
+          if (next_row && !next_col && j < n) Cn[j * GJB + lr] = v[a][b][r];
+          if (k + 1 == nb && bi != bj && i < n && j < n) A[j * n + i] = v[a][b][r];
+        } else {
+          if (next_row && j < n) Rn[lr * n + j] = v[a][b][r];
+          if (next_col && i < n) Cn[i * GJB + lc] = v[a][b][r];
+        }
       }
   if (!(next_row && next_col)) return;
   __syncthreads();  // sB was read by the last product
@@ -816,7 +848,17 @@ int launch_dense_from_stencil(const GridDims& g, const double* S, double* A, hip
   return check_launch("dense_from_stencil_kernel");
 }
 
-int gj_invert(long long n, double* A, double* ws, hipStream_t s) {
+bool symmetric_matrix(int m, const double* K0) {
+  double scale = 0.0, skew = 0.0;
+  for (int i = 0; i < m; ++i)
+    for (int j = 0; j < m; ++j) {
+      scale = std::max(scale, std::fabs(K0[i * m + j]));
+      skew = std::max(skew, std::fabs(K0[i * m + j] - K0[j * m + i]));
+    }
+  return skew <= 1e-14 * scale;
+}
+
+int gj_invert(long long n, bool symmetric, double* A, double* ws, hipStream_t s) {
   const int nb = (int)((n + GJB - 1) / GJB);
   double *P[2], *C[2], *R[2];
   for (int h = 0; h < 2; ++h) {  // this panel's and the next one's
@@ -828,7 +870,11 @@ int gj_invert(long long n, double* A, double* ws, hipStream_t s) {
   PMT_TRY(check_launch("gj_first_kernel"));
   for (int k = 0; k < nb; ++k) {
     const int h = k & 1;
-    gj_step_kernel<<<nb * nb, 256, 0, s>>>(n, nb, k, A, P[h], P[1 - h], C[h], C[1 - h], R[h], R[1 - h]);
+    if (symmetric)
+      gj_step_kernel<true><<<nb * (nb + 1) / 2, 256, 0, s>>>(n, nb, k, A, P[h], P[1 - h], C[h], C[1 - h], nullptr,
+                                                             nullptr);
+    else
+      gj_step_kernel<false><<<nb * nb, 256, 0, s>>>(n, nb, k, A, P[h], P[1 - h], C[h], C[1 - h], R[h], R[1 - h]);
     PMT_TRY(check_launch("gj_step_kernel"));
   }
   return PMT_OK;

@@ -177,9 +177,11 @@ int launch_dk_up(const GridDims& gf, const uint8_t* cflag, const int* list, int 
 int launch_stencil_from_moments(const GridDims& g, const double* C, const double* M, const int* map,
                                 const double* dK, const StencilOut& out, hipStream_t s);
 int launch_dense_from_stencil(const GridDims& g, const double* S, double* A, hipStream_t s);
-// A (n x n, SPD) replaced by its inverse; ws: gj_work_size(n) doubles
+// A (n x n, no pivoting; symmetric: half the work) replaced by its inverse; ws: gj_work_size(n) doubles
 inline long long gj_work_size(long long n) { return 2 * 64 * 64 + 4 * 64 * n; }
-int gj_invert(long long n, double* A, double* ws, hipStream_t s);
+int gj_invert(long long n, bool symmetric, double* A, double* ws, hipStream_t s);
+// is the m x m element matrix symmetric to rounding?
+bool symmetric_matrix(int m, const double* K0_host);
 template <typename T>
 int launch_gemv(long long n, const T* A, const T* x, T* y, hipStream_t s, int cols = 1);
 int launch_gemv_f32io(long long n, const double* A, const float* x, float* y, hipStream_t s, int cols = 1);

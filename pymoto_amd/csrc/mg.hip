@@ -535,7 +535,7 @@ static int hex_coarse_stencils(pmt_mg* mg, hipStream_t s) {
   }
   PMT_HIP(hipStreamWaitEvent(mg->s2, mg->ev_fork, 0));
   PMT_TRY(launch_dense_from_stencil(Lc.g, Lc.d.S, mg->Ainv, mg->s2));
-  PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjw, mg->s2));
+  PMT_TRY(gj_invert(mg->nc, mg->sym, mg->Ainv, mg->gjw, mg->s2));
   PMT_HIP(hipEventRecord(mg->ev_join, mg->s2));
   // joined by the first coarsest solve on each stream: the V-cycle descent before it hides the inversion
   mg->pending_join = true;
@@ -571,6 +571,7 @@ int pmt_mg_create(int nelx, int nely, int nelz, int nlevels, const double* omega
   mg->l1free = mg->dim == 3 && nlevels >= 3 && (mg->k0pat & PMT_K0_REFLECTION) &&
                (coarse1 == 2 ? nodes1 > kStoredLevel1Nodes : coarse1 == 1);
   mg->lmax_elem = element_lmax(mg->NE, K0_host);
+  mg->sym = symmetric_matrix(mg->NE, K0_host);
   int ex = nelx, ey = nely, ez = nelz;
   for (int l = 0; l < nlevels; ++l) {
     Level& L = mg->L[l];
@@ -781,7 +782,7 @@ int pmt_mg_update(pmt_mg* mg, const double* xe, const uint8_t* bcmask, double bc
   if (mg->dim != 3) {  // hex8: inverted on the second stream inside hex_coarse_stencils
     Level& Cl = mg->L[mg->nlev - 1];
     PMT_TRY(launch_dense_from_stencil(Cl.g, Cl.d.S, mg->Ainv, s));
-    PMT_TRY(gj_invert(mg->nc, mg->Ainv, mg->gjw, s));
+    PMT_TRY(gj_invert(mg->nc, mg->sym, mg->Ainv, mg->gjw, s));
   }
   if (mg->smoother == 1) {
     for (int l = 0; l < mg->nlev - 1; ++l) {

@@ -117,6 +117,7 @@ struct pmt_mg {
   bool pending_join = false;
   std::vector<hipStream_t> joined;
   double* gjw = nullptr;  // workspace of the coarsest inversion
+  bool sym = false;       // of a symmetric matrix (K0 is)
   float* z32 = nullptr;  // FP32 V-cycle output on the fine grid
   double* p = nullptr;
   double* q = nullptr;

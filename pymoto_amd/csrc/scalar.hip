@@ -530,6 +530,7 @@ struct pmt_smg {
   double* t[kScalarMaxLevels] = {};  // work: iterate, residual
   double* t2[kScalarMaxLevels] = {};
   double* W[2] = {};                 // stencils of the first level coarsened along x, along x and y
+  bool sym = false;                  // P0 is symmetric
   bool elem = false;                 // P0[a][b] depends on a ^ b only: the fine grid is applied from the densities
   double pe[8] = {};                 // then P0[0][a]
   double* parts = nullptr;           // block parts of the dots fused with the fine operator
@@ -764,6 +765,7 @@ int pmt_smg_create(int nelx, int nely, int nelz, int nlevels, const double* omeg
   for (int a = 0; a < NN; ++a)
     for (int b = 0; b < NN; ++b)
       if (!(std::fabs(P0_host[a * NN + b] - P0_host[a ^ b]) <= 1e-14 * big)) h->elem = false;
+  h->sym = symmetric_matrix(NN, P0_host);
   for (int a = 0; a < NN; ++a) h->pe[a] = P0_host[a];
   A(&h->r, n0);
   A(&h->z, n0);
@@ -836,7 +838,7 @@ int pmt_smg_update(pmt_smg* h, const double* xe, const uint8_t* bcmask, double b
   else
     scalar_dense_kernel<2><<<blocks_for(nc, 128), 128, 0, s>>>(h->g[L], h->S[L], h->Ainv);
   PMT_TRY(check_launch("scalar_dense_kernel"));
-  PMT_TRY(gj_invert(nc, h->Ainv, h->gjw, s));
+  PMT_TRY(gj_invert(nc, h->sym, h->Ainv, h->gjw, s));
   h->ready = true;
   return PMT_OK;
 }

@@ -3,7 +3,7 @@ interpolation, coarse operators by Galerkin products, damped Jacobi sweeps, an e
 
 Grids: coarsest systems of 4 to 325 unknowns around the 64 of the blocked inversion's tiles (63, 64, 65, 128, 129), one
 plane to enough planes for each number of planes per thread, ragged blocks; 1 to 3 sweeps; box elements (whose matrix
-depends on the corners' difference only) and a general symmetric element matrix; with and without fixed nodes.
+depends on the corners' difference only), a general symmetric element matrix and one that is not symmetric; with and without fixed nodes.
 
 Tolerance: some hundred FP64 operations per entry, amplified by the coarsest solve (condition below 1e5 here): 1e-10 of
 the result's largest entry."""
@@ -47,13 +47,16 @@ GRIDS = [((2, 2, 0), 2), ((16, 12, 0), 2), ((14, 14, 0), 2), ((24, 8, 0), 2), ((
          ((48, 24, 0), 2), ((40, 24, 0), 3), ((2, 2, 2), 2), ((8, 8, 4), 3), ((12, 8, 16), 2), ((4, 4, 36), 3)]
 
 
-@pytest.mark.parametrize("kind", ["box", "general", "free"])
+@pytest.mark.parametrize("kind", ["box", "general", "free", "nonsymmetric"])
 @pytest.mark.parametrize("nel,levels", GRIDS)
 def test_vcycle_vs_dense(gpu_lib, nel, levels, kind):
     rng = np.random.default_rng(nel[0] + nel[1] + len(kind))
     d = pm.VoxelDomain(*nel)
     nodes = [n + 1 for n in nel]
     E = poisson_element(d)
+    if kind == "nonsymmetric":
+        G = rng.uniform(-0.1, 0.1, E.shape)
+        E = E + G @ G.T + 0.05 * (G - G.T)
     if kind == "general":
         G = rng.uniform(-0.1, 0.1, E.shape)
         E = E + G @ G.T
