@@ -101,6 +101,10 @@ int pmt_oc_step(long long n, const double* x, const double* dg, double xmin, dou
 
 /* Vector kernels.  y = a*x + b*y (x may be NULL: y = b*y). */
 int pmt_axpby(long long n, double a, const double* x, double b, double* y, void* stream);
+/* With alpha = r.b / b.b: r -= alpha b and (y given) y += sign alpha x, without the host seeing alpha (a projection
+ * of the linear dependency aware solver, solvers.py:160-248).  work: pmt_reduce_work_size() doubles. */
+int pmt_lda_project(long long n, const double* b, const double* x, double sign, double* r, double* y, double* work,
+                    void* stream);
 /* *out = x.y, deterministic two-stage reduction; work holds pmt_reduce_work_size() doubles.
  * Replaces numpy einsum('i,i->') of EinSum (generic.py:193-194) and the CG dots (iterative.py:377-394). */
 int pmt_dot(long long n, const double* x, const double* y, double* out, double* work, void* stream);

@@ -33,6 +33,7 @@ _SIGS = {
     "pmt_oc_work_size": (c_int, []),
     "pmt_oc_step": (c_int, [c_ll, c_vp, c_vp] + [c_dbl] * 7 + [c_vp, c_vp, c_vp]),
     "pmt_axpby": (c_int, [c_ll, c_dbl, c_vp, c_dbl, c_vp, c_vp]),
+    "pmt_lda_project": (c_int, [c_ll, c_vp, c_vp, c_dbl, c_vp, c_vp, c_vp, c_vp]),
     "pmt_dot": (c_int, [c_ll, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "pmt_reduce_work_size": (c_int, []),
     "pmt_dot_noalloc": (c_int, [c_int, c_ll, c_vp, c_vp, c_vp, c_vp]),

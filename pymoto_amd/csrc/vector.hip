@@ -469,6 +469,32 @@ cg_xr_update(long long n, double* __restrict__ sc, const double* __restrict__ do
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
+// alpha = r.b / b.b from their partials (dot_stage1's; the sums and bits of dot_stage2): r -= alpha b and, with y,
+// y += sign alpha x
+__global__ void __launch_bounds__(kReduceThreads)
+lda_project_kernel(long long n, const double* __restrict__ partial, const double* __restrict__ b,
+                   const double* __restrict__ x, double sign, double* __restrict__ r, double* __restrict__ y) {
+  double bv[kXrPer], xv[kXrPer], rv[kXrPer], yv[kXrPer], rb[2];
+  const long long base = (long long)blockIdx.x * (256 * kXrPer) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < kXrPer; ++k) {  // in flight during the sums
+    const long long i = base + 256LL * k < n ? base + 256LL * k : n - 1;
+    bv[k] = b[i];
+    rv[k] = r[i];
+    xv[k] = y ? x[i] : 0.0;
+    yv[k] = y ? y[i] : 0.0;
+  }
+  block_parts<2>(partial, kReduceBlocks, rb);
+  const double alpha = rb[0] / rb[1], ya = sign * alpha;
+#pragma unroll
+  for (int k = 0; k < kXrPer; ++k) {
+    const long long i = base + 256LL * k;
+    if (i >= n) return;
+    r[i] = fma(-alpha, bv[k], rv[k]);
+    if (y) y[i] = fma(ya, xv[k], yv[k]);
+  }
+}
+
 // partials of a0.b0 (entry 0..) and a1.b1 (entry np..), blocks as dot_flat
 __global__ void __launch_bounds__(kReduceThreads)
 dot2_flat(long long n, const double* __restrict__ a0, const double* __restrict__ b0, const double* __restrict__ a1,
@@ -924,6 +950,17 @@ int pmt_oc_update(long long n, const double* x, const double* dg, double xmin, d
 int pmt_axpby(long long n, double a, const double* x, double b, double* y, void* stream) {
   if (n < 0 || (n > 0 && !y)) return arg_error("pmt_axpby: bad argument");
   return launch_axpby(n, a, x, b, y, (hipStream_t)stream);
+}
+
+int pmt_lda_project(long long n, const double* b, const double* x, double sign, double* r, double* y, double* work,
+                    void* stream) {
+  if (n < 0 || !work || (n > 0 && (!b || !r || (y && !x)))) return arg_error("pmt_lda_project: bad argument");
+  if (n == 0) return PMT_OK;
+  hipStream_t s = (hipStream_t)stream;
+  dot_stage1<2><<<kReduceBlocks, kReduceThreads, 0, s>>>(n, r, b, b, b, work);
+  PMT_TRY(check_launch("dot_stage1<2>"));
+  lda_project_kernel<<<(unsigned)cg_xr_parts(n), kReduceThreads, 0, s>>>(n, work, b, x, sign, r, y);
+  return check_launch("lda_project_kernel");
 }
 
 int pmt_dot(long long n, const double* x, const double* y, double* out, double* work, void* stream) {

@@ -61,9 +61,12 @@ def _dots(pairs):
     return out.cpu().numpy()
 
 
-def _axpy(a, x, y):
-    """y += a x (in place)"""
-    _lib.check(_lib.lib().pmt_axpby(y.numel(), float(a), _lib.ptr(x), 1.0, _lib.ptr(y), _lib.stream()), "axpby")
+def _project(b, r, x=None, y=None, sign=1.0):
+    """r -= a b and y += sign a x with a = (r . b) / (b . b), in place (a stays on the device)"""
+    lib = _lib.lib()
+    work = torch.empty(lib.pmt_reduce_work_size(), dtype=torch.float64, device=r.device)
+    _lib.check(lib.pmt_lda_project(r.numel(), _lib.ptr(b), _lib.ptr(x), float(sign), _lib.ptr(r), _lib.ptr(y),
+                                   _lib.ptr(work), _lib.stream()), "lda projection")
 
 
 def _scale(a, y):
@@ -108,9 +111,7 @@ class LDAWrapper(LinearSolver):
         for rhs in cols:
             rl, sol = self._split(rhs)
             for x, b in zip(self.x_stored, self.b_stored):
-                alpha = _dot(rl, b) / _dot(b, b)
-                _axpy(-alpha, b, rl)
-                _axpy(alpha, x, sol)
+                _project(b, rl, x, sol)
             if self.x_stored or not isinstance(A, StiffnessMatrix):
                 r = A.residual(rhs, sol)
             else:
@@ -132,7 +133,7 @@ class LDAWrapper(LinearSolver):
                 for k in todo:
                     v, _ = self._split(_lib.as_device(x0s[k]))  # new tensors: x0 is not modified
                     for x in self.x_stored:
-                        _axpy(-_dot(v, x) / _dot(x, x), x, v)
+                        _project(x, v)
                     x0l.append(v)
             solve1 = getattr(self.solver, "_solve_1rhs", None)  # the device CG
             if len(todo) == 1 and x0l is not None and solve1 is not None:
@@ -152,9 +153,7 @@ class LDAWrapper(LinearSolver):
                 xadd, _ = self._split(xnew)
                 badd, _ = self._split(A @ xnew)
                 for x, b in zip(self.x_stored, self.b_stored):
-                    beta = _dot(badd, b) / _dot(b, b)
-                    _axpy(-beta, b, badd)
-                    _axpy(-beta, x, xadd)
+                    _project(b, badd, x, xadd, -1.0)
                 bnrm = np.sqrt(_dot(badd, badd))
                 if np.isfinite(bnrm) and bnrm > 0:
                     _scale(1.0 / bnrm, badd)
