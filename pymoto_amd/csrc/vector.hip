@@ -191,21 +191,24 @@ __global__ void oc_update_kernel(long long n, const double* __restrict__ x, cons
 
 // The whole OC bisection on the device (pmt_oc_step).  A pass evaluates the 2^kOcLv - 1 multipliers that the next
 // kOcLv bisection steps can ask for (the nodes of the bisection tree under [l1, l2]) in one sweep over x and
-// dg; oc_choose_kernel sums the partials, walks the kOcLv decisions and leaves the new interval in the state, so
-// the host reads nothing between the steps.  Every sum is formed as oc_update_kernel and dot_stage2 form it
+// dg; the next pass starts with summing the partials and walking the kOcLv decisions (every block for itself,
+// block 0 leaves the new interval in the other of two states), so the host reads nothing between the steps and
+// nothing is launched between the passes.  Every sum is formed as oc_update_kernel and dot_stage2 form it
 // (the same blocks, strides and tree), so the decisions and the design are those of the step-by-step
 // bisection, bit for bit.
 // x sqrt(s / l) falls with l: above s (x / lb)^2 the entry is lb, below s (x / ub)^2 it is ub; outside a
 // 1e-12 margin of the two (the computed value is good to 4e-16) the root is not evaluated.
-// 30 steps of 524,288 elements: 166 us (734 us with a launch pair and a host read per step), 106 us for 2,000.
-// More steps per pass save launches, but every multiplier costs every element a root: 4 steps took 193 and
-// 109 us, 5 took 255 and 127.  (Letting the pass's last block choose, behind a ticket, saves the second launch
+// 30 steps of 524,288 elements: 152 us (163 us with a launch for the decisions after each pass, 734 us with a launch
+// pair and a host read per step).  More steps per pass save launches, but every multiplier costs every element a
+// root: 4 steps took 193 instead of 166 us, 5 took 255.  (Letting the pass's last block choose, behind a ticket, saves the second launch
 // but costs every block a release fence: 27 instead of 8.8 us per pass.)
 struct OcState {
   double l1, l2, last, maxdg;  // last: the multiplier of the last step
 };
 constexpr int kOcLv = 3, kOcNodes = (1 << kOcLv) - 1;
-constexpr int kOcState = 8;  // doubles that hold the state
+constexpr int kOcState = 8;    // doubles that hold a state
+constexpr int kOcThreads = 1024;  // of a pass: kOcGroups blocks of oc_update_kernel in one, so that few blocks sum
+constexpr int kOcGroups = kOcThreads / kReduceThreads;
 
 __global__ void oc_init_kernel(double l1, double l2, OcState* st) { *st = OcState{l1, l2, 0.0, 0.0}; }
 
@@ -221,22 +224,92 @@ __device__ inline double oc_node(int h, double a, double b) {
   return 0.5 * (a + b);
 }
 
-__global__ void __launch_bounds__(kReduceThreads)
-oc_pass_kernel(long long n, const double* __restrict__ x, const double* __restrict__ dg, double xmin, double xmax,
-               double move, double tol, int first, const OcState* __restrict__ st, double* __restrict__ partial) {
+// the decisions of a pass (prev: its state before, partial: its sums) by a block of kOcThreads, into `out` of every
+// thread: a wave per sum, in dot_stage2's order (4 waves of strided sums, their trees, then wave after wave); nb
+// blocks wrote partials, the others have no entries
+__device__ inline void oc_choose(int nb, double tol, double target, int first, const OcState* __restrict__ prev,
+                                 const double* __restrict__ partial, OcState& out) {
+  constexpr int M = kOcNodes, NW = kReduceThreads / 64, NK = kReduceBlocks / kReduceThreads;
+  static_assert(M < kOcThreads / 64, "a wave per sum");
+  __shared__ double sums[M + 1];
+  out = *prev;
+  if (!(out.l2 - out.l1 > tol) && !first) return;
+  const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
+  if (c < M) {
+    double p[NW][NK];
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const int b = w * 64 + lane + k * kReduceThreads;
+        p[w][k] = b < nb ? partial[c * kReduceBlocks + b] : 0.0;
+      }
+    double r = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      double t = 0.0;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) t += p[w][k];
+      for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+      r += t;
+    }
+    if (lane == 0) sums[c] = r;
+  }
+  if (first && c == M) {
+    double m = -INFINITY;
+    for (int b = lane; b < nb; b += 64) {
+      const double o = partial[M * kReduceBlocks + b];
+      m = (o > m || o != o) ? o : m;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      const double o = __shfl_down(m, off, 64);
+      m = (o > m || o != o) ? o : m;
+    }
+    if (lane == 0) sums[M] = m;
+  }
+  __syncthreads();
+  int h = 1;
+  for (int step = 0; step < kOcLv && out.l2 - out.l1 > tol; ++step) {
+    out.last = 0.5 * (out.l1 + out.l2);
+    if (sums[h - 1] - target > 0.0) {
+      out.l1 = out.last;
+      h = 2 * h + 1;
+    } else {
+      out.l2 = out.last;
+      h = 2 * h;
+    }
+  }
+  if (first) out.maxdg = sums[M];
+}
+
+// pass p: the decisions of pass p - 1 (p > 0; states and partials alternate between two sets), then the sums of its
+// own multipliers.  A group of 256 threads forms one block's partials of oc_update_kernel.
+__global__ void __launch_bounds__(kOcThreads)
+oc_pass_kernel(long long n, int nb, const double* __restrict__ x, const double* __restrict__ dg, double xmin,
+               double xmax, double move, double tol, double target, int pass, const OcState* __restrict__ prev,
+               const double* __restrict__ pin, OcState* __restrict__ st, double* __restrict__ partial) {
   constexpr int M = kOcNodes;
-  __shared__ double lm[M], wsum[kReduceThreads / 64][M];
-  __shared__ double red[kReduceThreads / 64];
-  const double l1 = st->l1, l2 = st->l2;
-  if (!(l2 - l1 > tol) && !first) return;
+  __shared__ double lm[M], wsum[kOcThreads / 64][M];
+  __shared__ double red[kOcThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool first = pass == 0;
+  OcState now;
+  if (first) {
+    now = *prev;
+  } else {
+    oc_choose(nb, tol, target, pass == 1, prev, pin, now);
+    if (blockIdx.x == 0 && tid == 0) *st = now;
+  }
+  const double l1 = now.l1, l2 = now.l2;
+  if (!(l2 - l1 > tol) && !first) return;
   if (tid < M) lm[tid] = oc_node(tid + 1, l1, l2);
   __syncthreads();
+  const int group = tid / kReduceThreads, block = (int)blockIdx.x * kOcGroups + group, gt = tid % kReduceThreads;
   double s[M];
 #pragma unroll
   for (int c = 0; c < M; ++c) s[c] = 0.0;
   double mx = -INFINITY;
-  for (long long i = (long long)blockIdx.x * blockDim.x + tid; i < n; i += (long long)kReduceBlocks * blockDim.x) {
+  for (long long i = (long long)block * kReduceThreads + gt; i < n; i += (long long)kReduceBlocks * kReduceThreads) {
     const double xi = x[i], di = dg[i];
     const double lb = fmax(xmin, xi - move), ub = fmin(xmax, xi + move), g = -fmin(di, 0.0);
     mx = (di > mx || di != di) ? di : mx;
@@ -260,84 +333,36 @@ oc_pass_kernel(long long n, const double* __restrict__ x, const double* __restri
 #pragma unroll
     for (int c = 0; c < M; ++c) wsum[wave][c] = s[c];
   }
+  if (first) {
+    for (int off = 32; off > 0; off >>= 1) {
+      const double o = __shfl_down(mx, off, 64);
+      mx = (o > mx || o != o) ? o : mx;
+    }
+    if (lane == 0) red[wave] = mx;
+  }
   __syncthreads();
-  if (tid < M) {
+  if (block >= nb) return;
+  const int w0 = group * (kReduceThreads / 64);
+  if (gt < M) {
     double r = 0.0;
-    for (int w = 0; w < kReduceThreads / 64; ++w) r += wsum[w][tid];
-    partial[tid * kReduceBlocks + blockIdx.x] = r;
+    for (int w = 0; w < kReduceThreads / 64; ++w) r += wsum[w0 + w][gt];
+    partial[gt * kReduceBlocks + block] = r;
   }
-  if (!first) return;
-  for (int off = 32; off > 0; off >>= 1) {
-    const double o = __shfl_down(mx, off, 64);
-    mx = (o > mx || o != o) ? o : mx;
-  }
-  if (lane == 0) red[wave] = mx;
-  __syncthreads();
-  if (tid == 0) {
-    for (int w = 1; w < kReduceThreads / 64; ++w) mx = (red[w] > mx || red[w] != red[w]) ? red[w] : mx;
-    partial[M * kReduceBlocks + blockIdx.x] = mx;
+  if (first && gt == M) {
+    double m = red[w0];
+    for (int w = 1; w < kReduceThreads / 64; ++w) m = (red[w0 + w] > m || red[w0 + w] != red[w0 + w]) ? red[w0 + w] : m;
+    partial[M * kReduceBlocks + block] = m;
   }
 }
 
-// the decisions of a pass: a wave per sum, in dot_stage2's order (4 waves of strided sums, their trees, then
-// wave after wave); nb blocks wrote partials, the others have no entries
-__global__ void __launch_bounds__(1024)
-oc_choose_kernel(int nb, double tol, double target, int first, OcState* st, const double* __restrict__ partial) {
-  constexpr int M = kOcNodes, NW = kReduceThreads / 64, NK = kReduceBlocks / kReduceThreads;
-  __shared__ double sums[M + 1];
-  const double l1 = st->l1, l2 = st->l2;
-  if (!(l2 - l1 > tol) && !first) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int c = wave; c < M; c += 16) {
-    double p[NW][NK];
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-#pragma unroll
-      for (int k = 0; k < NK; ++k) {
-        const int b = w * 64 + lane + k * kReduceThreads;
-        p[w][k] = b < nb ? partial[c * kReduceBlocks + b] : 0.0;
-      }
-    double r = 0.0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      double t = 0.0;
-#pragma unroll
-      for (int k = 0; k < NK; ++k) t += p[w][k];
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
-      r += t;
-    }
-    if (lane == 0) sums[c] = r;
-  }
-  if (first && wave == 15) {
-    double m = -INFINITY;
-    for (int b = lane; b < nb; b += 64) {
-      const double o = partial[M * kReduceBlocks + b];
-      m = (o > m || o != o) ? o : m;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      const double o = __shfl_down(m, off, 64);
-      m = (o > m || o != o) ? o : m;
-    }
-    if (lane == 0) sums[M] = m;
-  }
+// the decisions of the last pass
+__global__ void __launch_bounds__(kOcThreads)
+oc_last_kernel(int nb, double tol, double target, int first, const OcState* __restrict__ prev,
+               const double* __restrict__ partial, OcState* st) {
+  OcState now;
+  oc_choose(nb, tol, target, first, prev, partial, now);
   __syncthreads();
-  if (threadIdx.x) return;
-  double a = l1, b = l2, last = st->last;
-  int h = 1;
-  for (int step = 0; step < kOcLv && b - a > tol; ++step) {
-    last = 0.5 * (a + b);
-    if (sums[h - 1] - target > 0.0) {
-      a = last;
-      h = 2 * h + 1;
-    } else {
-      b = last;
-      h = 2 * h;
-    }
-  }
-  st->l1 = a;
-  st->l2 = b;
-  st->last = last;
-  if (first) st->maxdg = sums[M];
+  if (threadIdx.x == 0) *st = now;
 }
 
 // the design of the last step's multiplier
@@ -911,28 +936,31 @@ int pmt_heaviside_bwd(long long n, double beta, double eta, const double* x, con
   return check_launch("heaviside_bwd_kernel");
 }
 
-int pmt_oc_work_size(void) { return kOcState + (kOcNodes + 1) * kReduceBlocks; }
+int pmt_oc_work_size(void) { return 2 * kOcState + 2 * (kOcNodes + 1) * kReduceBlocks; }
 
 int pmt_oc_step(long long n, const double* x, const double* dg, double xmin, double xmax, double move, double l1,
                 double l2, double tol, double target, double* xnew, double* work, void* stream) {
   if (n <= 0 || !x || !dg || !xnew || !work) return arg_error("pmt_oc_step: bad argument");
   hipStream_t s = (hipStream_t)stream;
-  OcState* st = (OcState*)work;
-  double* partial = work + kOcState;
+  OcState* st[2] = {(OcState*)work, (OcState*)(work + kOcState)};
+  double* partial[2] = {work + 2 * kOcState, work + 2 * kOcState + (kOcNodes + 1) * kReduceBlocks};
   static_assert(sizeof(OcState) <= kOcState * sizeof(double), "OC state");
-  oc_init_kernel<<<1, 1, 0, s>>>(l1, l2, st);
+  oc_init_kernel<<<1, 1, 0, s>>>(l1, l2, st[0]);
   PMT_TRY(check_launch("oc_init_kernel"));
   int steps = 0;
   for (double w = l2 - l1; w > tol && steps < 1100; w *= 0.5) ++steps;
-  const unsigned blocks = (unsigned)std::min<long long>(kReduceBlocks, (n + kReduceThreads - 1) / kReduceThreads);
+  const int nb = (int)std::min<long long>(kReduceBlocks, (n + kReduceThreads - 1) / kReduceThreads);
   const int passes = std::max(1, (steps + 1 + kOcLv - 1) / kOcLv);  // one step to spare for the rounding of the halvings
-  for (int p = 0; p < passes; ++p) {
-    oc_pass_kernel<<<blocks, kReduceThreads, 0, s>>>(n, x, dg, xmin, xmax, move, tol, p == 0, st, partial);
+  for (int p = 0; p < passes; ++p) {  // pass p leaves its state in st[p % 2] (pass 0: finds it there)
+    oc_pass_kernel<<<(nb + kOcGroups - 1) / kOcGroups, kOcThreads, 0, s>>>(
+        n, nb, x, dg, xmin, xmax, move, tol, target, p, st[p > 0 ? (p - 1) % 2 : 0], partial[(p + 1) % 2], st[p % 2],
+        partial[p % 2]);
     PMT_TRY(check_launch("oc_pass_kernel"));
-    oc_choose_kernel<<<1, 1024, 0, s>>>((int)blocks, tol, target, p == 0, st, partial);
-    PMT_TRY(check_launch("oc_choose_kernel"));
   }
-  oc_write_kernel<<<blocks_for(n, 256), 256, 0, s>>>(n, x, dg, xmin, xmax, move, st, xnew);
+  oc_last_kernel<<<1, kOcThreads, 0, s>>>(nb, tol, target, passes == 1, st[(passes - 1) % 2], partial[(passes - 1) % 2],
+                                          st[0]);
+  PMT_TRY(check_launch("oc_last_kernel"));
+  oc_write_kernel<<<blocks_for(n, 256), 256, 0, s>>>(n, x, dg, xmin, xmax, move, st[0], xnew);
   return check_launch("oc_write_kernel");
 }
 
