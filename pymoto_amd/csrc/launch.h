@@ -68,6 +68,10 @@ int launch_fine_apply_dots(const GridDims& g, const double* K0ext, int k0_patter
                            const uint8_t* bcm, double bcdiag, const double* p, const double* r, double* q,
                            double* ws, long long ws_parts, double* out, hipStream_t s, int* parts = nullptr);
 long long fine_apply_dots_parts(const GridDims& g);  // a sufficient ws_parts for the grid
+// Q4: q = A p with the q4_apply_dots_parts(g) partials of p.q and, behind them, of p.r in ws
+long long q4_apply_dots_parts(const GridDims& g);
+int launch_q4_apply_dots(const GridDims& g, const double* K0, int k0_pattern, const double* xe, const uint8_t* bcm,
+                         double bcdiag, const double* p, const double* r, double* q, double* ws, hipStream_t s);
 // refl.hip: dx = alpha u_e^T K0 v_e (accumulate: dx += ...) in the reflection basis over z-streamed node
 // columns; tab = the FP64 block entries behind K0; hex8 only
 int launch_sens_stream(const GridDims& g, const double* tab, const uint8_t* bcm, const double* u, const double* v,

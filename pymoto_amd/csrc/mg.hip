@@ -672,6 +672,10 @@ int pmt_mg_create(int nelx, int nely, int nelz, int nlevels, const double* omega
     mg->dotws_parts = fine_apply_dots_parts(mg->L[0].g);
     ALLOC(mg->dotws, 2 * mg->dotws_parts);
   }
+  if (!hex && cg_sums_inline(q4_apply_dots_parts(mg->L[0].g))) {
+    mg->dotws_parts = q4_apply_dots_parts(mg->L[0].g);
+    ALLOC(mg->dotws, 2 * mg->dotws_parts);
+  }
 #undef ALLOC
   if (rc == PMT_OK)
     rc = hip_status(hipHostMalloc((void**)&mg->host_rr, 2 * sizeof(double), hipHostMallocCoherent), "hipHostMalloc");
@@ -896,10 +900,14 @@ int pmt_pcg_solve(pmt_mg* mg, const double* b, double* x, int x0_is_zero, double
     const bool restart_now = i % restart == 0;
     const double* dots = nullptr;
     int np = 0;
-    const int frc = mg->dotws ? launch_fine_apply_dots(F.g, mg->K0, mg->k0pat, mg->xe, mg->bcm, mg->bcdiag, mg->p,
-                                                       mg->r, mg->q, mg->dotws, mg->dotws_parts, sc, s,
-                                                       restart_now ? nullptr : &np)
-                              : PMT_ERR_STATE;
+    int frc = PMT_ERR_STATE;
+    if (mg->dotws && mg->dim == 3) {
+      frc = launch_fine_apply_dots(F.g, mg->K0, mg->k0pat, mg->xe, mg->bcm, mg->bcdiag, mg->p, mg->r, mg->q, mg->dotws,
+                                   mg->dotws_parts, sc, s, restart_now ? nullptr : &np);
+    } else if (mg->dotws && !restart_now) {  // Q4: as long as the r update can add the partials
+      frc = launch_q4_apply_dots(F.g, mg->K0, mg->k0pat, mg->xe, mg->bcm, mg->bcdiag, mg->p, mg->r, mg->q, mg->dotws, s);
+      np = (int)mg->dotws_parts;
+    }
     if (frc == PMT_ERR_STATE) {
       PMT_TRY(level_apply<double>(mg, 0, MODE_APPLY, mg->p, nullptr, mg->q, s));
       if (!restart_now && cg_sums_inline(cg_xr_parts(n))) {

@@ -64,12 +64,15 @@ struct Tile<2> {
 // a one-node halo (structure of arrays, zero outside the grid) and the densities of the elements
 // touching the tile (zero outside the grid) in LDS; every thread then gathers its node's rows from
 // LDS with no bounds checks, so the 2^D*D*2^D*D multiply-adds run branch-free.
+// MODE_APPLY_DOTS: y = A u, and the tile's sums of u.y and u.r (b holds r) to partial[tile] and
+// partial[ntiles + tile]: 4.8 us at 120x40 (the product 4.2 and a pass for the dots 3.9), 50 instead of 53 us per
+// CG iteration.
 template <int DIM, int MODE, bool CLS, typename T>
 __global__ void __launch_bounds__(256)
 fine_node_kernel(GridDims g, int tiles_x, int tiles_y, int ntiles, const double* __restrict__ K0,
                  const T* __restrict__ xe, const uint8_t* __restrict__ bcm, T bcdiag,
                  const T* __restrict__ u, const T* __restrict__ b, const T* __restrict__ dinv,
-                 T omega, T* y, const T* up, T beta) {
+                 T omega, T* y, const T* up, T beta, double* __restrict__ partial = nullptr) {
   constexpr int NN = Cfg<DIM>::NN;
   constexpr int NE = Cfg<DIM>::NE;
   constexpr int TX = Tile<DIM>::X, TY = Tile<DIM>::Y, TZ = Tile<DIM>::Z;
@@ -122,7 +125,8 @@ fine_node_kernel(GridDims g, int tiles_x, int tiles_y, int ntiles, const double*
 
   const int lx = threadIdx.x % TX, ly = (threadIdx.x / TX) % TY, lz = threadIdx.x / (TX * TY);
   const int i = tx0 + lx, j = ty0 + ly, k = tz0 + lz;
-  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
+  const bool in = i < g.nx && j < g.ny && k < g.nz;
+  if (MODE != MODE_APPLY_DOTS && !in) return;  // (the sums need every thread; its LDS reads stay in the tile's halo)
 
   T acc[NN][DIM];
 #pragma unroll
@@ -178,6 +182,31 @@ fine_node_kernel(GridDims g, int tiles_x, int tiles_y, int ntiles, const double*
   }
 
   const long long n = ((long long)k * g.ny + j) * g.nx + i;
+  if constexpr (MODE == MODE_APPLY_DOTS) {
+    double s[2] = {0.0, 0.0};
+    if (in) {
+      const unsigned mk = bcm[n];
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) {
+        const long long q = n * DIM + d;
+        const T uq = u[q], ku = ((mk >> d) & 1u) ? bcdiag * uq : out[d];
+        y[q] = ku;
+        s[0] = fma((double)uq, (double)ku, s[0]);
+        s[1] = fma((double)uq, (double)b[q], s[1]);
+      }
+    }
+    __shared__ double red[2][4];
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      for (int off = 32; off > 0; off >>= 1) s[o] += __shfl_down(s[o], off, 64);
+      if ((threadIdx.x & 63) == 0) red[o][threadIdx.x >> 6] = s[o];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+      partial[threadIdx.x * ntiles + tile] =
+          ((red[threadIdx.x][0] + red[threadIdx.x][1]) + red[threadIdx.x][2]) + red[threadIdx.x][3];
+    return;
+  }
   const unsigned mk = bcm[n];
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
@@ -1025,6 +1054,25 @@ int launch_fine(int mode, const GridDims& g, const double* K0, int k0_pattern, c
       launch_fine_t<2, false, T>(mode, g, K0, xe, bcm, bd, u, b, dinv, om, y, s, up, be);
   }
   return check_launch("fine_node_kernel");
+}
+
+static long long q4_tiles(const GridDims& g) {
+  return (long long)((g.nx + Tile<2>::X - 1) / Tile<2>::X) * ((g.ny + Tile<2>::Y - 1) / Tile<2>::Y);
+}
+
+long long q4_apply_dots_parts(const GridDims& g) { return g.dim == 2 ? q4_tiles(g) : 0; }
+
+int launch_q4_apply_dots(const GridDims& g, const double* K0, int k0_pattern, const double* xe, const uint8_t* bcm,
+                         double bcdiag, const double* p, const double* r, double* q, double* ws, hipStream_t s) {
+  const int tx = (g.nx + Tile<2>::X - 1) / Tile<2>::X, ty = (g.ny + Tile<2>::Y - 1) / Tile<2>::Y, nt = tx * ty;
+  const unsigned grid = (unsigned)((nt + 7) & ~7);
+  if (k0_pattern & PMT_K0_CLASS_PATTERN)
+    fine_node_kernel<2, MODE_APPLY_DOTS, true, double><<<grid, 256, 0, s>>>(g, tx, ty, nt, K0, xe, bcm, bcdiag, p, r,
+                                                                           nullptr, 0.0, q, nullptr, 0.0, ws);
+  else
+    fine_node_kernel<2, MODE_APPLY_DOTS, false, double><<<grid, 256, 0, s>>>(g, tx, ty, nt, K0, xe, bcm, bcdiag, p, r,
+                                                                            nullptr, 0.0, q, nullptr, 0.0, ws);
+  return check_launch("fine_node_kernel<apply + dots>");
 }
 
 // Does a host element matrix follow the isotropic box pattern (so the SGPR kernel applies)?
