@@ -274,15 +274,22 @@ filter_bwd_fold_kernel(int nx, int ny, int nz, int kxy, int kz, const int32_t* _
   const int32_t* py = inv_ptr + (nx + 1) + j;
   const int32_t* pz = inv_ptr + (nx + 1) + (ny + 1) + k;
   const int pa = px[0], pb = py[0], pc = pz[0];
-  const int na = px[1] - pa, nb = py[1] - pb, cells = na * nb * (pz[1] - pc);
+  const int na = px[1] - pa, nb = py[1] - pb, nc = pz[1] - pc, cells = na * nb * nc;
   const long long lx = nx + kxy - 1, ly = ny + kxy - 1;
   double acc = 0.0;
+  // counted up instead of divided out of t: 75x51x33 with 7^3 8.9 us (two divisions per cell: 13.5), 256x128x128 with
+  // 3^3 5.8 (7.2)
+  int a = 0, b = 0, c = 0;
   for (int t = 0; t < cells; t += 8) {
     double v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int q = min(t + u, cells - 1), r = q / na, c = r / nb;
-      v[u] = g[(inv_idx[pc + c] * ly + inv_idx[pb + r - c * nb]) * lx + inv_idx[pa + q - r * na]];
+      v[u] = g[(inv_idx[pc + min(c, nc - 1)] * ly + inv_idx[pb + b]) * lx + inv_idx[pa + a]];
+      ++a;
+      b += a == na;
+      a = a == na ? 0 : a;
+      c += b == nb;
+      b = b == nb ? 0 : b;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc = t + u < cells ? acc + v[u] : acc;
