@@ -319,8 +319,8 @@ int g_filter_tiled = 1;  // PMT_TUNE_FILTER: 1 boxes in LDS (default), 0 per-ele
 // through the maps.  Adjoint: outputs are the padded cells, the box holds dy (zero outside the grid); the
 // cell of an element without other cells is its result, every other one goes to the workspace g (if given)
 // for filter_bwd_fold_kernel.
-// Forward / adjoint with its fold: 21.9 / 35.2 us at 256x128x128 with 3^3, 13.1 / 21.3 us at 130x70x60 with 5^3,
-// 13.6 / 17.6 us at 75x51x33 with 7^3.  A ring of LDS planes streamed in z took 26.3 / 47.6 and 62.9 / 151 us
+// Forward / adjoint with its fold: 22.9 / 34.2 us at 256x128x128 with 3^3, 14.8 / 23.3 us at 75x51x33 with 7^3 (with a
+// branch around each load of the box 23.2 / 35.3 and 15.2 / 24.1).  A ring of LDS planes streamed in z took 26.3 / 47.6 and 62.9 / 151 us
 // (5^3 held 450 registers, one wave per SIMD), the per-element gathers 69 / 165 us for 7^3 (which the adjoint
 // without a workspace still takes).
 template <int KXY, int OY, bool FWD>
@@ -367,25 +367,26 @@ filter_box_kernel(int nx, int ny, int nz, int kz, int nty, int tiles_x, int tile
     sx[t] = v;
   }
   __syncthreads();
-  // 8 values per thread and step: their loads are in flight together
+  // 8 values per thread and step: their loads are in flight together, without a branch around any (a cell outside
+  // everything reads in[0])
   for (int q0 = tid; q0 < nbox; q0 += 256 * 8) {
     double v[8];
+    unsigned keep = 0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int q = q0 + 256 * u;
+      const int q = min(q0 + 256 * u, nbox - 1);
       const int a = q % LX, t = q / LX, c = (int)(((unsigned)t * m_ly) >> 20), b = t - c * ly;
-      v[u] = 0.0;
-      if (q < nbox) {
-        const int ma = sx[a], mb = sy[b], mc = sz[c];
-        if (ma >= 0 && mb >= 0 && mc >= 0)
-          v[u] = in[(mc * ny + mb) * nx + ma];
-        else if (FWD && ma != -2 && mb != -2 && mc != -2)
-          v[u] = cval[mc < 0 ? plx + ply + k0 + c : mb < 0 ? plx + j0 + b : i0 + a];
-      }
+      const int ma = sx[a], mb = sy[b], mc = sz[c];
+      const bool inside = (ma | mb | mc) >= 0, fixed = FWD && !inside && ma != -2 && mb != -2 && mc != -2;
+      const double* src = fixed ? cval : in;
+      const int at = inside ? (mc * ny + mb) * nx + ma
+                            : fixed ? (mc < 0 ? plx + ply + k0 + c : mb < 0 ? plx + j0 + b : i0 + a) : 0;
+      v[u] = src[at];
+      keep |= (inside || fixed ? 1u : 0u) << u;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (q0 + 256 * u < nbox) box[q0 + 256 * u] = v[u];
+      if (q0 + 256 * u < nbox) box[q0 + 256 * u] = (keep >> u) & 1u ? v[u] : 0.0;
   }
   __syncthreads();
   double acc[OY];
