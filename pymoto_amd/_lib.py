@@ -134,7 +134,8 @@ def load(path: str = _LIBPATH):
 
 def lib():
     """The library, after checking that a GPU is visible (device modules call this)."""
-    if not torch.cuda.is_available():
+    # (an initialised torch.cuda has found one; is_available() reads the environment: 0.6 instead of 0.1 us)
+    if not (torch.cuda.is_initialized() or torch.cuda.is_available()):
         raise HIPError("pymoto_amd needs a ROCm GPU (gfx950); none is visible and there is no CPU fallback")
     return load()
 
@@ -151,6 +152,9 @@ def check(rc: int, what: str = ""):
 
 
 def stream():
+    """The current stream's handle (0.4 us; 2.8 us with a torch Stream object built around it)."""
+    if torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
