@@ -221,17 +221,18 @@ update_kernel(long long n, int k, VecSet P, VecSet Q, const double* __restrict__
 // alpha = (P^T Q)^-1 P^T R from the partial sums of both products (entries 0.. and K * K..), one block.  The
 // inverse of the active principal submatrix by Gauss-Jordan with row pivoting, a thread per entry of the
 // K x 2K tableau; an inactive (dropped) column has zero products and stands as a unit row and column, which
-// leaves the arithmetic of the others unchanged.  Its rows and columns of the inverse are zero.
+// leaves the arithmetic of the others unchanged.  Its rows and columns of the inverse are zero.  The columns from
+// k to K are never active: ACTIVE is written for the k columns of a solve only and may hold an earlier, wider one's.
 template <int K>
-__global__ void __launch_bounds__(1024) bcg_alpha_kernel(const double* __restrict__ partial, int nb, double* sm) {
+__global__ void __launch_bounds__(1024) bcg_alpha_kernel(int k, const double* __restrict__ partial, int nb, double* sm) {
   __shared__ double S[2 * K * K];
   __shared__ double a[K][2 * K];
   __shared__ double inv[K][K];
   const int tid = threadIdx.x, r = tid / (2 * K), c = tid % (2 * K);
   const bool own = r < K;
-  const double* act = sm + Small::ACTIVE;
+  auto active = [&](int j) { return j < k && sm[Small::ACTIVE + j] != 0.0; };
   sum_entries<2 * K * K, 1024>(partial, nb, S);
-  if (own) a[r][c] = c >= K ? (c - K == r ? 1.0 : 0.0) : act[r] != 0.0 && act[c] != 0.0 ? S[r * K + c] : r == c ? 1.0 : 0.0;
+  if (own) a[r][c] = c >= K ? (c - K == r ? 1.0 : 0.0) : active(r) && active(c) ? S[r * K + c] : r == c ? 1.0 : 0.0;
   __syncthreads();
   for (int d = 0; d < K; ++d) {
     double v = 0.0;
@@ -248,7 +249,7 @@ __global__ void __launch_bounds__(1024) bcg_alpha_kernel(const double* __restric
     if (own) a[r][c] = v;
     __syncthreads();
   }
-  if (own && c < K) inv[r][c] = act[r] != 0.0 && act[c] != 0.0 ? a[r][K + c] : 0.0;
+  if (own && c < K) inv[r][c] = active(r) && active(c) ? a[r][K + c] : 0.0;
   __syncthreads();
   if (tid < kMaxRhs * kMaxRhs) {
     const int i = tid / kMaxRhs, j = tid % kMaxRhs;
@@ -539,7 +540,7 @@ static int iter_part1(pmt_mg* mg, BlockCG* w, int k, bool restart_now, hipStream
       gram_kernel<K, 1, double><<<nb, 256, 0, s>>>(n, p, q, q, w->partial);
       gram_kernel<K, 1, double><<<nb, 256, 0, s>>>(n, p, r, r, w->partial + (long long)K * K * nb);
     }
-    bcg_alpha_kernel<K><<<1, 1024, 0, s>>>(w->partial, (int)nb, w->sm);
+    bcg_alpha_kernel<K><<<1, 1024, 0, s>>>(k, w->partial, (int)nb, w->sm);
     if (restart_now)
       update_kernel<K, false><<<nb, 256, 0, s>>>(n, k, p, q, alpha, x, xo, r, ro, w->partial);
     else

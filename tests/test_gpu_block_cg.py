@@ -89,3 +89,32 @@ def test_columns_through_every_level_operator(gpu_lib, k):
         tune.set_tuning(**tune.DEFAULT)
     base = its[False, 0, "fp64"]
     assert all(abs(n - base) <= (2 if key[2] == "bf16" else 1) for key, n in its.items()), its
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_fewer_columns_on_the_same_handle(gpu_lib, prec, graph):
+    """Blocks of falling and rising width on one handle, among them every width that the kernels round up (3, 5, 6, 7)
+    after a wider one: the columns of the earlier block leave nothing behind."""
+    d, K, B = problem((12, 8, 4), 15, 11)
+    mg = pm.solvers.build_hierarchy(d, 2, omega=0.4, smooth_steps=2, precision=prec)
+    cg = pm.solvers.CG(preconditioner=mg, tol=1e-10, maxit=300, graph=graph)
+    cg.update(K)
+    for k in (4, 3, 2, 4, 3, 8, 5, 3, 7, 2, 6, 1, 5, 8):
+        X = cg.solve(B[:, :k].contiguous())
+        assert cg.iterations < 300 and true_residual(K, X, B[:, :k]) < 2e-10, k
+    for k in (11, 13, 14, 15):  # one call, blocks of 8 and of 3, 5, 6 and 7 columns
+        X = cg.solve(B[:, :k].contiguous())
+        assert cg.iterations < 300 and true_residual(K, X, B[:, :k]) < 2e-10, k
+
+
+def test_solved_columns_leave_the_block(gpu_lib):
+    """Four loads, then four of which one is known: the linear dependency aware solver passes on three."""
+    d, K, B = problem((12, 8, 4), 8, 12)
+    mg = pm.solvers.build_hierarchy(d, 2, omega=0.4, smooth_steps=2)
+    lda = pm.solvers.LDAWrapper(pm.solvers.CG(preconditioner=mg, tol=1e-10, maxit=300), tol=1e-9)
+    lda.update(K)
+    lda.solve(B[:, :4].contiguous())
+    B[:, 5] = B[:, 0] - 2.0 * B[:, 3]
+    X = lda.solve(B[:, 4:].contiguous())
+    assert true_residual(K, X, B[:, 4:]) < 2e-9
