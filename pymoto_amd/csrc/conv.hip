@@ -601,7 +601,7 @@ static int conv_wgrad(const Vox& g, const unsigned short* X, const unsigned shor
       }
   const int nb = (int)std::min<long long>(best.ntiles, wgrad_blocks(CI, CO));
   const dim3 grid(nb, 3 / C::NDZ);
-  if (g.nx % 8 || g.ny % best.ty || g.nz % best.tz)
+  if (g.nx % (8 * best.xg) || g.ny % best.ty || g.nz % best.tz)
     conv3d_wgrad_kernel<CI, CO, true><<<grid, 256, lds, s>>>(g, best, X, G, work);
   else
     conv3d_wgrad_kernel<CI, CO, false><<<grid, 256, lds, s>>>(g, best, X, G, work);

@@ -99,3 +99,10 @@ def test_conv_non_finite_voxel_stays_local(gpu_lib, ci, co, nel):
             want[t, :, 0] = True
     assert torch.equal(bad, want)
     assert bool(torch.isfinite(db).all())
+
+
+@pytest.mark.parametrize("ci,co", [(8, 16), (16, 16), (32, 64), (64, 64)])
+@pytest.mark.parametrize("nel", [(56, 20, 8), (40, 12, 12), (88, 16, 8)])
+def test_conv_non_finite_voxel_beside_an_outer_group(gpu_lib, ci, co, nel):
+    """The same where whole groups of 8 voxels of the last box lie outside the grid."""
+    test_conv_non_finite_voxel_stays_local(gpu_lib, ci, co, nel)
