@@ -93,8 +93,9 @@ int pmt_oc_update(long long n, const double* x, const double* dg, double xmin, d
  * steps: from [l1, l2], while l2 - l1 > tol, lmid = (l1 + l2) / 2 and l1 = lmid if sum(xnew(lmid)) - target
  * > 0 else l2 = lmid; xnew receives the design of the last lmid (the same bits as pmt_oc_update step by
  * step).  work: pmt_oc_work_size() doubles; on completion work[0..3] = l1, l2, the last lmid, max(dg) (NaN if
- * dg has one).  l2 - l1 may still exceed tol where the halvings do not reach it (tol near the spacing of
- * doubles); with l2 - l1 <= tol at the start xnew is unspecified. */
+ * dg has one).  The interval has to be finite with 0 <= l1, so that every multiplier is positive; where the halvings
+ * underflow the last lmid is 0 and xnew unspecified.  l2 - l1 may still exceed tol where the halvings do not reach it
+ * (tol near the spacing of doubles); with l2 - l1 <= tol at the start xnew is unspecified. */
 int pmt_oc_work_size(void);
 int pmt_oc_step(long long n, const double* x, const double* dg, double xmin, double xmax, double move, double l1,
                 double l2, double tol, double target, double* xnew, double* work, void* stream);

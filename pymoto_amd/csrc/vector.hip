@@ -940,7 +940,9 @@ int pmt_oc_work_size(void) { return 2 * kOcState + 2 * (kOcNodes + 1) * kReduceB
 
 int pmt_oc_step(long long n, const double* x, const double* dg, double xmin, double xmax, double move, double l1,
                 double l2, double tol, double target, double* xnew, double* work, void* stream) {
-  if (n <= 0 || !x || !dg || !xnew || !work) return arg_error("pmt_oc_step: bad argument");
+  if (n <= 0 || !x || !dg || !xnew || !work || !(l1 >= 0.0) || !std::isfinite(l1) || !std::isfinite(l2) ||
+      std::isnan(tol))
+    return arg_error("pmt_oc_step: bad argument (finite interval with 0 <= l1)");
   hipStream_t s = (hipStream_t)stream;
   OcState* st[2] = {(OcState*)work, (OcState*)(work + kOcState)};
   double* partial[2] = {work + 2 * kOcState, work + 2 * kOcState + (kOcNodes + 1) * kReduceBlocks};

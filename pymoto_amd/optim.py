@@ -39,14 +39,18 @@ class OC:
         xnew = torch.empty_like(x)
         l1, l2 = self.l1init, self.l2init
         maxdg = None
-        if n > 0 and l2 - l1 > self.l1l2tol:
+        # a trial design needs a positive multiplier: with an interval from 0 on the bisection meets no other (but by
+        # underflow); any other interval goes step by step, and a step that comes to one is refused
+        if n > 0 and l2 - l1 > self.l1l2tol and 0.0 <= l1 < l2 < np.inf:
             work = torch.empty(lib.pmt_oc_work_size(), dtype=torch.float64, device=x.device)
             _lib.check(lib.pmt_oc_step(n, _lib.ptr(x), _lib.ptr(dg), self.xmin, self.xmax, self.move, float(l1), float(l2),
                                        float(self.l1l2tol), self.maxvol * n, _lib.ptr(xnew), _lib.ptr(work),
                                        _lib.stream()), "OC step")
-            l1, l2, _, maxdg = work[:4].tolist()
+            l1, l2, last, maxdg = work[:4].tolist()
         if (float(dg.max().item()) if maxdg is None else maxdg) > 1e-15:
             warnings.warn("OC only works for negative sensitivities; clipping positive values.")
+        if maxdg is not None and not last > 0.0:
+            raise _lib.HIPError("OC step: the interval halved to a multiplier of 0")
         # the steps left where the interval does not halve down to the tolerance
         while l2 - l1 > self.l1l2tol:
             tot = torch.empty(1, dtype=torch.float64, device=x.device)

@@ -71,3 +71,29 @@ def test_oc_module_warns_and_matches_oracle(gpu_lib):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         oc.step(None, torch.as_tensor(dg).cuda())
+
+
+def test_oc_refuses_multipliers_that_are_not_positive(gpu_lib):
+    """The trial design x sqrt(-dg / l) needs l > 0: an interval whose bisection comes to another multiplier is
+    refused, at its first step, at a later one or where the halvings underflow, and no other."""
+    x = torch.full((100,), 0.5, dtype=torch.float64, device="cuda")
+    dg = -torch.linspace(0.1, 1.0, 100, dtype=torch.float64, device="cuda")
+
+    def step(l1, l2, tol, maxvol=0.5, d=dg):
+        return pm.OC(pm.Signal("x", x), None, None, verbosity=0, l1init=l1, l2init=l2, l1l2tol=tol, maxvol=maxvol
+                     ).step(None, d)
+
+    for l1, l2, tol in ((-1.0, 1.0, 1e-4), (-3.0, 1.0, 1e-4), (float("-inf"), 1.0, 1e-4)):
+        with pytest.raises(_lib.HIPError):  # first multiplier 0, -1, -inf
+            step(l1, l2, tol)
+    with pytest.raises(_lib.HIPError):  # 49.5, then below: every volume is less than the whole
+        step(-1.0, 100.0, 1e-4, maxvol=1.0)
+    with pytest.raises(_lib.HIPError):  # (0, l2] halved to nothing
+        step(0.0, 1.0, 0.0, maxvol=1.0)
+    # a negative end that no multiplier of the bisection reaches: as step by step
+    ref, _, _ = stepwise(gpu_lib, x, 50.0 * dg, 0.0, 1.0, 0.1, 0.5 * 100, -1.0, 100.0, 1e-4)
+    assert torch.equal(step(-1.0, 100.0, 1e-4, d=50.0 * dg), ref)
+    work = torch.empty(gpu_lib.pmt_oc_work_size(), dtype=torch.float64, device="cuda")
+    for l1, l2 in ((-1.0, 1.0), (float("nan"), 1.0), (0.0, float("inf"))):
+        assert gpu_lib.pmt_oc_step(100, _lib.ptr(x), _lib.ptr(dg), 0.0, 1.0, 0.1, l1, l2, 1e-4, 50.0, _lib.ptr(x.clone()),
+                                   _lib.ptr(work), _lib.stream()) < 0
