@@ -121,9 +121,9 @@ def _zeros_like(state: Any) -> Any:
 def returns_new_arrays(f):
     """Marks a ``_sensitivity`` whose results are newly allocated, distinct, and kept by nobody: the first term
     of a signal's sensitivity is then taken over instead of copied (the copy of a 192x96x96 density vector took 5.6 us
-    on the device and 13 us per module with its launch).  The mark belongs to the function: an override without it
-    goes back to copies."""
-    f.returns_new_arrays = True
+    on the device and 13 us per module with its launch).  The mark is the function itself: an override without it, also
+    one that took over the attributes of the function it wraps (``functools.wraps``), goes back to copies."""
+    f.returns_new_arrays = f
     return f
 
 
@@ -362,7 +362,8 @@ class Module(metaclass=_ModuleMeta):
             d_in = list(d_in) if isinstance(d_in, (list, tuple)) else [d_in]
             if len(d_in) != len(self.sig_in):
                 raise TypeError(f"_sensitivity returned {len(d_in)} values for {len(self.sig_in)} inputs")
-            fresh = getattr(self._sensitivity, "returns_new_arrays", False)
+            f = self._sensitivity
+            fresh = getattr(f, "returns_new_arrays", None) is getattr(f, "__func__", f)
             for s, d in zip(self.sig_in, d_in):
                 if not _is_signal(s):
                     continue

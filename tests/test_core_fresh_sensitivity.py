@@ -1,4 +1,6 @@
 """Sensitivities that a module marks as newly allocated are taken over by the signal, all others are copied."""
+import functools
+
 import numpy as np
 
 import pymoto_amd as pm
@@ -50,3 +52,24 @@ def test_override_and_slice_get_private_copies():
     m = run(Fresh, z)
     assert z.sensitivity is not m.last
     np.testing.assert_array_equal(z.sensitivity, 2.0)
+
+
+def test_wrapper_of_a_marked_function_gets_private_copies():
+    """functools.wraps copies a function's attributes: a wrapper that keeps what it returns is not marked by them."""
+    kept = []
+
+    def recorded(f):
+        @functools.wraps(f)
+        def wrapper(*args):
+            kept.append(f(*args))
+            return kept[-1]
+        return wrapper
+
+    class Recorded(Fresh):
+        _sensitivity = recorded(Fresh._sensitivity)
+
+    x = pm.Signal("x", np.arange(4.0))
+    run(Recorded, x)
+    run(Recorded, x)
+    np.testing.assert_array_equal(x.sensitivity, 4.0)
+    np.testing.assert_array_equal(kept[0], 2.0)
