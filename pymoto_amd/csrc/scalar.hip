@@ -193,18 +193,24 @@ __global__ void scalar_stencil_fine_kernel(GridDims g, const double* __restrict_
 // w w S[j - i][i].  A stencil entry that points outside the grid is 0 by construction.  One thread per coarse
 // node; in: n x m x q nodes (x, y, z), out: the same with the axis halved.
 // 80x80x48: 66 us for the three axes of the first level (1.6 ms as one kernel of nested pair loops).
+// The three passes take a slab of coarse planes (rows in 2D) at a time, so that what lies between them stays
+// small (kSlab): S and T are the slab's part of arrays whose coefficients lie ss and ts apart, nl planes of the last
+// axis; the last axis itself is halved from its plane `first` (the image of the slab's first coarse plane) on to cl.
 template <int DIM, int AXIS>
 __global__ void __launch_bounds__(256)
-scalar_coarsen_kernel(int nx, int ny, int nz, const double* __restrict__ S, double* __restrict__ T) {
+scalar_coarsen_kernel(int nx, int ny, int nl, int first, int cl, const double* __restrict__ S, long long ss,
+                      double* __restrict__ T, long long ts) {
   constexpr int NS = SCfg<DIM>::NS, ST = AXIS == 0 ? 1 : AXIS == 1 ? 3 : 9;  // stride of the axis offset in c
-  const int cx = AXIS == 0 ? (nx + 1) / 2 : nx, cy = AXIS == 1 ? (ny + 1) / 2 : ny, cz = AXIS == 2 ? (nz + 1) / 2 : nz;
-  const long long N = (long long)blockIdx.x * blockDim.x + threadIdx.x, nc = (long long)cx * cy * cz;
-  if (N >= nc) return;
+  constexpr bool LAST = AXIS == DIM - 1;
+  if (DIM == 2) ny = nl;
+  const int nz = DIM == 3 ? nl : 1;
+  const int cx = AXIS == 0 ? (nx + 1) / 2 : nx, cy = AXIS == 1 ? (LAST ? cl : (ny + 1) / 2) : ny, cz = AXIS == 2 ? cl : nz;
+  const long long N = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (N >= (long long)cx * cy * cz) return;
   const int I = (int)(N % cx), J = (int)((N / cx) % cy), K = (int)(N / ((long long)cx * cy));
-  const long long nf = (long long)nx * ny * nz;
-  const long long at = ((long long)(AXIS == 2 ? 2 * K : K) * ny + (AXIS == 1 ? 2 * J : J)) * nx + (AXIS == 0 ? 2 * I : I);
+  const int pos = 2 * (AXIS == 0 ? I : AXIS == 1 ? J : K) + (LAST ? first : 0), len = AXIS == 0 ? nx : AXIS == 1 ? ny : nz;
+  const long long at = ((long long)(AXIS == 2 ? pos : K) * ny + (AXIS == 1 ? pos : J)) * nx + (AXIS == 0 ? pos : I);
   const long long step = AXIS == 0 ? 1 : AXIS == 1 ? nx : (long long)nx * ny;
-  const int pos = 2 * (AXIS == 0 ? I : AXIS == 1 ? J : K), len = AXIS == 0 ? nx : AXIS == 1 ? ny : nz;
   const bool in[3] = {pos > 0, true, pos + 1 < len};
 #pragma unroll
   for (int o = 0; o < NS / 3; ++o) {  // the offsets along the other axes
@@ -213,7 +219,7 @@ scalar_coarsen_kernel(int nx, int ny, int nz, const double* __restrict__ S, doub
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int f = 0; f < 3; ++f) v[d][f] = in[d] ? S[(c0 + f * ST) * nf + at + (d - 1) * step] : 0.0;
+      for (int f = 0; f < 3; ++f) v[d][f] = in[d] ? S[(c0 + f * ST) * ss + at + (d - 1) * step] : 0.0;
 #pragma unroll
     for (int cp = -1; cp <= 1; ++cp) {
       double acc = 0.0;
@@ -225,7 +231,7 @@ scalar_coarsen_kernel(int nx, int ny, int nz, const double* __restrict__ S, doub
           if (f < -1 || f > 1) continue;
           acc = fma((di ? 0.5 : 1.0) * (dj ? 0.5 : 1.0), v[di + 1][f + 1], acc);
         }
-      T[(c0 + (cp + 1) * ST) * nc + N] = acc;
+      T[(c0 + (cp + 1) * ST) * ts + N] = acc;
     }
   }
 }
@@ -528,8 +534,8 @@ struct pmt_smg {
   double* u[kScalarMaxLevels] = {};  // corrections (levels >= 1)
   double* b[kScalarMaxLevels] = {};  // right-hand sides (levels >= 1)
   double* t[kScalarMaxLevels] = {};  // work: iterate, residual
-  double* t2[kScalarMaxLevels] = {};
-  double* W[2] = {};                 // stencils of the first level coarsened along x, along x and y
+  double* W[2] = {};                 // a slab's stencils coarsened along x, along x and y
+  long long wlen[2] = {};            // doubles of W
   bool sym = false;                  // P0 is symmetric
   bool elem = false;                 // P0[a][b] depends on a ^ b only: the fine grid is applied from the densities
   double pe[8] = {};                 // then P0[0][a]
@@ -557,6 +563,17 @@ int smg_alloc(pmt_smg* h, double** p, long long count) {
   h->bytes += count * (long long)sizeof(double);
   *p = static_cast<double*>(q);
   return PMT_OK;
+}
+
+// Coarse planes of a slab whose 2 m + 1 fine planes, a and b doubles each after the first and second axis, fit
+// into wa and wb doubles; at least one.  64 MB after the first axis: one slab up to about 0.6 million nodes, and the
+// work arrays add 0.1 GB to a hierarchy instead of 0.75 of its fine stencil (162 bytes per node beside 310).  128^3: an
+// update in four slabs 7.76 ms, in one 7.73.
+constexpr long long kSlab = 1LL << 23;
+int slab_planes(long long a, long long b, int ncl, long long wa, long long wb) {
+  long long fine = wa / a;
+  if (b > 0) fine = std::min(fine, wb / b);
+  return fine >= 2LL * ncl - 1 ? ncl : (int)std::max(1LL, (fine - 1) / 2);
 }
 
 // node planes per block: 4, and 2 or 1 while the blocks do not give every CU two
@@ -600,6 +617,37 @@ int smg_level(pmt_smg* h, int l, LevelArgs a, hipStream_t s) {
   return check_launch("scalar_level_kernel");
 }
 
+// S[l + 1] = R^T S[l] R by slabs of the last axis, as many coarse planes (2D: rows) at a time as W takes: m of them
+// need the 2 m + 1 fine planes around their images
+template <int DIM>
+int smg_coarsen(pmt_smg* h, int l, hipStream_t s) {
+  constexpr int NS = SCfg<DIM>::NS;
+  const GridDims &gf = h->g[l], &gc = h->g[l + 1];
+  const int nl = DIM == 3 ? gf.nz : gf.ny, ncl = DIM == 3 ? gc.nz : gc.ny;
+  const long long fp = DIM == 3 ? (long long)gf.nx * gf.ny : gf.nx;  // nodes of a plane: fine, after x, after x and y
+  const long long xp = DIM == 3 ? (long long)gc.nx * gf.ny : gc.nx, cp = DIM == 3 ? (long long)gc.nx * gc.ny : gc.nx;
+  const int m = slab_planes(NS * xp, DIM == 3 ? NS * cp : 0, ncl, h->wlen[0], h->wlen[1]);
+  for (int c0 = 0; c0 < ncl; c0 += m) {
+    const int cl = std::min(m, ncl - c0), f0 = std::max(2 * c0 - 1, 0), f1 = std::min(2 * (c0 + cl - 1) + 2, nl);
+    const int n = f1 - f0, first = 2 * c0 - f0;
+    const double* S = h->S[l] + f0 * fp;
+    double* T = h->S[l + 1] + c0 * cp;
+    scalar_coarsen_kernel<DIM, 0><<<blocks_for(n * xp, 256), 256, 0, s>>>(gf.nx, gf.ny, n, 0, 0, S, gf.nnodes, h->W[0],
+                                                                        n * xp);
+    if constexpr (DIM == 3) {
+      scalar_coarsen_kernel<3, 1><<<blocks_for(n * cp, 256), 256, 0, s>>>(gc.nx, gf.ny, n, 0, 0, h->W[0], n * xp, h->W[1],
+                                                                        n * cp);
+      scalar_coarsen_kernel<3, 2><<<blocks_for(cl * cp, 256), 256, 0, s>>>(gc.nx, gc.ny, n, first, cl, h->W[1], n * cp, T,
+                                                                         gc.nnodes);
+    } else {
+      scalar_coarsen_kernel<2, 1><<<blocks_for(cl * cp, 256), 256, 0, s>>>(gc.nx, 0, n, first, cl, h->W[0], n * xp, T,
+                                                                         gc.nnodes);
+    }
+    PMT_TRY(check_launch("scalar_coarsen_kernel"));
+  }
+  return PMT_OK;
+}
+
 int smg_apply(pmt_smg* h, int l, const double* u, double* y, hipStream_t s, const double* r = nullptr) {
   LevelArgs a{};
   a.u = u;
@@ -622,8 +670,9 @@ int smg_vcycle(pmt_smg* h, int l, const double* r, double* z, hipStream_t s) {
   const GridDims& g = h->g[l];
   if (l == h->nlev - 1) return launch_gemv<double>(g.nnodes, h->Ainv, r, z, s);
   const int steps = h->steps[l];
-  // pre-smoothing from zero (iterative.py:232-233); the first two sweeps are one pass
-  double *cur = h->t[l], *oth = h->t2[l];
+  // pre-smoothing from zero (iterative.py:232-233); the first two sweeps are one pass.  The passes alternate between
+  // t and z, from the one that has the last of the `steps` post-sweeps write z
+  double *cur = steps == 1 ? h->t[l] : z, *oth = steps == 1 ? z : h->t[l];
   LevelArgs a{};
   a.b = r;
   if (steps == 1) {
@@ -648,10 +697,10 @@ int smg_vcycle(pmt_smg* h, int l, const double* r, double* z, hipStream_t s) {
     scalar_restrict_kernel<2><<<cblocks, 256, 0, s>>>(g, gc, oth, h->b[l + 1]);
   PMT_TRY(check_launch("scalar_restrict_kernel"));
   PMT_TRY(smg_vcycle(h, l + 1, h->b[l + 1], h->u[l + 1], s));
-  // post-smoothing, the prolongation within its first sweep; the last sweep writes z
+  // post-smoothing, the prolongation within its first sweep
   for (int k = 0; k < steps; ++k) {
     a.u = cur;
-    a.y = k == steps - 1 ? z : oth;
+    a.y = oth;
     if (k == 0) {
       a.e = h->u[l + 1];
       a.cnx = gc.nx;
@@ -662,7 +711,7 @@ int smg_vcycle(pmt_smg* h, int l, const double* r, double* z, hipStream_t s) {
     }
     std::swap(cur, oth);
   }
-  return PMT_OK;
+  return cur == z ? PMT_OK : arg_error("smg_vcycle: internal buffer parity error");
 }
 
 }  // namespace
@@ -744,7 +793,6 @@ int pmt_smg_create(int nelx, int nely, int nelz, int nlevels, const double* omeg
     if (l < nlevels - 1) {
       A(&h->dinv[l], h->g[l].nnodes);
       A(&h->t[l], h->g[l].nnodes);
-      A(&h->t2[l], h->g[l].nnodes);
     }
     if (l > 0) {
       A(&h->u[l], h->g[l].nnodes);
@@ -755,8 +803,17 @@ int pmt_smg_create(int nelx, int nely, int nelz, int nlevels, const double* omeg
   A(&h->gjw, gj_work_size(nc));
   const GridDims& g0 = h->g[0];
   const long long n0 = g0.nnodes;
-  A(&h->W[0], (long long)NS * h->g[1].nx * g0.ny * g0.nz);
-  if (h->dim == 3) A(&h->W[1], (long long)NS * h->g[1].nx * h->g[1].ny * g0.nz);
+  {
+    const GridDims& g1 = h->g[1];
+    const long long a = NS * (h->dim == 3 ? (long long)g1.nx * g0.ny : g1.nx);  // doubles of a fine plane after x
+    const long long b = h->dim == 3 ? (long long)NS * g1.nx * g1.ny : 0;        // after x and y
+    const int ncl = h->dim == 3 ? g1.nz : g1.ny;
+    const int m = slab_planes(a, 0, ncl, kSlab, 0), fine = m == ncl ? 2 * ncl - 1 : 2 * m + 1;
+    h->wlen[0] = a * fine;
+    h->wlen[1] = b * fine;
+    A(&h->W[0], h->wlen[0]);
+    if (h->dim == 3) A(&h->W[1], h->wlen[1]);
+  }
   A(&h->parts, 2LL * level_blocks(g0));
   // whether P0[a][b] depends on a ^ b only (to rounding): an isotropic box element
   double big = 0.0;
@@ -818,16 +875,7 @@ int pmt_smg_update(pmt_smg* h, const double* xe, const uint8_t* bcmask, double b
     scalar_dinv_kernel<<<blocks_for(gf.nnodes, 256), 256, 0, s>>>(
         gf.nnodes, h->S[l] + (h->dim == 3 ? 13 : 4) * gf.nnodes, h->dinv[l]);
     PMT_TRY(check_launch("scalar_dinv_kernel"));
-    const long long n1 = (long long)gc.nx * gf.ny * gf.nz, n2 = (long long)gc.nx * gc.ny * gf.nz;
-    if (h->dim == 3) {
-      scalar_coarsen_kernel<3, 0><<<blocks_for(n1, 256), 256, 0, s>>>(gf.nx, gf.ny, gf.nz, h->S[l], h->W[0]);
-      scalar_coarsen_kernel<3, 1><<<blocks_for(n2, 256), 256, 0, s>>>(gc.nx, gf.ny, gf.nz, h->W[0], h->W[1]);
-      scalar_coarsen_kernel<3, 2><<<blocks_for(gc.nnodes, 256), 256, 0, s>>>(gc.nx, gc.ny, gf.nz, h->W[1], h->S[l + 1]);
-    } else {
-      scalar_coarsen_kernel<2, 0><<<blocks_for(n1, 256), 256, 0, s>>>(gf.nx, gf.ny, 1, h->S[l], h->W[0]);
-      scalar_coarsen_kernel<2, 1><<<blocks_for(n2, 256), 256, 0, s>>>(gc.nx, gf.ny, 1, h->W[0], h->S[l + 1]);
-    }
-    PMT_TRY(check_launch("scalar_coarsen_kernel"));
+    PMT_TRY(h->dim == 3 ? smg_coarsen<3>(h, l, s) : smg_coarsen<2>(h, l, s));
   }
   const int L = h->nlev - 1;
   const long long nc = h->g[L].nnodes;

@@ -78,3 +78,50 @@ def test_vcycle_vs_dense(gpu_lib, nel, levels, kind):
     z = mg.solve(torch.as_tensor(r).cuda()).cpu().numpy()
     ref = dense_vcycle(A, nodes, levels, 0.6, steps, r)
     assert np.abs(z - ref).max() < 1e-10 * np.abs(ref).max()
+
+
+def axis_interpolate(c, ax):
+    """(bi/tri)linear interpolation of one axis: nodes 2 I are copied, those between are means."""
+    n = c.shape[ax]
+    lo, hi = c.narrow(ax, 0, n - 1), c.narrow(ax, 1, n - 1)
+    pairs = torch.stack([lo, 0.5 * (lo + hi)], dim=ax + 1).flatten(ax, ax + 1)
+    return torch.cat([pairs, c.narrow(ax, n - 1, 1)], dim=ax)
+
+
+def axis_restrict(f, ax):
+    """Its transpose."""
+    n = f.shape[ax]
+    even, odd = f.index_select(ax, torch.arange(0, n, 2, device=f.device)), \
+        f.index_select(ax, torch.arange(1, n, 2, device=f.device))
+    zero = torch.zeros_like(odd.narrow(ax, 0, 1))
+    return even + 0.5 * (torch.cat([zero, odd], ax) + torch.cat([odd, zero], ax))
+
+
+@pytest.mark.parametrize("nel,levels", [((256, 256, 128), 5), ((2048, 2048, 0), 6)])
+def test_large_grid_memory_and_coarse_operator(gpu_lib, nel, levels):
+    """A grid whose coarse stencils are formed slab by slab: the level-1 product is R^T A R of the fine one (sums of at
+    most 27 x 27 products and 27 + 8 terms of the transfers, each good to 2^-53: 1e-12 of the largest entry), and the
+    handle takes the stencils (NS doubles per node and 1/(2^D - 1) more), six vectors (r, z, p, q, D^-1, work) on the fine grid
+    and four on each coarse one, and 0.3 GB for the coarsest inverse, sums and slabs."""
+    d = pm.VoxelDomain(*nel)
+    nodes = [n + 1 for n in nel if n]
+    g = torch.Generator().manual_seed(1)
+    P = pm.AssemblePoisson(d, bc=np.arange(0, 500, 3))(0.1 + torch.rand(d.nel, generator=g, dtype=torch.float64).cuda())
+    mg = pm.solvers.build_hierarchy(d, levels, omega=0.5, smooth_steps=2)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    mg._ensure_handle(P)
+    used = free - torch.cuda.mem_get_info()[0]
+    n, more = P.shape[0], 1.0 / (2 ** d.dim - 1)
+    assert used < 8 * n * (3 ** d.dim * (1 + more) + 6 + 4 * more) * 1.02 + 3e8
+    mg.update(P)
+    shape = [(m + 1) // 2 for m in reversed(nodes)]
+    c = torch.randn(shape, generator=g, dtype=torch.float64).cuda()
+    f = c
+    for ax in range(len(shape)):
+        f = axis_interpolate(f, ax)
+    f = mg.level_apply(0, f.reshape(-1).contiguous()).reshape(list(reversed(nodes)))
+    for ax in range(len(shape)):
+        f = axis_restrict(f, ax)
+    got = mg.level_apply(1, c.reshape(-1).contiguous()).reshape(shape)
+    assert float((got - f).abs().max() / f.abs().max()) < 1e-12
