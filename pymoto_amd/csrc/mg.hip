@@ -232,7 +232,7 @@ static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool fir
   Level& L = mg->L[l];
   Level& C = mg->L[l + 1];
   const LevelCols<T> B = level_vectors<T>(mg, l, cols), CB = level_vectors<T>(mg, l + 1, cols);
-  if (v2_ok(mg, L.steps)) {  // Q4: all sweeps of a visit in one launch
+  if (v2_ok(mg, l, sizeof(T) == 4, cols)) {  // Q4: all sweeps of a visit in one launch
     const Sweeps2 sw = sweep_coefficients(mg, l);
     PMT_TRY(launch_v2_down<T>(mg, l, fine_x<T>(mg), sw, b, B.t, CB.b, s, cols));
     PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s, false, cols));
@@ -243,9 +243,9 @@ static int vcycle(pmt_mg* mg, int l, const T* b, T* out, hipStream_t s, bool fir
   T* oth = out;
   PMT_TRY(smooth<T>(mg, l, b, cur, oth, true, s, first_done, cols));
   PMT_TRY(level_apply<T>(mg, l, MODE_RESIDUAL, cur, b, B.r, s, cols));
-  // a smoothed coarse level starts from zero: the restriction also writes its first sweep into the
+  // a coarse level smoothed by launches starts from zero: the restriction also writes its first sweep into the
   // buffer that sweep would write (CB.t), with the factor the smoother would use
-  const bool fuse = l + 1 < mg->nlev - 1;
+  const bool fuse = l + 1 < mg->nlev - 1 && !v2_ok(mg, l + 1, sizeof(T) == 4, cols);
   const double w0 = first_sweep_factor(mg, l + 1);
   PMT_TRY(launch_restrict<T>(L.g, C.g, B.r, CB.b, s, fuse ? C.buf<T>().dinv : nullptr, w0, fuse ? CB.t : nullptr, cols));
   PMT_TRY(vcycle<T>(mg, l + 1, CB.b, CB.u, s, fuse, cols));
@@ -927,7 +927,7 @@ int pmt_pcg_solve(pmt_mg* mg, const double* b, double* x, int x0_is_zero, double
     // the update also writes the V-cycle's first fine sweep from zero into the fine level's work vector:
     // omega D^-1 r (damped Jacobi) or D^-1 r / theta (Chebyshev) in the V-cycle's precision, the expression
     // of the sweep kernel
-    const bool first = !v2_ok(mg, F.steps);  // (the Q4 V-cycle starts from r)
+    const bool first = !v2_ok(mg, 0, mixed, 1);  // (those sweeps start from r)
     const double first_factor = first_sweep_factor(mg, 0);
     bool r_ready = false;  // the V-cycle's input (and first sweep) are written
     bool published = false;  // r.r already on its way to the host (with the r update's reduction)

@@ -155,7 +155,7 @@ struct Sweeps2 {
   int n;
   double a[kV2MaxSweeps], b[kV2MaxSweeps];
 };
-bool v2_ok(const pmt_mg* mg, int steps);
+bool v2_ok(const pmt_mg* mg, int l, bool fp32, int cols);  // does level l take them?
 // u = the sweeps from zero on level l, bc = R^T (b - A u)
 template <typename T>
 int launch_v2_down(pmt_mg* mg, int l, const T* xe, const Sweeps2& sw, const T* b, T* u, T* bc, hipStream_t s,

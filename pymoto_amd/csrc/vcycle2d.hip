@@ -10,7 +10,8 @@
 //   up:   prolongation of the correction, the sweeps.
 // Blocks are up to 32 x 32 threads, one node each: with the default 5 sweeps 22 x 22 nodes (up) and 10 x 10
 // coarse nodes (down) per block, so half of the arithmetic is the halo's - cheaper than a launch at small
-// sizes, and at large ones the operator rows are read once instead of once per sweep.
+// sizes; at large ones the operator rows are read once instead of once per sweep, which pays for a middle range
+// of sweep counts (v2_ok).
 // 120x40, 5 sweeps, 4 grids: 37 us per cycle in 7 launches (18 x 18 threads on the fine grid); about 150 us in 37
 // launches of one sweep or transfer each.
 #include "mg_impl.h"
@@ -223,7 +224,29 @@ V2Op<T> v2_op(const pmt_mg* mg, const Level& L, const LevelBuf<T>& B, bool fine,
 
 }  // namespace
 
-bool v2_ok(const pmt_mg* mg, int steps) { return mg->dim == 2 && steps <= kV2MaxSweeps; }
+// Up to how many thousand nodes (0: any number) a level's visit of 1 to 10 sweeps goes in two launches, on the fine
+// grid and on the others, in FP64 and FP32.  Small levels save the launches and win with every sweep count.  On a
+// grid that fills the chip the halo counts: a launch per sweep computes a node once per sweep, a block here
+// (32 / (32 - 2 n))^2 times, which the operator rows kept in registers pay for in the middle of the range only, and
+// least where a launch per sweep forms them from the densities or reads half the bytes.  Microseconds saved by the two
+// launches, at 148,000 / 263,000 / 1,051,000 nodes (fine) and 37,000 / 263,000 / 1,051,000 (stencil):
+//   sweeps                  1              2               5                8                10
+//   FP64 fine          4/ -1/ -21     11/  6/  -8     20/ 13/  10     18/ -8/ -106    -13/-85/ -423
+//   FP32 fine          2/ -4/ -28     10/  1/ -19     18/  9/  -9     17/ -7/ -107     -6/-65/ -381
+//   FP64 stencil       3/-11/ -33      9/  4/  15     22/ 44/ 137     40/ 52/   97     23/  5/ -194
+//   FP32 stencil       3/-11/ -34      8/ -4/ -10     27/ 13/  40     37/  4/   -4     31/-35/ -214
+// (a V-cycle of a 1024x1024 grid with 5 sweeps takes 318 us in FP64).  In FP64 2 to 6 sweeps of the fine grid lose up to
+// 49 us between 0.6 and 2.4 million nodes and gain 29 to 159 us at 4.2 million or with 4 and more columns.  The fine
+// operator takes one column per launch, the stencils all columns of a block, so there the limit is one of all columns' nodes.
+bool v2_ok(const pmt_mg* mg, int l, bool fp32, int cols) {
+  static const int limit[2][2][kV2MaxSweeps] = {
+      {{150, 0, 0, 0, 0, 0, 265, 150, 150, 70}, {100, 0, 0, 0, 0, 0, 0, 0, 0, 265}},
+      {{150, 265, 265, 265, 265, 265, 265, 150, 150, 70}, {70, 150, 0, 0, 0, 0, 0, 0, 150, 100}}};
+  const Level& L = mg->L[l];
+  if (mg->dim != 2 || L.steps < 1 || L.steps > kV2MaxSweeps) return false;
+  const int most = limit[fp32 ? 1 : 0][l > 0 ? 1 : 0][L.steps - 1];
+  return most == 0 || L.g.nnodes * (l > 0 ? cols : 1) <= 1000LL * most;
+}
 
 // Threads per block side for a grid of nx x ny outputs, `out(w)` of them per side: the fewest wavefronts per
 // compute unit.  A sweep is bound by the LDS reads of a block's wavefronts, so while the blocks do not fill

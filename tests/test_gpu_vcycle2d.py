@@ -91,3 +91,31 @@ def test_q4_chebyshev_vcycle_vs_oracle(gpu_lib, nel, levels, steps):
     mg.update(pm.AssembleStiffness(d, bc=bc)(dev(x)))
     cheb = [Cheb(*mg.smoother_interval(l), steps) for l in range(levels - 1)]
     assert relerr(mg.solve(dev(r)).cpu().numpy(), cheb_cycle(omg, cheb, r)) < 1e-9
+
+
+@pytest.mark.parametrize("steps", [1, 2, 8, 10])
+def test_q4_large_level_by_launches(gpu_lib, steps):
+    """A fine grid (164,000 nodes) above the size up to which a visit of 1, 8 and 10 sweeps goes in one launch, over levels
+    below it; 2 sweeps still do.  The V-cycle, and CG with one and with three columns, whose update forms the first sweep."""
+    nel, levels = (1024, 160), 4
+    x, bc, r = problem(nel, steps)
+    Kref = fe.Assembly(*nel, 0, fe.element_stiffness(2), bc=bc).matrix(x)
+    omg = build_mg((*nel, 0), levels, omega=0.4, smooth_steps=steps)
+    omg.update(Kref)
+    d = pm.VoxelDomain(*nel)
+    K = pm.AssembleStiffness(d, bc=bc)(dev(x))
+    ref = omg.solve(r)
+    B = torch.stack([dev(r), dev(np.roll(r, 2)), dev(r * r)], dim=1)
+    B[torch.as_tensor(bc)] = 0.0
+    its = {}
+    for prec, tol in (("fp64", 1e-9), ("fp32", 1e-4)):
+        mg = pm.solvers.build_hierarchy(d, levels, omega=0.4, smooth_steps=steps, precision=prec)
+        cg = pm.solvers.CG(preconditioner=mg, tol=1e-8, maxit=1000)
+        cg.update(K)
+        assert relerr(mg.solve(dev(r)).cpu().numpy(), ref) < tol, prec
+        for b in (B[:, 0].contiguous(), B):
+            u = cg.solve(b)
+            its[prec, b.ndim] = cg.iterations
+            assert cg.iterations < 1000 and float((K.residual(B[:, 0].contiguous(), u if u.ndim == 1 else u[:, 0].contiguous())
+                                                  ).norm() / B[:, 0].norm()) < 2e-8, prec
+    assert abs(its["fp64", 1] - its["fp32", 1]) <= 2 and abs(its["fp64", 2] - its["fp32", 2]) <= 2, its
