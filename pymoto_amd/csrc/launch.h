@@ -112,7 +112,6 @@ int launch_fine_mfma(int mode, const GridDims& g, const double* K0, const float*
 
 // vector.hip
 int launch_dot(long long n, const double* x, const double* y, double* out, double* work, hipStream_t s);
-int launch_dot(long long n, const double* x, const float* y, double* out, double* work, hipStream_t s);
 int launch_dot2(long long n, const double* a0, const double* b0, const double* a1, const double* b1, double* out,
                 double* work, hipStream_t s);
 int launch_axpby(long long n, double a, const double* x, double b, double* y, hipStream_t s);

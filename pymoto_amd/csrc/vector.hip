@@ -109,16 +109,14 @@ __device__ inline double block_sum(double v) {
   return r;  // valid in thread 0
 }
 
-// stage 1: NOUT dot products sharing the grid-stride loop; partial[o*kReduceBlocks + block].  B0: type of
-// the first product's second operand (an FP32 vector is widened exactly: the sums are those of its
-// FP64 copy)
-template <int NOUT, typename B0 = double>
+// stage 1: NOUT dot products sharing the grid-stride loop; partial[o*kReduceBlocks + block]
+template <int NOUT>
 __global__ void __launch_bounds__(kReduceThreads)
-dot_stage1(long long n, const double* __restrict__ a0, const B0* __restrict__ b0, const double* __restrict__ a1,
+dot_stage1(long long n, const double* __restrict__ a0, const double* __restrict__ b0, const double* __restrict__ a1,
            const double* __restrict__ b1, double* __restrict__ partial) {
   double s0 = 0.0, s1 = 0.0;
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    s0 = fma(a0[i], (double)b0[i], s0);
+    s0 = fma(a0[i], b0[i], s0);
     if (NOUT > 1) s1 = fma(a1[i], b1[i], s1);
   }
   double r0 = block_sum(s0);
@@ -378,13 +376,6 @@ __global__ void oc_write_kernel(long long n, const double* __restrict__ x, const
 int launch_dot(long long n, const double* x, const double* y, double* out, double* work, hipStream_t s) {
   dot_stage1<1><<<kReduceBlocks, kReduceThreads, 0, s>>>(n, x, y, nullptr, nullptr, work);
   PMT_TRY(check_launch("dot_stage1"));
-  dot_stage2<1><<<1, kReduceThreads, 0, s>>>(work, out);
-  return check_launch("dot_stage2");
-}
-
-int launch_dot(long long n, const double* x, const float* y, double* out, double* work, hipStream_t s) {
-  dot_stage1<1, float><<<kReduceBlocks, kReduceThreads, 0, s>>>(n, x, y, nullptr, nullptr, work);
-  PMT_TRY(check_launch("dot_stage1<float>"));
   dot_stage2<1><<<1, kReduceThreads, 0, s>>>(work, out);
   return check_launch("dot_stage2");
 }
