@@ -194,7 +194,7 @@ int pmt_k0_extend(int dim, const double* K0_host, double* ext_host);
  * the reflection basis from the transformed child densities, no stencil stored (used when k0_pattern has
  * PMT_K0_REFLECTION and the level is not the coarsest), 0 = half stencil, 2 = 1 for levels of more than
  * 100,000 nodes, else 0 (default).  Read by pmt_mg_create: it applies to hierarchies created afterwards.
- * PMT_TUNE_FILTER: FilterConv kernels for extents k x k x kz up to 15 whose box of outputs fits LDS, 1 = boxes
+ * PMT_TUNE_FILTER: FilterConv kernels for extents k x k x kz with k from 3 to 15 whose box of outputs fits LDS, 1 = boxes
  * staged in LDS (default), 0 = one thread per element gathering through the caches; both sum the taps in
  * the same order.
  * pmt_get_tuning returns the current value or a negative status.

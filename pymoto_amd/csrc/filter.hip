@@ -462,8 +462,9 @@ inline FilterBox filter_box(int kxy, int kz, long long lx, long long ly, long lo
   return b;
 }
 
-// whether the box kernels take these extents: boxes above 64 KB of LDS (3D from 11^3) stay with the gather
-// kernels, and so does the adjoint of the kernels above 5 without a workspace
+// whether the box kernels take these extents: equal ones of 3 to 15 in x and y (their weights of a z tap lie one per
+// lane), any in z whose box fits: boxes above 64 KB of LDS (3D from 11^3, 3 x 3 x 21 with 4 outputs per thread, 3 x 3 x 37
+// with 2) stay with the gather kernels, and so does the adjoint of the kernels above 5 without a workspace
 inline bool filter_box_ok(bool fwd, int nx, int ny, int nz, int kx, int ky, int kz, const double* work) {
   if (kx != ky || kx < 3 || kx > 15) return false;
   if (!fwd && !work && !(kx <= 5 && (kz == kx || kz == 1))) return false;
@@ -478,7 +479,9 @@ void launch_filter_box_k(bool fwd, int nx, int ny, int nz, int kz, const double*
   const FilterBox b = filter_box(KXY, kz, lx, ly, lz);
   const int ntz = 8 / b.nty, tiles_x = (lx + 31) / 32, tiles_y = (ly + b.oy * b.nty - 1) / (b.oy * b.nty);
   const unsigned blocks = (unsigned)(tiles_x * tiles_y * ((lz + ntz - 1) / ntz));
-  const unsigned m_ly = (1u << 20) / b.ly + 1;  // t / ly for t < ly * lz, ly <= 46, lz <= 18
+  // t / ly for t < ly lz as t m_ly >> 20: exact while t ly < 2^20, and 64 KB of LDS in rows of 34 doubles and more hold
+  // ly lz <= 240 of them, with ly <= 46
+  const unsigned m_ly = (1u << 20) / b.ly + 1;
   auto run = [&](auto kernel) {
     kernel<<<blocks, 256, b.lds, s>>>(nx, ny, nz, kz, b.nty, tiles_x, tiles_y, m_ly, w, m0, m1, cv, in, out, work);
   };

@@ -39,3 +39,33 @@ def test_filter_wide_equals_gather(gpu_lib, nel, radius, bcs):
     filt = ConvFilter(nel, m.weights, (bcs[0:2], bcs[2:4], bcs[4:6]))
     npt.assert_allclose(out[1][0], filt.forward(x), rtol=1e-12, atol=1e-14)
     npt.assert_allclose(out[1][1], filt.adjoint(dy), rtol=1e-12, atol=1e-13)
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 17), (3, 3, 19), (3, 3, 21), (3, 3, 35), (3, 3, 37), (5, 5, 9), (15, 15, 1), (7, 7, 3),
+                                   (3, 5, 3)])
+@pytest.mark.parametrize("nel", [(9, 7, 40), (200, 130, 70)])
+def test_filter_unequal_extents(gpu_lib, shape, nel):
+    """Weights that are not the same in z, up to the extents whose box just fits into LDS and the first that do not, with 2
+    and with 4 outputs per thread: the bits of the gather kernels, with every kind of face in z."""
+    d = pm.VoxelDomain(*nel)
+    rng = np.random.default_rng(shape[2])
+    w = rng.uniform(-1.0, 1.0, shape)
+    x, dy = rng.uniform(0.0, 1.0, d.nel), rng.standard_normal(d.nel)
+    out = {}
+    try:
+        for tiled in (1, 0):
+            assert gpu_lib.pmt_set_tuning(6, tiled) == 0
+            m = pm.FilterConv(d, weights=w, zmin_bc="wrap", zmax_bc=0.5, ymin_bc="edge")
+            sx = pm.Signal("x", torch.as_tensor(x).cuda())
+            sy = m(sx)
+            sy.sensitivity = torch.as_tensor(dy).cuda()
+            m.sensitivity()
+            out[tiled] = (sy.state.cpu().numpy(), sx.sensitivity.cpu().numpy())
+    finally:
+        gpu_lib.pmt_set_tuning(6, 1)
+    npt.assert_array_equal(out[1][0], out[0][0])
+    npt.assert_array_equal(out[1][1], out[0][1])
+    if nel[0] < 100:
+        filt = ConvFilter(nel, w, (("symmetric",) * 2, ("edge", "symmetric"), ("wrap", 0.5)))
+        npt.assert_allclose(out[1][0], filt.forward(x), rtol=1e-12, atol=1e-12)
+        npt.assert_allclose(out[1][1], filt.adjoint(dy), rtol=1e-12, atol=1e-12)
