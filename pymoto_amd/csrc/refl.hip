@@ -279,7 +279,7 @@ __device__ inline void coarse1_element(const T* tab, const T (&X)[8], T (&v)[8][
 
 // OP 0: the fine grid (element factor x_e, Dirichlet-masked nodes, bcdiag rows).  OP 1: the first
 // coarse level of a hex8 hierarchy (element factors X^[8], layout [layer][m][element]; no mask: the
-// elements with Dirichlet children get their corrections from coarse1_correct_kernel afterwards).
+// elements with Dirichlet children get their corrections from coarse1_tapply_kernel afterwards).
 // Waves per SIMD the register allocation must leave room for: the fine FP64 residual and the CG product
 // fit 168 VGPRs (3 waves) without spilling (2 waves otherwise); every other instance keeps the
 // compiler's choice (a bound on the sweeps makes them spill, which costs more than the wave gains).
